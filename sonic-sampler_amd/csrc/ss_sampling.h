@@ -1025,15 +1025,28 @@ __device__ __forceinline__ uint32_t wave_survivors_masked(TileSmem<E> &sm, const
     return total;
 }
 
+// The wave's share of a tile's `want` candidates, in proportion to the columns it holds of the
+// tile's `valid` (rounded up, so the shares add up to at least `want`): want / 4 in a full tile.
+// A row's partial last tile fills its first waves first; with the full tile's share a wave of few
+// columns had no bound, every column of the tile survived and the tile took the exact cut (48 decode rows
+// of 50,003 columns in 8192-column tiles: tile kernel 31.2 -> 20.2 us).
+template <int E>
+__device__ __forceinline__ int wave_share(int want, int valid, int wave) {
+    if (valid == SS_BLOCK * E) return (want + SS_WAVES - 1) / SS_WAVES;
+    // whole 1024-column chunks give every wave 256 columns; the last chunk fills the waves in turn
+    const int rest = valid & (SS_BLOCK * 4 - 1);
+    const int n = (valid >> 10) * 256 + min(max(rest - 256 * wave, 0), 256);
+    return (want * n + valid - 1) / valid;
+}
+
 // Tile stage. Greedy rows store one u32 per tile: (key << 16) | (0xffff - column offset), whose
 // maximum picks the lowest column among equal maxima. Other rows store their exact top-128 as the
 // same composites, sorted in descending order (0 for absent entries), at scratch[tile * 128 ...].
 //
 // The top-128 is found without a selection over the whole tile. Lower bound: per wave, the
 // largest multiple of 4, t, such that the lanes' largest and second-largest keys include at least
-// 32 keys >= t,
-// so the wave holds at least 32 keys >= t; with lo the smallest of the four wave bounds, the tile
-// holds at least 128 keys >= lo. Every wave then collects its survivors (keys >= lo: about 160 of
+// the wave's share of the 128 (wave_share: 32 in a full tile) keys >= t; with lo the smallest of
+// the waves' bounds, the tile holds at least 128 keys >= lo. Every wave then collects its survivors (keys >= lo: about 160 of
 // a 4096-wide tile of unstructured logits, 30-50 per wave) in its own LDS region and sorts them;
 // a two-level merge tree keeps the top-128 of the four sorted runs.
 //
@@ -1044,9 +1057,12 @@ __device__ __forceinline__ uint32_t wave_survivors_masked(TileSmem<E> &sm, const
 // order with one workgroup scan; the waves then collect the elements with key > T and the first
 // 128 - #(key > T) of the ties: exactly the first 128 of the stable descending order, so no wave
 // can exceed 128.
-template <int E>
+//
+// TOPK (the bounded top-k): only the first k <= 128 of the tile's list are stored, at
+// scratch[tile * k ...].
+template <int E, bool TOPK = false>
 __device__ __forceinline__ void tile_stage(TileSmem<E> &sm, bool greedy, const Keys<E> &keys,
-                                           uint32_t *scr, int tile, int valid) {
+                                           uint32_t *scr, int tile, int valid, int k = SS_K) {
     const int lane = lane_id();
     const int wave = (int)threadIdx.x >> 6;
     if (greedy) {
@@ -1067,11 +1083,25 @@ __device__ __forceinline__ void tile_stage(TileSmem<E> &sm, bool greedy, const K
         return;
     }
     typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    // keys the wave's bound must leave: its share of the list's length by its valid columns
+    const int want = TOPK ? k : SS_K;
+    const int need = wave_share<E>(want, valid, __builtin_amdgcn_readfirstlane(wave));
     uint32_t bound = 0;
-    if constexpr (E >= 64) {
+    if (valid <= SS_BLOCK * 4 && valid < SS_BLOCK * E) {
+        // One partly filled chunk: the lane's four keys are all it holds, and a wave may hold most
+        // of the tile's columns, so that its share exceeds what its lanes' largest keys can bound
+        // (and all 16 key bits count: a share near 128 leaves a run of 128 no slack).
+#pragma unroll 1
+        for (int b = 15; b >= 0; --b) {
+            const uint32_t c = bound | (1u << b);
+            const int n = (int)(__popcll(__ballot(keys.ge(0, c))) + __popcll(__ballot(keys.ge(1, c))) +
+                                __popcll(__ballot(keys.ge(2, c))) + __popcll(__ballot(keys.ge(3, c))));
+            if (n >= need) bound = c;
+        }
+    } else if constexpr (E >= 64) {
         // At 64 elements a lane its largest key alone bounds well: the bound is the largest t (to
-        // 14 of the 16 key bits) that at least 32 lane maxima reach, so the wave holds at least 32
-        // keys >= t. One packed max a pair, one ballot a bisection step.
+        // 14 of the 16 key bits) that at least `need` lane maxima reach, so the wave holds at least
+        // `need` keys >= t. One packed max a pair, one ballot a bisection step.
         u16x2 a1 = {0, 0};
 #pragma unroll
         for (int i = 0; i < E / 2; ++i) a1 = __builtin_elementwise_max(a1, __builtin_bit_cast(u16x2, keys.p[i]));
@@ -1079,7 +1109,7 @@ __device__ __forceinline__ void tile_stage(TileSmem<E> &sm, bool greedy, const K
 #pragma unroll
         for (int b = 15; b >= 2; --b) {
             const uint32_t c = bound | (1u << b);
-            if (__popcll(__ballot(m1 >= c)) >= 32) bound = c;
+            if ((int)__popcll(__ballot(m1 >= c)) >= need) bound = c;
         }
     } else {
         // The lane's largest and second-largest key: the two largest of its even and of its odd
@@ -1099,7 +1129,7 @@ __device__ __forceinline__ void tile_stage(TileSmem<E> &sm, bool greedy, const K
 #pragma unroll
         for (int b = 15; b >= 2; --b) {
             const uint32_t c = bound | (1u << b);
-            if (__popcll(__ballot(m1 >= c)) + __popcll(__ballot(m2 >= c)) >= 32) bound = c;
+            if ((int)(__popcll(__ballot(m1 >= c)) + __popcll(__ballot(m2 >= c))) >= need) bound = c;
         }
     }
     // A wave with fewer than 32 keys above -inf among its lanes' largest ones (few tokens admitted
@@ -1109,6 +1139,7 @@ __device__ __forceinline__ void tile_stage(TileSmem<E> &sm, bool greedy, const K
     // waves' counts add up to it, which the check after the survivor pass makes. A tile of fewer
     // than 128 valid columns (`valid`) keeps the plain bounds: all of its columns survive.
     if (bound <= KEY_NEG_INF && valid >= SS_K) bound = KEY_NEG_INF + 1;
+    if (need == 0) bound = 0xfffcu;  // no columns: no part in the tile's bound
     if (lane == 0) sm.red[wave] = bound;
     __syncthreads();
     const uint32_t lo = min(min(sm.red[0], sm.red[1]), min(sm.red[2], sm.red[3]));
@@ -1227,14 +1258,19 @@ __device__ __forceinline__ void tile_stage(TileSmem<E> &sm, bool greedy, const K
         uint32_t c0 = max(sm.run2[0][2 * lane], sm.run2[1][127 - 2 * lane]);
         uint32_t c1 = max(sm.run2[0][2 * lane + 1], sm.run2[1][126 - 2 * lane]);
         wave_bitonic128_desc<128>(c0, c1);
-        *(uint2 *)(scr + tile * SS_K + 2 * lane) = make_uint2(c0, c1);
+        if constexpr (TOPK) {
+            if (2 * lane < k) scr[(int64_t)tile * k + 2 * lane] = c0;
+            if (2 * lane + 1 < k) scr[(int64_t)tile * k + 2 * lane + 1] = c1;
+        } else {
+            *(uint2 *)(scr + tile * SS_K + 2 * lane) = make_uint2(c0, c1);
+        }
         if (__builtin_expect(fill, 0)) {
             // The merged survivors took positions 0 .. survivors - 1 and zeros the rest; the -inf
             // key of column c = 4 * lane + i (c < 256) with rank r among them overwrites position
-            // survivors + r while r < 128 - survivors. Its keys come from the survivor pass's
+            // survivors + r while that is below the list's length. Its keys come from the survivor pass's
             // spill (nothing has written over them since). The list's store, which other lanes
             // of the wave made to the same positions, completes before these issue (vmcnt(0)).
-            const uint32_t need = (uint32_t)SS_K - survivors;
+            const uint32_t limit = TOPK ? (uint32_t)k : (uint32_t)SS_K;
             const uint32_t w0 = sm.keys[0][lane], w1 = sm.keys[0][64 + lane];
             const uint32_t k4[4] = {w0 & 0xffffu, w0 >> 16, w1 & 0xffffu, w1 >> 16};
             uint32_t r = 0;
@@ -1244,8 +1280,9 @@ __device__ __forceinline__ void tile_stage(TileSmem<E> &sm, bool greedy, const K
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if (k4[i] == KEY_NEG_INF) {
-                    if (r < need)
-                        scr[tile * SS_K + survivors + r] = (KEY_NEG_INF << 16) | (0xffffu - (uint32_t)(4 * lane + i));
+                    const uint32_t at = survivors + r;
+                    if (at < limit)
+                        scr[(int64_t)tile * limit + at] = (KEY_NEG_INF << 16) | (0xffffu - (uint32_t)(4 * lane + i));
                     ++r;
                 }
             }

@@ -3,7 +3,8 @@
 // 1024-thread workgroup per row (topk_wide_kernel) for many rows of at most 32768 columns.
 //
 // Tile stage, grid rows * tiles: each workgroup turns block_n logits into order-preserving keys
-// and writes its exact top-k (ties to the lowest column) to the scratch row in column order.
+// (16 bits of bfloat16 logits, two to a register; 32 bits of float32 ones) and writes its exact
+// top-k (ties to the lowest column) to the scratch row, sorted.
 // Merge stage, grid rows: selects the row's top-k among the tiles * k candidates from a sample of
 // at most 512 (the first entries of every sorted list), completed list by list where the sample
 // was not exact and by a radix selection over every candidate where many lists were cut short;
@@ -32,21 +33,15 @@ template <>
 struct TopkTraits<false> {
     using Cand = uint32_t;
     static constexpr int KEYBITS = 16;
-    __device__ static uint32_t key_of(const void *p, int64_t off) {
-        return key16(((const uint16_t *)p)[off]);
-    }
-    __device__ static Cand pack(uint32_t key, int li) { return (key << 16) | (uint32_t)li; }
+    // the tile stage's composites: (key << 16) | (0xffff - column)
     __device__ static uint32_t cand_key(Cand c) { return c >> 16; }
-    __device__ static int cand_li(Cand c) { return (int)(c & 0xffffu); }
+    __device__ static int cand_li(Cand c) { return (int)(0xffffu - (c & 0xffffu)); }
 };
 
 template <>
 struct TopkTraits<true> {
     using Cand = uint64_t;
     static constexpr int KEYBITS = 32;
-    __device__ static uint32_t key_of(const void *p, int64_t off) {
-        return key32(__float_as_uint(((const float *)p)[off]));
-    }
     __device__ static Cand pack(uint32_t key, int li) { return ((uint64_t)key << 32) | (uint32_t)li; }
     __device__ static uint32_t cand_key(Cand c) { return (uint32_t)(c >> 32); }
     __device__ static int cand_li(Cand c) { return (int)(c & 0xffffffffu); }
@@ -296,9 +291,61 @@ __global__ __launch_bounds__(SS_BLOCK) void topk_merge_kernel(void *p_scratch, i
 }
 
 // ---------------------------------------------------------------------------------------------
-// Block selection: one workgroup holds a block of SS_BLOCK * E columns (E values per thread,
-// element j of thread t at column (j / 4) * 1024 + 4 t + j % 4 of the block, loaded as 16-byte fp32
-// / 8-byte bf16 chunks) and selects its top-k: the block is tile blockIdx.x % tiles of row
+// bfloat16 tile stage: tile blockIdx.x % tiles of row blockIdx.x / tiles, its exact top-k by the
+// fused kernels' tile selection (tile_stage) on 16-bit keys held two per register and 32-bit
+// composites. Selected as the float32 logits below (values widened to a register each, 64-bit
+// composites) a wave of a 16384-column tile took 1770 vector instructions; it takes 566, and the
+// kernel 17.2 us instead of 45.5 at 256 rows of 128256 (3.8 TB/s; bound by its instructions and the
+// four workgroups a CU that the spilled keys leave).
+// ---------------------------------------------------------------------------------------------
+template <bool VEC, int E>
+__global__ __launch_bounds__(SS_BLOCK) void topk_tiles_kernel(const uint16_t *p_logits, int64_t p_stride,
+                                                              int p_block_n, int p_vocab, int p_k, int tiles,
+                                                              uint32_t *p_scratch, int64_t p_stride_scratch) {
+    __shared__ TileSmem<E> sm;
+    const int row = (int)blockIdx.x / tiles;
+    const int tile = (int)blockIdx.x - row * tiles;
+    const int col0 = tile * p_block_n;
+    const uint16_t *lrow = p_logits + (int64_t)row * p_stride;
+    const int lane4 = 4 * (int)threadIdx.x;
+    u32x2 lw[E / 4];
+    if constexpr (VEC) {
+        load_logits_vec<E>(lrow, col0, p_vocab, lw);
+    } else {
+        const __amdgpu_buffer_rsrc_t rb = row_buffer(lrow, (int64_t)p_vocab * 2);
+#pragma unroll
+        for (int c = 0; c < E / 4; ++c) {
+            uint32_t h[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                h[i] = __builtin_amdgcn_raw_buffer_load_b16(rb, (lane4 + i) * 2, (col0 + c * (SS_BLOCK * 4)) * 2, NT);
+            lw[c].x = h[0] | (h[1] << 16);
+            lw[c].y = h[2] | (h[3] << 16);
+        }
+    }
+    Keys<E> keys;
+#pragma unroll
+    for (int c = 0; c < E / 4; ++c) {
+        keys.p[2 * c] = packed_keys(lw[c].x);
+        keys.p[2 * c + 1] = packed_keys(lw[c].y);
+    }
+    if (col0 + SS_BLOCK * E > p_vocab) {
+        // columns past the vocabulary are absent (key 0)
+#pragma unroll
+        for (int c = 0; c < E / 4; ++c) {
+            const int left = p_vocab - (col0 + c * (SS_BLOCK * 4) + lane4);  // columns of the chunk in it
+            keys.p[2 * c] &= (left > 0 ? 0xffffu : 0u) | (left > 1 ? 0xffff0000u : 0u);
+            keys.p[2 * c + 1] &= (left > 2 ? 0xffffu : 0u) | (left > 3 ? 0xffff0000u : 0u);
+        }
+    }
+    tile_stage<E, true>(sm, false, keys, p_scratch + (int64_t)row * p_stride_scratch, tile,
+                        min(p_block_n, p_vocab - col0), p_k);
+}
+
+// ---------------------------------------------------------------------------------------------
+// float32 tile stage: one workgroup holds a block of SS_BLOCK * E columns (E values per thread,
+// element j of thread t at column (j / 4) * 1024 + 4 t + j % 4 of the block, loaded as 16-byte
+// chunks) and selects its top-k: the block is tile blockIdx.x % tiles of row
 // blockIdx.x / tiles and its top-k goes to the scratch row as packed candidates for the merge
 // kernel.
 //
@@ -324,7 +371,7 @@ __device__ __forceinline__ uint32_t float_key(float v) {
     return u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
 }
 
-template <bool F32, bool VEC, int E>
+template <bool VEC, int E>
 __global__ __launch_bounds__(SS_BLOCK) void topk_block_kernel(const void *p_logits, int64_t p_stride,
                                                               int p_block_n, int p_vocab, int p_k, int tiles,
                                                               ss_topk_args a) {
@@ -337,16 +384,10 @@ __global__ __launch_bounds__(SS_BLOCK) void topk_block_kernel(const void *p_logi
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane4 = 4 * (int)threadIdx.x;
-    const int64_t bytes = (int64_t)V * (F32 ? 4 : 2);
-    const char *base = (const char *)p_logits + ((int64_t)row * p_stride + col0) * (F32 ? 4 : 2);
-    const __amdgpu_buffer_rsrc_t rb = row_buffer(base, bytes);
+    const __amdgpu_buffer_rsrc_t rb = row_buffer((const float *)p_logits + (int64_t)row * p_stride + col0, (int64_t)V * 4);
     // the block's top-k: packed candidates of the merge kernel
     auto emit = [&](int e, uint32_t key, int col) {
-        using Tr = TopkTraits<F32>;
-        typename Tr::Cand *scr = (typename Tr::Cand *)a.scratch + (int64_t)row * a.stride_scratch;
-        // absent elements (key 0) keep key 0 in the 16-bit packing too
-        const uint32_t pk = F32 ? key : key ? key16(__float_as_uint(__uint_as_float(unkey32(key))) >> 16) : 0u;
-        scr[tile * k + e] = Tr::pack(pk, col);
+        ((uint64_t *)a.scratch)[(int64_t)row * a.stride_scratch + tile * k + e] = TopkTraits<true>::pack(key, col);
     };
 
     // ---- the row, every load issued before any is used; columns past V read -inf -----------------
@@ -356,18 +397,11 @@ __global__ __launch_bounds__(SS_BLOCK) void topk_block_kernel(const void *p_logi
         const int col = c * (SS_BLOCK * 4) + lane4;
         uint32_t w[4];
         if (VEC) {
-            if (F32) {
-                const i32x4 q = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, col * 4, 0, NT));
-                w[0] = q.x; w[1] = q.y; w[2] = q.z; w[3] = q.w;
-            } else {
-                const u32x2 q = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rb, col * 2, 0, NT));
-                w[0] = q.x << 16; w[1] = q.x & 0xffff0000u; w[2] = q.y << 16; w[3] = q.y & 0xffff0000u;
-            }
+            const i32x4 q = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, col * 4, 0, NT));
+            w[0] = q.x; w[1] = q.y; w[2] = q.z; w[3] = q.w;
         } else {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                w[i] = F32 ? __builtin_amdgcn_raw_buffer_load_b32(rb, (col + i) * 4, 0, NT)
-                           : (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rb, (col + i) * 2, 0, NT) << 16;
+            for (int i = 0; i < 4; ++i) w[i] = __builtin_amdgcn_raw_buffer_load_b32(rb, (col + i) * 4, 0, NT);
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[4 * c + i] = col + i < V ? __uint_as_float(w[i]) : -INFINITY;
@@ -743,14 +777,22 @@ static int launch_topk_rows(const ss_topk_args *a) {
     return hipGetLastError() == hipSuccess ? SS_OK : SS_ERR_LAUNCH;
 }
 
+template <bool F32, bool VEC, int E>
+static void launch_topk_tile(const ss_topk_args *a, int tiles, dim3 grid, hipStream_t s) {
+    if constexpr (F32)
+        hipLaunchKernelGGL((topk_block_kernel<VEC, E>), grid, dim3(SS_BLOCK), 0, s, a->logits, a->stride_logits, a->block_n, a->vocab_size, a->k, tiles, *a);
+    else
+        hipLaunchKernelGGL((topk_tiles_kernel<VEC, E>), grid, dim3(SS_BLOCK), 0, s, (const uint16_t *)a->logits, a->stride_logits, a->block_n, a->vocab_size, a->k, tiles, (uint32_t *)a->scratch, a->stride_scratch);
+}
+
 template <bool F32, bool VEC>
-static int launch_topk_tiles(const ss_topk_args *a, int tiles, dim3 grid, dim3 block, hipStream_t s) {
+static int launch_topk_tiles(const ss_topk_args *a, int tiles, dim3 grid, hipStream_t s) {
     switch (a->block_n) {
-        case 1024: hipLaunchKernelGGL((topk_block_kernel<F32, VEC, 4>), grid, block, 0, s, a->logits, a->stride_logits, a->block_n, a->vocab_size, a->k, tiles, *a); break;
-        case 2048: hipLaunchKernelGGL((topk_block_kernel<F32, VEC, 8>), grid, block, 0, s, a->logits, a->stride_logits, a->block_n, a->vocab_size, a->k, tiles, *a); break;
-        case 4096: hipLaunchKernelGGL((topk_block_kernel<F32, VEC, 16>), grid, block, 0, s, a->logits, a->stride_logits, a->block_n, a->vocab_size, a->k, tiles, *a); break;
-        case 8192: hipLaunchKernelGGL((topk_block_kernel<F32, VEC, 32>), grid, block, 0, s, a->logits, a->stride_logits, a->block_n, a->vocab_size, a->k, tiles, *a); break;
-        case 16384: hipLaunchKernelGGL((topk_block_kernel<F32, VEC, 64>), grid, block, 0, s, a->logits, a->stride_logits, a->block_n, a->vocab_size, a->k, tiles, *a); break;
+        case 1024: launch_topk_tile<F32, VEC, 4>(a, tiles, grid, s); break;
+        case 2048: launch_topk_tile<F32, VEC, 8>(a, tiles, grid, s); break;
+        case 4096: launch_topk_tile<F32, VEC, 16>(a, tiles, grid, s); break;
+        case 8192: launch_topk_tile<F32, VEC, 32>(a, tiles, grid, s); break;
+        case 16384: launch_topk_tile<F32, VEC, 64>(a, tiles, grid, s); break;
         default: return SS_ERR_UNSUPPORTED;
     }
     return SS_OK;
@@ -761,8 +803,8 @@ static int launch_topk(const ss_topk_args *a, int tiles) {
     dim3 grid((unsigned)(a->rows * tiles)), block(SS_BLOCK);
     hipStream_t s = (hipStream_t)a->stream;
     // tiles start at multiples of block_n, so the 16 / 8-byte chunks of every tile stay aligned
-    const int st = topk_vec<F32>(a) ? launch_topk_tiles<F32, true>(a, tiles, grid, block, s)
-                                    : launch_topk_tiles<F32, false>(a, tiles, grid, block, s);
+    const int st = topk_vec<F32>(a) ? launch_topk_tiles<F32, true>(a, tiles, grid, s)
+                                    : launch_topk_tiles<F32, false>(a, tiles, grid, s);
     if (st != SS_OK) return st;
     if (hipGetLastError() != hipSuccess) return SS_ERR_LAUNCH;
     hipLaunchKernelGGL((topk_merge_kernel<F32>), dim3((unsigned)a->rows), block, 0, s, a->scratch, a->stride_scratch, a->vocab_size, a->k,
@@ -787,16 +829,18 @@ extern "C" int ss_topk(const ss_topk_args *a) {
     if (a->rows == 0) return SS_OK;
     if (a->strategy < SS_STRATEGY_AUTO || a->strategy > SS_STRATEGY_ROWWISE) return SS_ERR_INVALID_ARGUMENT;
     // One 1024-thread workgroup per row (one launch) serves rows of at most 32768 columns on
-    // request. AUTO takes it where it measured faster than the tile grid at the tuned widths: at
-    // least 48 rows of more than 16384 columns and k <= 32 (rows of 32000 columns at k = 32, back
-    // to back: fp32 48 rows 9.3 us against 9.6, 128 rows 9.7 against 11.3, 256 rows 12.1 against
-    // 17.0; bf16 64 rows 8.8 against 9.5). Fewer rows leave CUs idle while one CU streams each
-    // row (fp32 32 rows: 9.2 against 8.6 us), narrower rows leave most of a thread's 32 elements
-    // empty, and a larger k overflows the survivor list into the exact selection.
+    // request. AUTO takes it where it measured faster than the tile grid: float32, at least 48 rows
+    // of more than 16384 columns and k <= 32 (rows of 32000 columns at k = 32, back to back: 48 rows
+    // 9.3 us against 9.6, 128 rows 9.7 against 11.3, 256 rows 12.1 against 17.0). Fewer rows leave
+    // CUs idle while one CU streams each row (32 rows: 9.2 against 8.6 us), narrower rows leave most
+    // of a thread's 32 elements empty, and a larger k overflows the survivor list into the exact
+    // selection. bfloat16 rows take the tile grid (20000-32768 columns, k 8 and 32, at the best
+    // width: 48 rows 6.7-7.2 us against 8.4-9.0, 512 rows 11.7-12.9 against 16.6-17.9; only at 256
+    // rows are the two level, 8.9-9.8 against 8.9-9.6).
     if (a->strategy == SS_STRATEGY_ROWWISE && a->vocab_size > ss::TOPK_WIDE_THREADS * ss::TOPK_WIDE_E) return SS_ERR_UNSUPPORTED;
     const bool wide = a->strategy == SS_STRATEGY_ROWWISE ||
-                      (a->strategy == SS_STRATEGY_AUTO && a->rows >= 48 && a->k <= 32 && a->vocab_size > 16384 &&
-                       a->vocab_size <= ss::TOPK_WIDE_THREADS * ss::TOPK_WIDE_E);
+                      (a->strategy == SS_STRATEGY_AUTO && a->dtype == SS_DTYPE_F32 && a->rows >= 48 && a->k <= 32 &&
+                       a->vocab_size > 16384 && a->vocab_size <= ss::TOPK_WIDE_THREADS * ss::TOPK_WIDE_E);
     if (wide)
         return a->dtype == SS_DTYPE_F32 ? ss::launch_topk_rows<true>(a) : ss::launch_topk_rows<false>(a);
     return a->dtype == SS_DTYPE_F32 ? ss::launch_topk<true>(a, tiles)
