@@ -112,8 +112,8 @@ __global__ __launch_bounds__(SS_BLOCK) void multistep_tiles_kernel(const uint16_
     const int tile = blockIdx.x;
     // the request search, the slot and the indicator start from preloaded pointers
     const int pivot = request_pivot(p_cu, p_batch);
-    u32x2 lw[E / 4];
-    if (MODE != MODE_SCALAR) load_logits_vec<E>(p_logits + (int64_t)row * p_stride, tile * p_block_n, p_vocab, lw);
+    LogitChunk<MODE> lw[E / 4];
+    load_logits<E, (MODE & MODE_ANY) != 0>(p_logits + (int64_t)row * p_stride, tile * p_block_n, p_vocab, lw);
     const Request rq = resolve_request(a, row, pivot);
     const int step = row - rq.margin;
     if (!row_in_contract(a, rq, step)) return;
@@ -440,11 +440,6 @@ static int launch_multistep(const ss_multistep_args *a, int tiles) {
     return hipGetLastError() == hipSuccess ? SS_OK : SS_ERR_LAUNCH;
 }
 
-static bool aligned_ms(const void *p, int64_t stride, int bytes) {
-    if (!p) return true;
-    return ((uintptr_t)p % bytes) == 0 && (stride % 4) == 0;
-}
-
 }  // namespace ss
 
 extern "C" int ss_fused_multistep(const ss_multistep_args *a) {
@@ -467,10 +462,7 @@ extern "C" int ss_fused_multistep(const ss_multistep_args *a) {
     if (a->max_top_logprobs < 0 || a->max_top_logprobs > SS_MAX_K) return SS_ERR_INVALID_ARGUMENT;
     if (!a->philox.enabled && !a->gumbel) return SS_ERR_INVALID_ARGUMENT;
     if (a->rows == 0 || a->batch == 0) return SS_OK;
-    const bool vec = (a->vocab_size % 4) == 0 && aligned_ms(a->logits, a->stride_logits, 8) &&
-                     aligned_ms(a->decode_counts, a->stride_decode, 16) &&
-                     aligned_ms(a->context_counts, a->stride_context, 16) &&
-                     aligned_ms(a->logit_bias, a->stride_bias, 8);
-    if (!vec) return launch_multistep<MODE_SCALAR>(a, tiles);
-    return launch_multistep<MODE_DIRECT>(a, tiles);
+    const bool any = (a->vocab_size % 4) != 0 || !half_rows_on_dwords(a->logits, a->stride_logits) ||
+                     !half_rows_on_dwords(a->logit_bias, a->stride_bias);
+    return any ? launch_multistep<MODE_DIRECT | MODE_ANY>(a, tiles) : launch_multistep<MODE_DIRECT>(a, tiles);
 }

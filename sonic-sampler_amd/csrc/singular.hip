@@ -63,29 +63,29 @@ __global__ __launch_bounds__(SS_BLOCK) void singular_tiles_kernel(const uint16_t
     TileSmem<E> &sm = *reinterpret_cast<TileSmem<E> *>(tile_smem);
     uint32_t *grammar_words = tile_smem + TILE_OVERLAY / 4;
     int row = blockIdx.y, tile = blockIdx.x;
-    if (MODE != MODE_DIRECT && stage_words > 0) {
+    if ((MODE & MODE_GATHER) && stage_words > 0) {
         // the tiles of a row stage the same grammar row: run them on one XCD, whose L2 then
         // fetches it once
         const int v = xcd_grouped((int)(blockIdx.y * gridDim.x + blockIdx.x), (int)(gridDim.x * gridDim.y));
         row = v / tiles;
         tile = v - row * tiles;
     }
-    u32x2 lw[E / 4];
-    if (MODE != MODE_SCALAR) load_logits_vec<E>(p_logits + (int64_t)row * p_stride, tile * p_block_n, p_vocab, lw);
+    LogitChunk<MODE> lw[E / 4];
+    load_logits<E, (MODE & MODE_ANY) != 0>(p_logits + (int64_t)row * p_stride, tile * p_block_n, p_vocab, lw);
     // the row's slot and indicator decide which planes the tile reads: through preloaded pointers
     const int slot = p_slots ? uniform_i32(p_slots, row) : row;
     const uint32_t ind = uniform_u16(p_ind, slot);
     RowState rs = singular_row_state(a, row, slot, ind);
     bool sync = false;
     const Uses u = row_uses(rs);
-    if (MODE != MODE_DIRECT && stage_words > 0 && u.g && u.remap) {
+    if ((MODE & MODE_GATHER) && stage_words > 0 && u.g && u.remap) {
         stage_grammar(rs.grammar, rs.vt, grammar_words);
         rs.glds = grammar_words;
         sync = true;
     }
     // the d2t targets of the tile's columns, requested while the grammar row is staged: the
     // workgroup barrier below then waits for both rounds of loads at once
-    constexpr bool PRE = MODE == MODE_GATHER_VEC && E <= 32;
+    constexpr bool PRE = (MODE & MODE_GATHER) && E <= 32;
     int32_t pre[PRE ? E : 1];
     if constexpr (PRE) {
         if (u.remap) load_d2t<E>(rs, tile * a.block_n, a.vocab_size, pre);
@@ -265,8 +265,8 @@ __global__ __launch_bounds__(SS_BLOCK) void singular_rowwise_kernel(ss_singular_
     extern __shared__ __align__(16) uint32_t grammar_words[];
     const int row = blockIdx.x;
     const uint16_t *lrow = a.logits + (int64_t)row * a.stride_logits;
-    u32x2 lw[E / 4];
-    if (MODE != MODE_SCALAR) load_logits_vec<E>(lrow, 0, a.vocab_size, lw);
+    LogitChunk<MODE> lw[E / 4];
+    load_logits<E, (MODE & MODE_ANY) != 0>(lrow, 0, a.vocab_size, lw);
     const int slot = a.slot_mapping ? uniform_i32(a.slot_mapping, row) : row;
     const uint32_t ind = uniform_u16(a.indicators, slot);
     RowState rs = singular_row_state(a, row, slot, ind);
@@ -285,18 +285,16 @@ __global__ __launch_bounds__(SS_BLOCK) void singular_rowwise_kernel(ss_singular_
     const bool greedy = (ind & IND_GREEDY) != 0;
 #pragma unroll 1
     for (int t = 0; t < tiles; ++t) {
-        u32x2 nx[E / 4];
-        if (MODE != MODE_SCALAR && t + 1 < tiles)
-            load_logits_vec<E>(lrow, (t + 1) * a.block_n, a.vocab_size, nx);
+        LogitChunk<MODE> nx[E / 4];
+        if (t + 1 < tiles)
+            load_logits<E, (MODE & MODE_ANY) != 0>(lrow, (t + 1) * a.block_n, a.vocab_size, nx);
         Keys<E> keys;
         prologue_keys<E, MODE>(rs, t * a.block_n, a.vocab_size, sm.tile.hist, lw, keys);
         tile_stage<E>(sm.tile, greedy, keys, sm.lists, t, min(a.block_n, a.vocab_size - t * a.block_n));
         // the next tile reuses the tile stage's memory, and the lists feed the row stage
         __syncthreads();
-        if (MODE != MODE_SCALAR) {
 #pragma unroll
-            for (int c = 0; c < E / 4; ++c) lw[c] = nx[c];
-        }
+        for (int c = 0; c < E / 4; ++c) lw[c] = nx[c];
     }
     const uint32_t *scr = sm.lists;
     const ListMap lm = make_list_map(tiles, 0, a.block_n);
@@ -381,11 +379,6 @@ static int launch_singular(const ss_singular_args *a, int tiles) {
     return SS_OK;
 }
 
-static bool aligned(const void *p, int64_t stride, int bytes_per_vec) {
-    if (!p) return true;
-    return ((uintptr_t)p % bytes_per_vec) == 0 && (stride % 4) == 0;
-}
-
 }  // namespace ss
 
 extern "C" int ss_fused_singular(const ss_singular_args *a) {
@@ -413,13 +406,11 @@ extern "C" int ss_fused_singular(const ss_singular_args *a) {
     if (a->return_logprobs && a->max_top_logprobs > 0 && a->top_values && !a->top_tokens)
         return SS_ERR_INVALID_ARGUMENT;
     if (a->rows == 0) return SS_OK;
-    // a shard whose offset is not a multiple of 32 columns cannot read grammar words and counts as
-    // aligned vectors: it takes the per-element gather layout
+    // a shard whose offset is not a multiple of 32 columns starts inside a grammar word: it takes the
+    // per-element gather layout
     const bool direct = a->d2t == nullptr && (world == 1 || (a->local_rank * a->shard_size) % 32 == 0);
-    const bool vec = (a->vocab_size % 4) == 0 && aligned(a->logits, a->stride_logits, 8) &&
-                     (!direct || (aligned(a->decode_counts, a->stride_decode, 16) &&
-                                  aligned(a->context_counts, a->stride_context, 16) &&
-                                  aligned(a->logit_bias, a->stride_bias, 8)));
+    const bool any = (a->vocab_size % 4) != 0 || !half_rows_on_dwords(a->logits, a->stride_logits) ||
+                     (direct && !half_rows_on_dwords(a->logit_bias, a->stride_bias));
     if (a->strategy < SS_STRATEGY_AUTO || a->strategy > SS_STRATEGY_ROWWISE) return SS_ERR_INVALID_ARGUMENT;
     if (a->strategy == SS_STRATEGY_ROWWISE && (tiles > ROWWISE_MAX_TILES || world > 1 || a->stages))
         return SS_ERR_UNSUPPORTED;
@@ -428,11 +419,11 @@ extern "C" int ss_fused_singular(const ss_singular_args *a) {
     // shape tried (config 4: 36 us for the row kernel against 23 + 7 us for the two launches).
     const bool rowwise = a->strategy == SS_STRATEGY_ROWWISE;
     if (rowwise) {
-        if (!vec) return launch_rowwise<MODE_SCALAR>(a, tiles);
-        return direct ? launch_rowwise<MODE_DIRECT>(a, tiles) : launch_rowwise<MODE_GATHER_VEC>(a, tiles);
+        if (any) return direct ? launch_rowwise<MODE_DIRECT | MODE_ANY>(a, tiles) : launch_rowwise<MODE_GATHER | MODE_ANY>(a, tiles);
+        return direct ? launch_rowwise<MODE_DIRECT>(a, tiles) : launch_rowwise<MODE_GATHER>(a, tiles);
     }
-    if (!vec) return launch_singular<MODE_SCALAR>(a, tiles);
-    return direct ? launch_singular<MODE_DIRECT>(a, tiles) : launch_singular<MODE_GATHER_VEC>(a, tiles);
+    if (any) return direct ? launch_singular<MODE_DIRECT | MODE_ANY>(a, tiles) : launch_singular<MODE_GATHER | MODE_ANY>(a, tiles);
+    return direct ? launch_singular<MODE_DIRECT>(a, tiles) : launch_singular<MODE_GATHER>(a, tiles);
 }
 
 namespace ss {

@@ -1,8 +1,9 @@
-// Host-side launch helper shared by the fused entry points.
+// Host-side launch helpers shared by the entry points.
 #pragma once
 
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
+#include <stdint.h>
 
 namespace ss {
 
@@ -16,6 +17,11 @@ inline void launch_timed(Kernel kernel, dim3 grid, dim3 block, size_t shared, hi
         hipExtLaunchKernelGGL(kernel, grid, block, shared, stream, (hipEvent_t)start, (hipEvent_t)end, 0, args...);
     else
         hipLaunchKernelGGL(kernel, grid, block, shared, stream, args...);
+}
+
+// Whether every row of a bf16 plane (or an absent one) starts on a dword.
+inline bool half_rows_on_dwords(const void *p, int64_t stride) {
+    return !p || ((uintptr_t)p % 4 == 0 && stride % 2 == 0);
 }
 
 }  // namespace ss

@@ -20,6 +20,7 @@ constexpr uint32_t IND_GRAMMAR = 0x001, IND_MULT = 0x002, IND_FREQ = 0x004, IND_
 
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
 
 struct SampleSmem {
     SelectSmem sel;
@@ -393,17 +394,53 @@ __device__ __forceinline__ Chain row_chain(const RowState &rs, const Uses &u, bo
     return k;
 }
 
-// The logits of one tile as 4-column words (VEC layout). They depend on the row only, so the
-// kernels issue them first, before the request state that decides how the other planes are read.
-template <int E>
-__device__ __forceinline__ void load_logits_vec(const uint16_t *lrow, int col0, int V,
-                                                u32x2 (&lw)[E / 4]) {
-    const __amdgpu_buffer_rsrc_t lg = row_buffer(lrow, (int64_t)V * 2);
+// A row of bf16 values read four columns at a time (columns 4 * lane + 1024 c of the tile). ANY:
+// rows that start at any 2-byte address and end at any column, as those of a vocabulary that 2 does
+// not divide do: each chunk is the three dwords around it (a dword buffer load needs no more than
+// dword alignment), shifted down by the row's odd half (HalfRow::words). Element by element, as
+// these rows were read before, a wave issued four times the loads and, at 48 decode rows of 50003
+// columns, the tile kernel took 20.2 us instead of 13.1.
+template <bool ANY>
+struct HalfRow;
+
+template <>
+struct HalfRow<false> {
+    using Raw = u32x2;
+    __amdgpu_buffer_rsrc_t rb;
+    __device__ __forceinline__ HalfRow(const uint16_t *row, int n) : rb(row_buffer(row, (int64_t)n * 2)) {}
+    __device__ __forceinline__ Raw load(int voff, int soff) const {
+        return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rb, voff, soff, NT));
+    }
+    static __device__ __forceinline__ u32x2 words(const Raw &r, const uint16_t *) { return r; }
+};
+
+template <>
+struct HalfRow<true> {
+    using Raw = u32x3;
+    __amdgpu_buffer_rsrc_t rb;
+    // from the dword that holds the row's first half to the one that holds its last, both mapped
+    // whole (a dword never crosses a page)
+    __device__ __forceinline__ HalfRow(const uint16_t *row, int n)
+        : rb(row_buffer((const void *)((uintptr_t)row & ~(uintptr_t)3),
+                        row ? ((int64_t)n * 2 + (int64_t)((uintptr_t)row & 2) + 3) & ~(int64_t)3 : 0)) {}
+    __device__ __forceinline__ Raw load(int voff, int soff) const {
+        return __builtin_bit_cast(u32x3, __builtin_amdgcn_raw_buffer_load_b96(rb, voff, soff, NT));
+    }
+    static __device__ __forceinline__ u32x2 words(const Raw &r, const uint16_t *row) {
+        const uint32_t sh = ((uint32_t)(uintptr_t)row & 2u) << 3;  // 16 for a row at an odd half
+        return u32x2{__builtin_amdgcn_alignbit(r.y, r.x, sh), __builtin_amdgcn_alignbit(r.z, r.y, sh)};
+    }
+};
+
+// The logits of one tile as 4-column chunks. They depend on the row only, so the kernels issue
+// them first, before the request state that decides how the other planes are read.
+template <int E, bool ANY>
+__device__ __forceinline__ void load_logits(const uint16_t *lrow, int col0, int V,
+                                            typename HalfRow<ANY>::Raw (&lw)[E / 4]) {
+    const HalfRow<ANY> lg(lrow, V);
     const int lane4 = (int)threadIdx.x * 4;
 #pragma unroll
-    for (int c = 0; c < E / 4; ++c)
-        lw[c] = __builtin_bit_cast(
-            u32x2, __builtin_amdgcn_raw_buffer_load_b64(lg, lane4 * 2, (col0 + c * (SS_BLOCK * 4)) * 2, NT));
+    for (int c = 0; c < E / 4; ++c) lw[c] = lg.load(lane4 * 2, (col0 + c * (SS_BLOCK * 4)) * 2);
 }
 
 // Reads at workgroup-uniform addresses through the constant address space, which the compiler
@@ -463,57 +500,59 @@ __device__ __forceinline__ uint32_t row_params(const uint16_t *ind, const int32_
     return v;
 }
 
-// Direct layout (no d2t remap, vocabulary a multiple of 4, 8 / 16-byte aligned rows): the side
-// planes of one tile -- grammar words, decode and context counts, bias -- as loaded words.
-template <int E>
+// Direct layout (no d2t remap): the side planes of one tile -- grammar words, decode and context
+// counts, bias -- as loaded words.
+template <int E, bool ANY>
 struct Planes {
-    u32x2 bw[E / 4];
+    typename HalfRow<ANY>::Raw bw[E / 4];
     i32x4 dw[E / 4], cw[E / 4];
     uint32_t gw[E / 4];
 };
 
 // Issues every side-plane load of the tile before any loaded word is consumed. A plane that is
 // off reads through an empty buffer, which returns zeros without touching memory.
-template <int E>
+template <int E, bool ANY>
 __device__ __forceinline__ void issue_planes(const RowState &rs, const Uses &u, bool on, int col0,
-                                             Planes<E> &pl) {
+                                             Planes<E, ANY> &pl) {
     const int lane4 = (int)threadIdx.x * 4;
     const bool g = on && u.g, rep = on && u.rep, mult = on && u.mult, bias = on && u.bias;
     const __amdgpu_buffer_rsrc_t gb =
         row_buffer(g ? rs.grammar : nullptr, g ? (int64_t)((rs.vt + 31) >> 5) * 4 : 0);
     const __amdgpu_buffer_rsrc_t db = row_buffer(rep ? rs.dec : nullptr, rep ? (int64_t)rs.vt * 4 : 0);
     const __amdgpu_buffer_rsrc_t cb = row_buffer(mult ? rs.ctx : nullptr, mult ? (int64_t)rs.vt * 4 : 0);
-    const __amdgpu_buffer_rsrc_t bb = row_buffer(bias ? rs.bias : nullptr, bias ? (int64_t)rs.vt * 2 : 0);
+    const HalfRow<ANY> bb(bias ? rs.bias : nullptr, bias ? rs.vt : 0);
 #pragma unroll
     for (int c = 0; c < E / 4; ++c) {
         const int base = col0 + c * (SS_BLOCK * 4);  // uniform, a multiple of 32
         pl.dw[c] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(db, lane4 * 4, base * 4, NT));
         pl.cw[c] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(cb, lane4 * 4, base * 4, NT));
-        pl.bw[c] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(bb, lane4 * 2, base * 2, NT));
+        pl.bw[c] = bb.load(lane4 * 2, base * 2);
         pl.gw[c] = __builtin_amdgcn_raw_buffer_load_b32(gb, (lane4 >> 5) * 4, (base >> 5) * 4, 0);
     }
 }
 
-template <int E>
+template <int E, bool ANY>
 __device__ __forceinline__ void direct_keys(const RowState &rs, const Uses &u, int col0, int V,
-                                            const int32_t *hist, const u32x2 (&lw_in)[E / 4],
-                                            const Planes<E> &pl, Keys<E> &keys) {
+                                            const int32_t *hist,
+                                            const typename HalfRow<ANY>::Raw (&lw_in)[E / 4],
+                                            const Planes<E, ANY> &pl, Keys<E> &keys) {
     constexpr int NCH = E / 4;
     const int lane4 = (int)threadIdx.x * 4;
     bool all_exc;
     const Chain k = row_chain(rs, u, all_exc);
     // logits and bias stay in their loaded bf16 pairs and are widened where they are used
-    u32x2 lw[NCH];
+    u32x2 lw[NCH], bw[NCH];
     bool ok[E];
     int32_t dec[E], ctx[E];
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
-        lw[c] = lw_in[c];
-        const bool in = col0 + c * (SS_BLOCK * 4) + lane4 < V;
+        lw[c] = HalfRow<ANY>::words(lw_in[c], rs.logits);
+        bw[c] = HalfRow<ANY>::words(pl.bw[c], rs.bias);
+        const int col = col0 + c * (SS_BLOCK * 4) + lane4;
         dec[4 * c + 0] = pl.dw[c].x; dec[4 * c + 1] = pl.dw[c].y; dec[4 * c + 2] = pl.dw[c].z; dec[4 * c + 3] = pl.dw[c].w;
         ctx[4 * c + 0] = pl.cw[c].x; ctx[4 * c + 1] = pl.cw[c].y; ctx[4 * c + 2] = pl.cw[c].z; ctx[4 * c + 3] = pl.cw[c].w;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ok[4 * c + i] = in;
+        for (int i = 0; i < 4; ++i) ok[4 * c + i] = (ANY ? col + i : col) < V;
     }
     if (u.g) {
         // a masked element becomes bf16 -inf (0xff80) in place
@@ -545,30 +584,32 @@ __device__ __forceinline__ void direct_keys(const RowState &rs, const Uses &u, i
         return __uint_as_float((j & 1) ? (w & 0xffff0000u) : (w << 16));
     };
     auto bb = [&](int j) {
-        const uint32_t w = (j & 2) ? pl.bw[j >> 2].y : pl.bw[j >> 2].x;
+        const uint32_t w = (j & 2) ? bw[j >> 2].y : bw[j >> 2].x;
         return (j & 1) ? (w & 0xffff0000u) : (w << 16);
     };
     // the bias word of the element's pair, shifted so that -0 in the high half does not count
-    auto bw = [&](int j) { return ((j & 2) ? pl.bw[j >> 2].y : pl.bw[j >> 2].x) << 1; };
+    auto bz = [&](int j) { return ((j & 2) ? bw[j >> 2].y : bw[j >> 2].x) << 1; };
     auto pair = [&](int j) { return (j & 2) ? lw[j >> 2].y : lw[j >> 2].x; };
     finish_keys<E>(k, all_exc, col0 + SS_BLOCK * E > V, x, pair, all_exc || u.rep || u.mult || u.bias, ok,
-                   dec, ctx, bb, bw, keys);
+                   dec, ctx, bb, bz, keys);
 }
 
 // Direct layout, row with every side plane off (no grammar, penalty or bias): the keys come from
 // the logits alone and no other plane is read.
-template <int E>
+template <int E, bool ANY>
 __device__ __forceinline__ void plain_keys(const RowState &rs, const Uses &u, int col0, int V,
-                                           const u32x2 (&lw)[E / 4], Keys<E> &keys) {
+                                           const typename HalfRow<ANY>::Raw (&lw_in)[E / 4], Keys<E> &keys) {
     const int lane4 = (int)threadIdx.x * 4;
     bool all_exc;
     const Chain k = row_chain(rs, u, all_exc);
+    u32x2 lw[E / 4];
     bool ok[E];
 #pragma unroll
     for (int c = 0; c < E / 4; ++c) {
-        const bool in = col0 + c * (SS_BLOCK * 4) + lane4 < V;
+        lw[c] = HalfRow<ANY>::words(lw_in[c], rs.logits);
+        const int col = col0 + c * (SS_BLOCK * 4) + lane4;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ok[4 * c + i] = in;
+        for (int i = 0; i < 4; ++i) ok[4 * c + i] = (ANY ? col + i : col) < V;
     }
     const int32_t zero[E] = {};
     auto x = [&](int j) {
@@ -580,15 +621,16 @@ __device__ __forceinline__ void plain_keys(const RowState &rs, const Uses &u, in
     finish_keys<E>(k, false, col0 + SS_BLOCK * E > V, x, pair, false, ok, zero, zero, none, none, keys);
 }
 
-// General layout: d2t-remapped columns (gathers through the target vocabulary) or unaligned rows.
+// Gather layout: columns remapped by d2t into the target vocabulary, or a shard that starts inside
+// a grammar word.
 // Largest grammar row that stage_grammar copies into workgroup memory, and the 16-byte quads it
 // stages for a vt-token vocabulary.
 constexpr int SS_STAGE_MAX_WORDS = 8192;
 
 __host__ __device__ __forceinline__ int stage_quads(int vt) { return (((vt + 31) >> 5) + 3) >> 2; }
 
-// The d2t targets of a tile's E columns (GATHER_VEC layout: each 4-column chunk is one 16-byte
-// load), for callers that issue them ahead of the prologue.
+// The d2t targets of a tile's E columns (each 4-column chunk is one 16-byte load), for callers that
+// issue them ahead of the prologue.
 template <int E>
 __device__ __forceinline__ void load_d2t(const RowState &rs, int col0, int V, int32_t (&tcol)[E]) {
     const __amdgpu_buffer_rsrc_t m = row_buffer(rs.d2t, (int64_t)(rs.shard + V) * 4);
@@ -603,9 +645,10 @@ __device__ __forceinline__ void load_d2t(const RowState &rs, int col0, int V, in
 
 // PRE: the d2t targets of the E columns come in `pre` (load_d2t, issued by the caller before the
 // grammar staging's barrier, so that both round trips overlap) instead of being loaded here.
-template <int E, bool VEC, bool PRE = false>
+template <int E, bool ANY, bool PRE = false>
 __device__ __forceinline__ void gather_keys(const RowState &rs, const Uses &u, int col0, int V,
-                                            const int32_t *hist, const u32x2 (&lw)[E / 4],
+                                            const int32_t *hist,
+                                            const typename HalfRow<ANY>::Raw (&lw)[E / 4],
                                             Keys<E> &keys, const int32_t *pre = nullptr) {
     constexpr int NCH = E / 4;
     const int lane4 = (int)threadIdx.x * 4;
@@ -616,25 +659,12 @@ __device__ __forceinline__ void gather_keys(const RowState &rs, const Uses &u, i
     // they are used, they would hold one register per element
     u32x2 lv[NCH];
     bool ok[E];
-    const __amdgpu_buffer_rsrc_t lg = row_buffer(rs.logits, (int64_t)V * 2);
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
-        const int base = col0 + c * (SS_BLOCK * 4);  // uniform
-        if (VEC) {
-            lv[c] = lw[c];
-            const bool in = base + lane4 < V;
+        lv[c] = HalfRow<ANY>::words(lw[c], rs.logits);
+        const int col = col0 + c * (SS_BLOCK * 4) + lane4;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) ok[4 * c + i] = in;
-        } else {
-            uint32_t h[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                h[i] = __builtin_amdgcn_raw_buffer_load_b16(lg, (lane4 + i) * 2, base * 2, NT);
-                ok[4 * c + i] = base + lane4 + i < V;
-            }
-            lv[c].x = h[0] | (h[1] << 16);
-            lv[c].y = h[2] | (h[3] << 16);
-        }
+        for (int i = 0; i < 4; ++i) ok[4 * c + i] = (ANY ? col + i : col) < V;
     }
 
     int32_t dec[E], ctx[E];
@@ -654,19 +684,7 @@ __device__ __forceinline__ void gather_keys(const RowState &rs, const Uses &u, i
 #pragma unroll
             for (int j = 0; j < E; ++j) tcol[j] = pre[j];
         } else if (u.remap) {
-            const __amdgpu_buffer_rsrc_t m = row_buffer(rs.d2t, (int64_t)(rs.shard + V) * 4);
-            if (VEC) {
-                // the 4 columns of a chunk are consecutive (and V % 4 == 0): one 16-byte load
-#pragma unroll
-                for (int c = 0; c < NCH; ++c) {
-                    const i32x4 t = __builtin_bit_cast(
-                        i32x4, __builtin_amdgcn_raw_buffer_load_b128(m, lane4 * 4, (rs.shard + col0 + c * (SS_BLOCK * 4)) * 4, 0));
-                    tcol[4 * c + 0] = t.x; tcol[4 * c + 1] = t.y; tcol[4 * c + 2] = t.z; tcol[4 * c + 3] = t.w;
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < E; ++j) tcol[j] = __builtin_amdgcn_raw_buffer_load_b32(m, tcol[j] * 4, 0, 0);
-            }
+            load_d2t<E>(rs, col0, V, tcol);
         }
         // a masked element becomes bf16 -inf (0xff80) in place; a column outside the target
         // vocabulary (negative, or at or past it) reads 0 (masked) on either path
@@ -786,11 +804,14 @@ __device__ __forceinline__ void stage_grammar_finish(int vt, uint32_t *dst) {
 }
 
 // Memory layouts of the prologue, fixed per launch by the host:
-//   MODE_DIRECT      no d2t, vocabulary a multiple of 4, 8 / 16-byte aligned rows: vector loads
-//                    of every plane, all issued before any is consumed;
-//   MODE_GATHER_VEC  d2t given: vector logit loads, per-element gathers through the target vocab;
-//   MODE_SCALAR      anything else: per-element loads throughout.
-enum { MODE_DIRECT = 0, MODE_GATHER_VEC = 1, MODE_SCALAR = 2 };
+//   MODE_DIRECT   no d2t: vector loads of every plane, all issued before any is consumed;
+//   MODE_GATHER   d2t given: vector logit loads, per-element gathers through the target vocab;
+// | MODE_ANY      for a vocabulary that is not a multiple of 4, or bf16 rows that do not all start
+//                 on a dword (HalfRow<true>).
+enum { MODE_DIRECT = 0, MODE_GATHER = 1, MODE_ANY = 2 };
+
+template <int MODE>
+using LogitChunk = typename HalfRow<(MODE & MODE_ANY) != 0>::Raw;
 
 // Gather pass H of a tile (elements j + 16 H, 4 H chunks of 1024 columns further) and the passes
 // after it. H is a template parameter so that the keys each pass writes keep constant indices: a
@@ -798,35 +819,32 @@ enum { MODE_DIRECT = 0, MODE_GATHER_VEC = 1, MODE_SCALAR = 2 };
 // would index the key array at run time and place it in scratch memory.
 template <int E, int MODE, int H>
 __device__ __forceinline__ void gather_pass(const RowState &rs, const Uses &u, int col0, int V,
-                                            const int32_t *hist, const u32x2 (&lw)[E / 4], Keys<E> &keys) {
+                                            const int32_t *hist, Keys<E> &keys) {
+    constexpr bool ANY = (MODE & MODE_ANY) != 0;
     if constexpr (H < E / 16) {
-        u32x2 lh[4];
-        if constexpr (MODE != MODE_SCALAR && E >= 64) {
-            load_logits_vec<16>(rs.logits, col0 + 4 * 4 * SS_BLOCK * H, V, lh);
-        } else if constexpr (MODE != MODE_SCALAR) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) lh[c] = lw[4 * H + c];
-        }
+        LogitChunk<MODE> lh[4];
+        load_logits<16, ANY>(rs.logits, col0 + 4 * 4 * SS_BLOCK * H, V, lh);
         Keys<16> kh;
-        gather_keys<16, MODE == MODE_GATHER_VEC>(rs, u, col0 + 4 * 4 * SS_BLOCK * H, V, hist, lh, kh);
+        gather_keys<16, ANY>(rs, u, col0 + 4 * 4 * SS_BLOCK * H, V, hist, lh, kh);
 #pragma unroll
         for (int i = 0; i < 8; ++i) keys.p[8 * H + i] = kh.p[i];
-        gather_pass<E, MODE, H + 1>(rs, u, col0, V, hist, lw, keys);
+        gather_pass<E, MODE, H + 1>(rs, u, col0, V, hist, keys);
     }
 }
 
 // Streams one tile of one row through the processor chain and returns the keys (0 = absent).
-// `lw` holds the tile's logits from load_logits_vec unless MODE is MODE_SCALAR.
-// PRE (GATHER_VEC, E <= 32): the d2t targets of the tile's columns come in `pre` (load_d2t).
+// `lw` holds the tile's logits from load_logits.
+// PRE (gather layout, E <= 32): the d2t targets of the tile's columns come in `pre` (load_d2t).
 template <int E, int MODE, bool PRE = false>
 __device__ __forceinline__ void prologue_keys(const RowState &rs, int col0, int V,
-                                              const int32_t *hist, const u32x2 (&lw)[E / 4],
+                                              const int32_t *hist, const LogitChunk<MODE> (&lw)[E / 4],
                                               Keys<E> &keys, const int32_t *pre = nullptr) {
-    static_assert(!PRE || (MODE == MODE_GATHER_VEC && E <= 32), "pre-loaded d2t targets: GATHER_VEC, E <= 32");
+    constexpr bool ANY = (MODE & MODE_ANY) != 0;
+    static_assert(!PRE || ((MODE & MODE_GATHER) && E <= 32), "pre-loaded d2t targets: gather layout, E <= 32");
     const Uses u = row_uses(rs);
-    if constexpr (MODE == MODE_DIRECT) {
+    if constexpr (!(MODE & MODE_GATHER)) {
         if (!(u.g || u.rep || u.mult || u.bias)) {
-            plain_keys<E>(rs, u, col0, V, lw, keys);
+            plain_keys<E, ANY>(rs, u, col0, V, lw, keys);
         } else if constexpr (E >= 32) {
             // The processor chain in 4096-column passes: element j of pass h is element j + 16 h
             // of the tile (4 h chunks of 1024 columns further). Its per-element state for all E
@@ -837,49 +855,44 @@ __device__ __forceinline__ void prologue_keys(const RowState &rs, int col0, int 
             for (int h = 0; h < E / 16; ++h) {
                 // at E = 64 a pass reloads its logits with its planes (in the same round of loads):
                 // the preloaded ones would stay live through every pass
-                u32x2 lh[4];
+                LogitChunk<MODE> lh[4];
                 if constexpr (E >= 64) {
-                    load_logits_vec<16>(rs.logits, col0 + 4 * 4 * SS_BLOCK * h, V, lh);
+                    load_logits<16, ANY>(rs.logits, col0 + 4 * 4 * SS_BLOCK * h, V, lh);
                 } else {
 #pragma unroll
                     for (int c = 0; c < 4; ++c) lh[c] = lw[4 * h + c];
                 }
-                Planes<16> pl;
-                issue_planes<16>(rs, u, true, rs.shard + col0 + 4 * 4 * SS_BLOCK * h, pl);
+                Planes<16, ANY> pl;
+                issue_planes<16, ANY>(rs, u, true, rs.shard + col0 + 4 * 4 * SS_BLOCK * h, pl);
                 Keys<16> kh;
-                direct_keys<16>(rs, u, col0 + 4 * 4 * SS_BLOCK * h, V, hist, lh, pl, kh);
+                direct_keys<16, ANY>(rs, u, col0 + 4 * 4 * SS_BLOCK * h, V, hist, lh, pl, kh);
 #pragma unroll
                 for (int i = 0; i < 8; ++i) keys.p[8 * h + i] = kh.p[i];
             }
         } else {
-            Planes<E> pl;
-            issue_planes<E>(rs, u, true, rs.shard + col0, pl);
-            direct_keys<E>(rs, u, col0, V, hist, lw, pl, keys);
+            Planes<E, ANY> pl;
+            issue_planes<E, ANY>(rs, u, true, rs.shard + col0, pl);
+            direct_keys<E, ANY>(rs, u, col0, V, hist, lw, pl, keys);
         }
-    } else if constexpr ((E >= 32 && MODE == MODE_GATHER_VEC) || E >= 64) {
-        // 4096-column passes, as above: the gathered columns and planes of all 32 elements at
-        // once would hold 156 VGPRs (three waves per SIMD).
-        if constexpr (E >= 64) {
-            gather_pass<E, MODE, 0>(rs, u, col0, V, hist, lw, keys);
-        } else {
-            // two passes, which the compiler unrolls (and schedules in fewer registers than the
-            // recursive form: 96 VGPRs against 102 at E = 32)
+    } else if constexpr (E >= 64) {
+        // 4096-column passes, as above: the gathered columns and planes of all elements at once
+        // would hold 156 VGPRs at E = 32 (three waves per SIMD).
+        gather_pass<E, MODE, 0>(rs, u, col0, V, hist, keys);
+    } else if constexpr (E >= 32) {
+        // two passes, which the compiler unrolls (and schedules in fewer registers than the
+        // recursive form: 96 VGPRs against 102 at E = 32)
 #pragma unroll
-            for (int h = 0; h < E / 16; ++h) {
-                u32x2 lh[4];
-                if constexpr (MODE != MODE_SCALAR) {
+        for (int h = 0; h < E / 16; ++h) {
+            LogitChunk<MODE> lh[4];
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) lh[c] = lw[4 * h + c];
-                }
-                Keys<16> kh;
-                gather_keys<16, MODE == MODE_GATHER_VEC, PRE>(rs, u, col0 + 4 * 4 * SS_BLOCK * h, V, hist, lh, kh,
-                                                              PRE ? pre + 16 * h : nullptr);
+            for (int c = 0; c < 4; ++c) lh[c] = lw[4 * h + c];
+            Keys<16> kh;
+            gather_keys<16, ANY, PRE>(rs, u, col0 + 4 * 4 * SS_BLOCK * h, V, hist, lh, kh, PRE ? pre + 16 * h : nullptr);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) keys.p[8 * h + i] = kh.p[i];
-            }
+            for (int i = 0; i < 8; ++i) keys.p[8 * h + i] = kh.p[i];
         }
     } else {
-        gather_keys<E, MODE == MODE_GATHER_VEC, PRE>(rs, u, col0, V, hist, lw, keys, pre);
+        gather_keys<E, ANY, PRE>(rs, u, col0, V, hist, lw, keys, pre);
     }
 }
 

@@ -10,6 +10,7 @@
 // was not exact and by a radix selection over every candidate where many lists were cut short;
 // sorts them by (value desc, column asc) with wave64 bitonic networks and writes values / indices
 // densely as [rows, k].
+#include "ss_launch.h"
 #include "ss_sampling.h"
 #include "../../include/sonic_sampler.h"
 
@@ -298,7 +299,7 @@ __global__ __launch_bounds__(SS_BLOCK) void topk_merge_kernel(void *p_scratch, i
 // kernel 17.2 us instead of 45.5 at 256 rows of 128256 (3.8 TB/s; bound by its instructions and the
 // four workgroups a CU that the spilled keys leave).
 // ---------------------------------------------------------------------------------------------
-template <bool VEC, int E>
+template <bool ANY, int E>
 __global__ __launch_bounds__(SS_BLOCK) void topk_tiles_kernel(const uint16_t *p_logits, int64_t p_stride,
                                                               int p_block_n, int p_vocab, int p_k, int tiles,
                                                               uint32_t *p_scratch, int64_t p_stride_scratch) {
@@ -308,26 +309,14 @@ __global__ __launch_bounds__(SS_BLOCK) void topk_tiles_kernel(const uint16_t *p_
     const int col0 = tile * p_block_n;
     const uint16_t *lrow = p_logits + (int64_t)row * p_stride;
     const int lane4 = 4 * (int)threadIdx.x;
-    u32x2 lw[E / 4];
-    if constexpr (VEC) {
-        load_logits_vec<E>(lrow, col0, p_vocab, lw);
-    } else {
-        const __amdgpu_buffer_rsrc_t rb = row_buffer(lrow, (int64_t)p_vocab * 2);
-#pragma unroll
-        for (int c = 0; c < E / 4; ++c) {
-            uint32_t h[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                h[i] = __builtin_amdgcn_raw_buffer_load_b16(rb, (lane4 + i) * 2, (col0 + c * (SS_BLOCK * 4)) * 2, NT);
-            lw[c].x = h[0] | (h[1] << 16);
-            lw[c].y = h[2] | (h[3] << 16);
-        }
-    }
+    typename HalfRow<ANY>::Raw lw[E / 4];
+    load_logits<E, ANY>(lrow, col0, p_vocab, lw);
     Keys<E> keys;
 #pragma unroll
     for (int c = 0; c < E / 4; ++c) {
-        keys.p[2 * c] = packed_keys(lw[c].x);
-        keys.p[2 * c + 1] = packed_keys(lw[c].y);
+        const u32x2 w = HalfRow<ANY>::words(lw[c], lrow);
+        keys.p[2 * c] = packed_keys(w.x);
+        keys.p[2 * c + 1] = packed_keys(w.y);
     }
     if (col0 + SS_BLOCK * E > p_vocab) {
         // columns past the vocabulary are absent (key 0)
@@ -371,7 +360,7 @@ __device__ __forceinline__ uint32_t float_key(float v) {
     return u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
 }
 
-template <bool VEC, int E>
+template <int E>
 __global__ __launch_bounds__(SS_BLOCK) void topk_block_kernel(const void *p_logits, int64_t p_stride,
                                                               int p_block_n, int p_vocab, int p_k, int tiles,
                                                               ss_topk_args a) {
@@ -395,14 +384,9 @@ __global__ __launch_bounds__(SS_BLOCK) void topk_block_kernel(const void *p_logi
 #pragma unroll
     for (int c = 0; c < E / 4; ++c) {
         const int col = c * (SS_BLOCK * 4) + lane4;
-        uint32_t w[4];
-        if (VEC) {
-            const i32x4 q = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, col * 4, 0, NT));
-            w[0] = q.x; w[1] = q.y; w[2] = q.z; w[3] = q.w;
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) w[i] = __builtin_amdgcn_raw_buffer_load_b32(rb, (col + i) * 4, 0, NT);
-        }
+        // (dword-aligned, whatever the row's start and width)
+        const i32x4 q = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, col * 4, 0, NT));
+        const uint32_t w[4] = {(uint32_t)q.x, (uint32_t)q.y, (uint32_t)q.z, (uint32_t)q.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[4 * c + i] = col + i < V ? __uint_as_float(w[i]) : -INFINITY;
     }
@@ -579,7 +563,7 @@ __device__ __forceinline__ uint32_t wide_exclusive_scan(uint32_t n, uint32_t *re
     return before + inc - n;
 }
 
-template <bool F32, bool VEC>
+template <bool F32, bool ANY>
 __global__ __launch_bounds__(TOPK_WIDE_THREADS) void topk_wide_kernel(const void *p_logits, int64_t p_stride, int p_vocab,
                                                                      int p_k, ss_topk_args a) {
     __shared__ TopkWideSmem sm;
@@ -592,6 +576,7 @@ __global__ __launch_bounds__(TOPK_WIDE_THREADS) void topk_wide_kernel(const void
     const int lane4 = 4 * (int)threadIdx.x;
     const char *base = (const char *)p_logits + (int64_t)row * p_stride * (F32 ? 4 : 2);
     const __amdgpu_buffer_rsrc_t rb = row_buffer(base, (int64_t)V * (F32 ? 4 : 2));
+    const HalfRow<ANY> hr((const uint16_t *)base, V);
     auto emit = [&](int e, uint64_t c) {
         const float val = __uint_as_float(unkey32((uint32_t)(c >> 32)));
         const int col = (int)(0xffffffffu - (uint32_t)c);
@@ -606,19 +591,12 @@ __global__ __launch_bounds__(TOPK_WIDE_THREADS) void topk_wide_kernel(const void
     for (int c = 0; c < E / 4; ++c) {
         const int col = c * TOPK_WIDE_CHUNK + lane4;
         uint32_t w[4];
-        if (VEC) {
-            if (F32) {
-                const i32x4 q = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, col * 4, 0, NT));
-                w[0] = q.x; w[1] = q.y; w[2] = q.z; w[3] = q.w;
-            } else {
-                const u32x2 q = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rb, col * 2, 0, NT));
-                w[0] = q.x << 16; w[1] = q.x & 0xffff0000u; w[2] = q.y << 16; w[3] = q.y & 0xffff0000u;
-            }
+        if constexpr (F32) {
+            const i32x4 q = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, col * 4, 0, NT));
+            w[0] = q.x; w[1] = q.y; w[2] = q.z; w[3] = q.w;
         } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                w[i] = F32 ? __builtin_amdgcn_raw_buffer_load_b32(rb, (col + i) * 4, 0, NT)
-                           : (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rb, (col + i) * 2, 0, NT) << 16;
+            const u32x2 q = HalfRow<ANY>::words(hr.load(col * 2, 0), (const uint16_t *)base);
+            w[0] = q.x << 16; w[1] = q.x & 0xffff0000u; w[2] = q.y << 16; w[3] = q.y & 0xffff0000u;
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[4 * c + i] = col + i < V ? __uint_as_float(w[i]) : -INFINITY;
@@ -762,50 +740,39 @@ __global__ __launch_bounds__(TOPK_WIDE_THREADS) void topk_wide_kernel(const void
     }
 }
 
-template <bool F32>
-static bool topk_vec(const ss_topk_args *a) {
-    const int esz = F32 ? 4 : 2;
-    return (a->vocab_size % 4) == 0 && (a->stride_logits % 4) == 0 && ((uintptr_t)a->logits % (4 * esz)) == 0;
+// Whether bf16 rows need the loads of HalfRow<true>.
+static bool topk_any(const ss_topk_args *a) {
+    return a->dtype == SS_DTYPE_BF16 && (a->vocab_size % 4 != 0 || !half_rows_on_dwords(a->logits, a->stride_logits));
 }
 
-template <bool F32>
+template <bool F32, bool ANY>
 static int launch_topk_rows(const ss_topk_args *a) {
     dim3 grid((unsigned)a->rows), block(TOPK_WIDE_THREADS);
     hipStream_t s = (hipStream_t)a->stream;
-    if (topk_vec<F32>(a)) hipLaunchKernelGGL((topk_wide_kernel<F32, true>), grid, block, 0, s, a->logits, a->stride_logits, a->vocab_size, a->k, *a);
-    else hipLaunchKernelGGL((topk_wide_kernel<F32, false>), grid, block, 0, s, a->logits, a->stride_logits, a->vocab_size, a->k, *a);
+    hipLaunchKernelGGL((topk_wide_kernel<F32, ANY>), grid, block, 0, s, a->logits, a->stride_logits, a->vocab_size, a->k, *a);
     return hipGetLastError() == hipSuccess ? SS_OK : SS_ERR_LAUNCH;
 }
 
-template <bool F32, bool VEC, int E>
+template <bool F32, bool ANY, int E>
 static void launch_topk_tile(const ss_topk_args *a, int tiles, dim3 grid, hipStream_t s) {
     if constexpr (F32)
-        hipLaunchKernelGGL((topk_block_kernel<VEC, E>), grid, dim3(SS_BLOCK), 0, s, a->logits, a->stride_logits, a->block_n, a->vocab_size, a->k, tiles, *a);
+        hipLaunchKernelGGL((topk_block_kernel<E>), grid, dim3(SS_BLOCK), 0, s, a->logits, a->stride_logits, a->block_n, a->vocab_size, a->k, tiles, *a);
     else
-        hipLaunchKernelGGL((topk_tiles_kernel<VEC, E>), grid, dim3(SS_BLOCK), 0, s, (const uint16_t *)a->logits, a->stride_logits, a->block_n, a->vocab_size, a->k, tiles, (uint32_t *)a->scratch, a->stride_scratch);
+        hipLaunchKernelGGL((topk_tiles_kernel<ANY, E>), grid, dim3(SS_BLOCK), 0, s, (const uint16_t *)a->logits, a->stride_logits, a->block_n, a->vocab_size, a->k, tiles, (uint32_t *)a->scratch, a->stride_scratch);
 }
 
-template <bool F32, bool VEC>
-static int launch_topk_tiles(const ss_topk_args *a, int tiles, dim3 grid, hipStream_t s) {
-    switch (a->block_n) {
-        case 1024: launch_topk_tile<F32, VEC, 4>(a, tiles, grid, s); break;
-        case 2048: launch_topk_tile<F32, VEC, 8>(a, tiles, grid, s); break;
-        case 4096: launch_topk_tile<F32, VEC, 16>(a, tiles, grid, s); break;
-        case 8192: launch_topk_tile<F32, VEC, 32>(a, tiles, grid, s); break;
-        case 16384: launch_topk_tile<F32, VEC, 64>(a, tiles, grid, s); break;
-        default: return SS_ERR_UNSUPPORTED;
-    }
-    return SS_OK;
-}
-
-template <bool F32>
+template <bool F32, bool ANY>
 static int launch_topk(const ss_topk_args *a, int tiles) {
     dim3 grid((unsigned)(a->rows * tiles)), block(SS_BLOCK);
     hipStream_t s = (hipStream_t)a->stream;
-    // tiles start at multiples of block_n, so the 16 / 8-byte chunks of every tile stay aligned
-    const int st = topk_vec<F32>(a) ? launch_topk_tiles<F32, true>(a, tiles, grid, s)
-                                    : launch_topk_tiles<F32, false>(a, tiles, grid, s);
-    if (st != SS_OK) return st;
+    switch (a->block_n) {
+        case 1024: launch_topk_tile<F32, ANY, 4>(a, tiles, grid, s); break;
+        case 2048: launch_topk_tile<F32, ANY, 8>(a, tiles, grid, s); break;
+        case 4096: launch_topk_tile<F32, ANY, 16>(a, tiles, grid, s); break;
+        case 8192: launch_topk_tile<F32, ANY, 32>(a, tiles, grid, s); break;
+        case 16384: launch_topk_tile<F32, ANY, 64>(a, tiles, grid, s); break;
+        default: return SS_ERR_UNSUPPORTED;
+    }
     if (hipGetLastError() != hipSuccess) return SS_ERR_LAUNCH;
     hipLaunchKernelGGL((topk_merge_kernel<F32>), dim3((unsigned)a->rows), block, 0, s, a->scratch, a->stride_scratch, a->vocab_size, a->k,
                        a->block_n, tiles, *a);
@@ -841,8 +808,9 @@ extern "C" int ss_topk(const ss_topk_args *a) {
     const bool wide = a->strategy == SS_STRATEGY_ROWWISE ||
                       (a->strategy == SS_STRATEGY_AUTO && a->dtype == SS_DTYPE_F32 && a->rows >= 48 && a->k <= 32 &&
                        a->vocab_size > 16384 && a->vocab_size <= ss::TOPK_WIDE_THREADS * ss::TOPK_WIDE_E);
-    if (wide)
-        return a->dtype == SS_DTYPE_F32 ? ss::launch_topk_rows<true>(a) : ss::launch_topk_rows<false>(a);
-    return a->dtype == SS_DTYPE_F32 ? ss::launch_topk<true>(a, tiles)
-                                    : ss::launch_topk<false>(a, tiles);
+    if (a->dtype == SS_DTYPE_F32)
+        return wide ? ss::launch_topk_rows<true, false>(a) : ss::launch_topk<true, false>(a, tiles);
+    if (ss::topk_any(a))
+        return wide ? ss::launch_topk_rows<false, true>(a) : ss::launch_topk<false, true>(a, tiles);
+    return wide ? ss::launch_topk_rows<false, false>(a) : ss::launch_topk<false, false>(a, tiles);
 }

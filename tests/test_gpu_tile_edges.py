@@ -53,3 +53,75 @@ def test_partial_last_tile(block, values):
             want_values, want = oracle_topk(x, k)
             assert torch.equal(got.cpu(), want)
             assert torch.equal(got_values.cpu(), want_values)
+
+
+def shifted(plane, offset, pad):
+    """A copy of the bf16 [rows, n] plane whose rows start `offset` halves into their storage and
+    lie n + pad apart."""
+
+    rows, n = plane.shape
+    flat = torch.full((offset + rows * (n + pad) + 8,), -7.0, dtype=plane.dtype, device=plane.device)
+    view = flat[offset:].as_strided((rows, n), (n + pad, 1), offset)
+    view.copy_(plane)
+
+    return view
+
+
+@pytest.mark.parametrize("offset,pad", [(1, 0), (0, 1), (3, 3), (2, 0), (0, 2)])
+@pytest.mark.parametrize("block,vocab", [(1024, 2052), (2048, 9000), (4096, 8196), (8192, 33000), (16384, 50280)])
+def test_rows_at_any_half_word(block, vocab, offset, pad):
+    """Logit and bias rows at every 2-byte address and stride take the three-dword loads; the same
+    values in aligned rows take the aligned ones. Every output of the decode step, of drafting
+    through d2t, of the verification and of the top-k is the same bits."""
+
+    from sonic_sampler.core.buffer import SamplingBuffers
+    from sonic_sampler.core.flags import Flags, Indicator
+    from sonic_sampler.interface import UnshardedBoundedTopK
+    from sonic_sampler.interface.functional import fused_multistep, fused_singular
+
+    rows = 6
+    g = torch.Generator().manual_seed(vocab + offset)
+    logits = (torch.randn(rows, vocab, generator=g) * 3).to(torch.bfloat16).to(DEV)
+    buffers = SamplingBuffers.random(size=rows, timesteps=1, vocab_size=vocab, device=DEV, seed=vocab,
+                                     indicators=Indicator(0x7BF), max_top_logprobs=5)
+    # rows of every kind: all processors, none (the logits alone), penalties only, bias only, greedy
+    kinds = [0x7BF, 0x400, 0x40E, 0x410, 0x05E, 0x4B1]
+    buffers.flags = Flags.from_values(rows, 1, [Indicator(k) for k in kinds], device=torch.device(DEV))
+    rep = buffers.repetition
+    d2t = torch.randperm(vocab, generator=g)[: vocab - 1].to(torch.int32).to(DEV)
+    common = dict(
+        indicators=buffers.flags.target, block_n=block, context_counts=rep.counts.context,
+        repetition_penalties=rep.multiplicative, frequency_penalties=rep.frequency,
+        presence_penalties=rep.presence, temperature=buffers.temperature, top_k=buffers.top_k,
+        top_p=buffers.top_p, min_p=buffers.min_p, philox_seed=5)
+
+    def outputs(x, bias):
+
+        print(f"block {block} vocab {vocab} offset {offset} pad {pad}", flush=True)
+        grammar = buffers.grammar[:, 0].as_subclass(torch.Tensor)
+        one = fused_singular(x, logit_bias=bias, grammar=grammar, decode_counts=rep.counts.decode, **common)
+        probabilities = torch.zeros(rows, vocab, dtype=torch.bfloat16, device=DEV)
+        draft = fused_singular(x[:, : vocab - 1], logit_bias=bias, grammar=grammar, decode_counts=rep.counts.decode,
+                               d2t_mapping=d2t, target_vocab=vocab, return_probabilities=True,
+                               draft_probabilities=probabilities, **common)
+        values = torch.zeros(rows, 128, device=DEV)
+        indices = torch.zeros(rows, 128, dtype=torch.int32, device=DEV)
+        drafted = x.float().argmax(-1).to(torch.int32)
+        keep = {k: v for k, v in common.items() if k != "indicators"}
+        check = fused_multistep(x.unflatten(0, (rows // 2, 2)), drafted_tokens=drafted.view(rows // 2, 2),
+                                indicators=buffers.flags.target[: rows // 2].clone(), lookahead=1, logit_bias=bias,
+                                decode_counts=rep.counts.decode, values=values, indices=indices,
+                                uniform_noise=buffers.weights.uniform.as_subclass(torch.Tensor), **keep)
+        topk = UnshardedBoundedTopK.initialize(vocab_size=vocab, batch_size=rows, k=128, block_size=block, device=DEV)
+        best, columns = topk(x)
+
+        return [t.clone() for t in (one.tokens, draft.tokens, probabilities, check.tokens, check.offsets, indices, values,
+                                    best, columns)]
+
+    want = outputs(logits, buffers.bias)
+    got = outputs(shifted(logits, offset, pad), shifted(buffers.bias, offset, pad))
+
+    for name, a, b in zip(("decode", "drafts", "probabilities", "tokens", "offsets", "indices", "values", "top-k", "columns"),
+                          want, got):
+
+        assert torch.equal(a, b), f"{name} differ between aligned rows and rows at offset {offset}, pad {pad}"
