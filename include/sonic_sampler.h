@@ -80,8 +80,8 @@ typedef struct ss_philox {
  * top-128 to the scratchpad, then one workgroup per row merges and selects (two launches).
  * ROWWISE: one workgroup per row streams the row tile by tile and selects in the same launch
  * (rows of at most 16 tiles; the scratchpad is not touched). AUTO: ss_fused_singular always takes
- * TILES; ss_topk takes ROWWISE for at least 48 float32 rows of 16385-32768 columns at k <= 32 and
- * TILES otherwise. */
+ * TILES; ss_topk takes ROWWISE for at least 48 rows (of bf16 at most 256) of 16385-32768 columns at
+ * k <= 32 and TILES otherwise. */
 typedef enum ss_strategy {
     SS_STRATEGY_AUTO = 0,
     SS_STRATEGY_TILES = 1,
@@ -103,7 +103,7 @@ typedef struct ss_topk_args {
     int32_t k;           /* power of two, 1 <= k <= 128 */
     int32_t block_n;     /* tile width: 1024, 2048, 4096, 8192 or 16384 */
     int32_t strategy;    /* ss_strategy: 0 automatic (tile grid; one workgroup per row for >= 48
-                            float32 rows of 16385-32768 columns at k <= 32), 2 one workgroup per row (V <= 32768) */
+                            rows, of bf16 <= 256, of 16385-32768 columns at k <= 32), 2 one workgroup per row (V <= 32768) */
     void *scratch;       /* rows * stride_scratch elements (uint32 or uint64) */
     int64_t stride_scratch;
     void *values;        /* [rows, k] bf16 or fp32 */

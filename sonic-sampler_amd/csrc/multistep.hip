@@ -87,7 +87,7 @@ __device__ __forceinline__ RowState multistep_row_state(const ss_multistep_args 
     rs.temp = (ind & IND_TEMP) ? temp : 1.0f;
     if (!a.temperature) rs.ind &= ~IND_TEMP;
     rs.vt = a.vocab_size;
-    rs.nhist = 0;
+    rs.hist = 0;
     rs.glds = nullptr;
     rs.shard = 0;
     return rs;
@@ -123,13 +123,13 @@ __global__ __launch_bounds__(SS_BLOCK) void multistep_tiles_kernel(const uint16_
     if (step > 0 && (ind & (IND_MULT | IND_FREQ | IND_PRES))) {
         // Step s of a request sees the drafts of steps < s as extra decode history
         // (core/naive.py:179-198, the `tril` history with timestep None).
-        rs.nhist = step;
-        if ((int)threadIdx.x < step) sm.hist[threadIdx.x] = a.drafted_tokens[rq.margin + threadIdx.x];
-        __syncthreads();
+        if (lane_id() < step) rs.hist = a.drafted_tokens[rq.margin + lane_id()];
     }
+    uint32_t *scr = computed_here(a.scratch + (int64_t)row * a.stride_scratch);
     Keys<E> keys;
-    prologue_keys<E, MODE>(rs, tile * a.block_n, a.vocab_size, sm.hist, lw, keys);
-    tile_stage<E>(sm, (ind & IND_GREEDY) != 0, keys, a.scratch + (int64_t)row * a.stride_scratch, tile,
+    // the rows of a request read the same side planes: cached, not streamed
+    prologue_keys<E, MODE, false, 0>(rs, tile * a.block_n, a.vocab_size, &sm.keys[0][0], ExcList<E>::CAP, lw, keys);
+    tile_stage<E>(sm, (ind & IND_GREEDY) != 0, keys, scr, tile,
                   min(a.block_n, a.vocab_size - tile * a.block_n));
 }
 

@@ -41,7 +41,7 @@ __device__ __forceinline__ RowState singular_row_state(const ss_singular_args &a
     rs.temp = (ind & IND_TEMP) ? temp : 1.0f;
     if (!a.temperature) rs.ind &= ~IND_TEMP;
     rs.vt = a.target_vocab > 0 ? a.target_vocab : a.vocab_size;
-    rs.nhist = 0;
+    rs.hist = 0;
     rs.glds = nullptr;
     rs.shard = a.world_size > 1 ? a.local_rank * a.shard_size : 0;
     return rs;
@@ -76,12 +76,10 @@ __global__ __launch_bounds__(SS_BLOCK) void singular_tiles_kernel(const uint16_t
     const int slot = p_slots ? uniform_i32(p_slots, row) : row;
     const uint32_t ind = uniform_u16(p_ind, slot);
     RowState rs = singular_row_state(a, row, slot, ind);
-    bool sync = false;
     const Uses u = row_uses(rs);
     if ((MODE & MODE_GATHER) && stage_words > 0 && u.g && u.remap) {
         stage_grammar(rs.grammar, rs.vt, grammar_words);
         rs.glds = grammar_words;
-        sync = true;
     }
     // the d2t targets of the tile's columns, requested while the grammar row is staged: the
     // workgroup barrier below then waits for both rounds of loads at once
@@ -90,18 +88,25 @@ __global__ __launch_bounds__(SS_BLOCK) void singular_tiles_kernel(const uint16_t
     if constexpr (PRE) {
         if (u.remap) load_d2t<E>(rs, tile * a.block_n, a.vocab_size, pre);
     }
-    if (a.drafted_tokens && a.timestep > 0 && (ind & (IND_MULT | IND_FREQ | IND_PRES))) {
-        rs.nhist = a.timestep;
-        if ((int)threadIdx.x < rs.nhist)
-            sm.hist[threadIdx.x] = a.drafted_tokens[(int64_t)row * a.stride_drafted + threadIdx.x];
-        sync = true;
+    if (a.drafted_tokens && (ind & (IND_MULT | IND_FREQ | IND_PRES)) && lane_id() < a.timestep)
+        rs.hist = a.drafted_tokens[(int64_t)row * a.stride_drafted + lane_id()];
+    if (rs.glds) {
+        stage_grammar_finish(rs.vt, grammar_words);
+        __syncthreads();
     }
-    if (rs.glds) stage_grammar_finish(rs.vt, grammar_words);
-    if (sync) __syncthreads();
-    Keys<E> keys;
-    prologue_keys<E, MODE, PRE>(rs, tile * a.block_n, a.vocab_size, sm.hist, lw, keys, pre);
+    // the waves' exception lists: in the memory of their spilled keys, or behind a staged grammar
+    // row, which overlays it
+    uint32_t *exc = &sm.keys[0][0];
+    uint32_t cap = ExcList<E>::CAP;
+    if ((MODE & MODE_GATHER) && stage_words > 0) {
+        exc = grammar_words + 4 * stage_region_quads(rs.vt);
+        cap = EXC_STAGED_CAP;
+    }
     // this shard's slice of the row's [world_size, tiles, 128] lists
-    uint32_t *scr = a.scratch + (int64_t)row * a.stride_scratch + (a.world_size > 1 ? a.local_rank * tiles * SS_K : 0);
+    uint32_t *scr = computed_here(a.scratch + (int64_t)row * a.stride_scratch +
+                                  (a.world_size > 1 ? a.local_rank * tiles * SS_K : 0));
+    Keys<E> keys;
+    prologue_keys<E, MODE, PRE>(rs, tile * a.block_n, a.vocab_size, exc, cap, lw, keys, pre);
     tile_stage<E>(sm, (ind & IND_GREEDY) != 0, keys, scr, tile, min(a.block_n, a.vocab_size - tile * a.block_n));
 }
 
@@ -275,11 +280,8 @@ __global__ __launch_bounds__(SS_BLOCK) void singular_rowwise_kernel(ss_singular_
         stage_grammar(rs.grammar, rs.vt, grammar_words);
         rs.glds = grammar_words;
     }
-    if (a.drafted_tokens && a.timestep > 0 && (ind & (IND_MULT | IND_FREQ | IND_PRES))) {
-        rs.nhist = a.timestep;
-        if ((int)threadIdx.x < rs.nhist)
-            sm.tile.hist[threadIdx.x] = a.drafted_tokens[(int64_t)row * a.stride_drafted + threadIdx.x];
-    }
+    if (a.drafted_tokens && (ind & (IND_MULT | IND_FREQ | IND_PRES)) && lane_id() < a.timestep)
+        rs.hist = a.drafted_tokens[(int64_t)row * a.stride_drafted + lane_id()];
     if (rs.glds) stage_grammar_finish(rs.vt, grammar_words);
     __syncthreads();
     const bool greedy = (ind & IND_GREEDY) != 0;
@@ -289,7 +291,7 @@ __global__ __launch_bounds__(SS_BLOCK) void singular_rowwise_kernel(ss_singular_
         if (t + 1 < tiles)
             load_logits<E, (MODE & MODE_ANY) != 0>(lrow, (t + 1) * a.block_n, a.vocab_size, nx);
         Keys<E> keys;
-        prologue_keys<E, MODE>(rs, t * a.block_n, a.vocab_size, sm.tile.hist, lw, keys);
+        prologue_keys<E, MODE>(rs, t * a.block_n, a.vocab_size, &sm.tile.keys[0][0], ExcList<E>::CAP, lw, keys);
         tile_stage<E>(sm.tile, greedy, keys, sm.lists, t, min(a.block_n, a.vocab_size - t * a.block_n));
         // the next tile reuses the tile stage's memory, and the lists feed the row stage
         __syncthreads();
@@ -326,12 +328,13 @@ static size_t staged_grammar_bytes(const ss_singular_args *a) {
 }
 
 // Dynamic shared memory of singular_tiles_kernel<E>: its TileSmem, or a staged grammar row from
-// TILE_OVERLAY on where that is larger.
+// TILE_OVERLAY on and the exception lists behind it where that is larger.
 template <int E>
 static size_t tile_smem_bytes(const ss_singular_args *a) {
-    const size_t g = staged_grammar_bytes(a);
+    const size_t row = staged_grammar_bytes(a);
+    const size_t g = row ? TILE_OVERLAY + row + SS_WAVES * EXC_STAGED_CAP * ExcList<E>::WORDS * 4 : 0;
     const size_t t = sizeof(TileSmem<E>);
-    return g && TILE_OVERLAY + g > t ? TILE_OVERLAY + g : t;
+    return g > t ? g : t;
 }
 
 template <int MODE>

@@ -216,6 +216,19 @@ __device__ __forceinline__ void touch_kernargs() {
     asm volatile("" ::"s"(acc));
 }
 
+// Set bits of m below the lane's own.
+__device__ __forceinline__ uint32_t mbcnt64(uint64_t m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// A uniform pointer, computed here and not where it is first used: what it takes from the kernel's
+// arguments is then read while other loads are in flight.
+template <typename T>
+__device__ __forceinline__ T *computed_here(T *p) {
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
 // Value of lane `src` (uniform) in every lane, through the scalar unit.
 __device__ __forceinline__ uint32_t lane_u32(uint32_t v, int src) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, __builtin_amdgcn_readfirstlane(src));

@@ -30,7 +30,6 @@ struct SampleSmem {
     int32_t flag;
     uint64_t cand[SS_K];
     int32_t idx[SS_K];
-    int32_t hist[64];
     uint32_t red[SS_WAVES];
     int32_t tok[SS_K];         // selection: the candidates' tokens (columns, then remapped)
     float noise[SS_K];         // selection: their Gumbel noise
@@ -45,16 +44,15 @@ struct TileSmem {
     uint32_t scan[SS_WAVES * 16];  // workgroup scans of up to 16 values per thread
     uint32_t red[SS_WAVES];
     uint32_t cnt[SS_WAVES];       // survivors of each wave
-    int32_t hist[64];             // drafted tokens that extend the decode history
     uint32_t run[SS_WAVES][SS_K + 64];  // each wave's survivors, then its sorted run
     uint32_t run2[2][SS_K];       // merge tree: the top-128 of runs (0, 1) and (2, 3)
     // each wave's packed keys, pair i of lane l at [i * 64 + l], read back by the survivors of
-    // wave_survivors_masked
+    // wave_survivors_masked; before that the wave's exception list (ExcList)
     uint32_t keys[SS_WAVES][E / 2 * 64];
 };
 
 // Byte offset in TileSmem where a staged grammar row may begin.
-constexpr int TILE_OVERLAY = (SS_WAVES * 16 + 2 * SS_WAVES + 64) * 4;
+constexpr int TILE_OVERLAY = (SS_WAVES * 16 + 2 * SS_WAVES) * 4;
 static_assert(TILE_OVERLAY % 16 == 0, "16-byte grammar stores");
 static_assert(TILE_OVERLAY == __builtin_offsetof(TileSmem<16>, run), "overlay starts at the runs");
 
@@ -70,7 +68,7 @@ struct RowState {
     const uint16_t *bias;
     float rep, freq, pres, temp;
     int vt;     // width of the counts / bias / grammar rows (target vocabulary)
-    int nhist;  // drafted tokens of the history staged in SampleSmem::hist
+    int hist;   // the lane's token of the drafted history (lane l: position l; 0: none there)
     // The row's grammar words staged in workgroup memory (gather layout only), or NULL: the
     // gathers through d2t then read LDS instead of scattered global words.
     const uint32_t *glds;
@@ -156,20 +154,6 @@ struct Keys {
 
 typedef float f2v __attribute__((ext_vector_type(2)));
 typedef __bf16 b2v __attribute__((ext_vector_type(2)));
-
-// Rounds two fp32 values to bf16 (round-to-nearest-even, v_cvt_pk_bf16_f32) in place.
-__device__ __forceinline__ void round_pair(float &a, float &b) {
-    const f2v v = {a, b};
-    const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, b2v));
-    a = __uint_as_float(u << 16);
-    b = __uint_as_float(u & 0xffff0000u);
-}
-
-template <int E>
-__device__ __forceinline__ void round_all(float (&x)[E]) {
-#pragma unroll
-    for (int j = 0; j < E; j += 2) round_pair(x[j], x[j + 1]);
-}
 
 // Divisor state of a per-row constant d: rcp = 1/d from v_rcp_f32 (within 1 ulp); `fast` is
 // false when d is 0, infinite or NaN or the reciprocal is not a normal number (|d| near the ends
@@ -302,31 +286,56 @@ __device__ __forceinline__ float chain_ieee(const Chain &k, float x, int32_t dec
     return k.temp ? rnd(x / k.tdiv.d) : x;
 }
 
-// Keys of E elements from their (grammar-masked) logits x, decode counts, context counts and
-// bias bits. Most elements of a row have zero counts and zero bias; for them every penalty and the
-// bias are the identity and the chain reduces to the temperature division, which runs for all
-// elements with one multiply each. Elements with a nonzero count or bias (or every element, when a
-// non-finite frequency penalty turns 0 * f into NaN) then run the full chain one element position
-// at a time, so a wave pays for it only at the positions where one of its lanes holds one. Rows
-// whose divisors have no exact reciprocal take the IEEE chain on every element instead. `ok` marks
-// elements inside the vocabulary; it can be false only when `partial` is set. x(j) and bb(j) return
-// the (grammar-masked) logit and the bias bits of element j; bw(j) is nonzero whenever element j's
-// bias is nonzero (it may also be nonzero for a zero bias: the chain is exact for every element).
-// maybe_exc is false when no element can have a nonzero count or bias (no penalty or bias plane is
-// read) and the chain is not forced on every element: the keys are then the temperature keys.
-// pair(j) (j even) is the 32-bit word holding the masked bf16 logits of elements j and j + 1.
-template <int E, class XOf, class PairOf, class BiasOf, class BiasWordOf>
-__device__ __forceinline__ void finish_keys(const Chain &k, bool all_exc, bool partial, XOf x,
-                                            PairOf pair, bool maybe_exc,
-                                            const bool (&ok)[E], const int32_t (&dec)[E],
-                                            const int32_t (&ctx)[E], BiasOf bb, BiasWordOf bw,
-                                            Keys<E> &keys) {
+// The elements of a wave that the processor chain has to run on, collected over a tile's passes.
+// Most elements have zero counts and zero bias, for which every penalty and the bias are the
+// identity; with a prompt of 1500 tokens and 400 generated ones 1.5% of 128256 do not, and a wave
+// that ran the chain wherever one of its 64 lanes held such an element ran it at two positions in
+// three for one lane's sake. Instead the 4-column chunks that hold one go to a list in workgroup
+// memory (logits, bias, decode and context counts: 48 bytes), one lane then takes one chunk of it,
+// and every lane fetches its own chunks' keys back. 1280 verification rows of 128256 columns with such
+// requests: 2180 vector instructions a wave -> 1213, the tile kernel 240 -> 153 us (with the planes
+// cached between a request's rows and the logits no longer loaded twice: 0.58 GB fetched, not 1.25).
+template <int E>
+struct ExcList {
+    static constexpr uint32_t CAP = E / 2 * 64 * 4 / 48;  // records that fit TileSmem::keys
+    static constexpr int WORDS = 12;                      // of a record
+    uint32_t *mem;       // the wave's records
+    uint32_t cap;
+    uint32_t cnt;        // records (uniform)
+    uint64_t m[E / 4];   // per chunk: the lanes whose chunk is in the list (set where planes are read)
+};
+
+// Records of the list in the gather layout with a staged grammar row, which lies behind the row:
+// 40368 bytes of workgroup memory in all at 8192 grammar words, four workgroups a CU.
+constexpr uint32_t EXC_STAGED_CAP = 38;
+
+// Keys of the E / 4 chunks of one pass from their (grammar-masked) logits, decode counts, context
+// counts and bias bits. The temperature division, the chain's whole effect on an element with zero
+// counts and bias, runs for all elements with one multiply each; the chunks with a nonzero count or
+// bias go to `ex` (chunk c of the pass as chunk c0 + c of the tile), or, where the list has no room
+// for the pass's (or a non-finite frequency penalty turns 0 * f into NaN), the chain runs on every
+// element. Rows whose divisors have no exact reciprocal take the IEEE chain on every element.
+// lw / bw: the (grammar-masked) logits and the biases as loaded pairs. maybe_exc is false when no
+// element can have a nonzero count or bias (no penalty or bias plane is read) and the chain is not
+// forced on every element. Elements past the vocabulary get a key too (mask_absent clears them).
+template <int E, int ET>
+__device__ __forceinline__ void finish_keys(const Chain &k, bool all_exc, bool maybe_exc, const u32x2 (&lw)[E / 4],
+                                            const u32x2 (&bw)[E / 4], const i32x4 (&dec)[E / 4],
+                                            const i32x4 (&ctx)[E / 4], ExcList<ET> &ex, int c0, Keys<E> &keys) {
+    auto x = [&](int j) {
+        const uint32_t w = (j & 2) ? lw[j >> 2].y : lw[j >> 2].x;
+        return __uint_as_float((j & 1) ? (w & 0xffff0000u) : (w << 16));
+    };
+    auto bb = [&](int j) {
+        const uint32_t w = (j & 2) ? bw[j >> 2].y : bw[j >> 2].x;
+        return __uint_as_float((j & 1) ? (w & 0xffff0000u) : (w << 16));
+    };
     if ((!k.mult || k.rdiv.fast) && (!k.temp || k.tdiv.fast)) {
         const FastChain f = fast_chain(k);
         if (!k.temp) {
             // no temperature: the keys of the (grammar-masked) bf16 pairs as they are
 #pragma unroll
-            for (int j = 0; j < E; j += 2) keys.p[j >> 1] = packed_keys(pair(j));
+            for (int j = 0; j < E; j += 2) keys.p[j >> 1] = packed_keys((j & 2) ? lw[j >> 2].y : lw[j >> 2].x);
         } else {
 #pragma unroll
             for (int j = 0; j < E; j += 2) {
@@ -334,32 +343,105 @@ __device__ __forceinline__ void finish_keys(const Chain &k, bool all_exc, bool p
                 keys.p[j >> 1] = packed_keys(__builtin_bit_cast(uint32_t, __builtin_convertvector(v, b2v)));
             }
         }
-        // The branch at each element position is on the wave's ballot, so it is uniform: the
-        // chain then runs with every lane active and the ballot selects its result.
-        if (all_exc) {
+        if (!maybe_exc) return;
+        uint32_t total = 0;
 #pragma unroll
-            for (int j = 0; j < E; ++j)
-                keys.p[j >> 1] = keys.with(j, key_of(chain_fast(f, x(j), dec[j], ctx[j], __uint_as_float(bb(j)))));
-        } else if (maybe_exc) {
+        for (int c = 0; c < E / 4; ++c) {
+            const i32x4 n = dec[c] | ctx[c];
+            ex.m[c0 + c] = __ballot(((uint32_t)(n.x | n.y | n.z | n.w) | bw[c].x | bw[c].y) != 0u);
+            total += (uint32_t)__popcll(ex.m[c0 + c]);
+        }
+        if (all_exc || ex.cnt + total > ex.cap) {
 #pragma unroll
-            for (int j = 0; j < E; ++j) {
-                const uint64_t m = __ballot(((uint32_t)(dec[j] | ctx[j]) | bw(j)) != 0u);
-                if (m) {
-                    const uint32_t kc = key_of(chain_fast(f, x(j), dec[j], ctx[j], __uint_as_float(bb(j))));
-                    keys.p[j >> 1] = lane_select(m, keys.p[j >> 1], keys.with(j, kc));
+            for (int c = 0; c < E / 4; ++c) {
+                ex.m[c0 + c] = 0;
+#pragma unroll
+                for (int i = 0; i < 4; i += 2) {
+                    const int j = 4 * c + i;
+                    keys.p[j >> 1] = key_of(chain_fast(f, x(j), dec[c][i], ctx[c][i], bb(j))) |
+                                     (key_of(chain_fast(f, x(j + 1), dec[c][i + 1], ctx[c][i + 1], bb(j + 1))) << 16);
                 }
+            }
+        } else if (total) {
+#pragma unroll
+            for (int c = 0; c < E / 4; ++c) {
+                const uint64_t m = ex.m[c0 + c];
+                if (!m) continue;
+                if (__builtin_amdgcn_inverse_ballot_w64(m)) {
+                    uint32_t *r = ex.mem + (ex.cnt + mbcnt64(m)) * ExcList<ET>::WORDS;
+                    *(i32x4 *)r = i32x4{(int)lw[c].x, (int)lw[c].y, (int)bw[c].x, (int)bw[c].y};
+                    *(i32x4 *)(r + 4) = dec[c];
+                    *(i32x4 *)(r + 8) = ctx[c];
+                }
+                ex.cnt += (uint32_t)__popcll(m);
             }
         }
     } else {
 #pragma unroll
-        for (int j = 0; j < E; j += 2)
-            keys.p[j >> 1] = key_of(chain_ieee(k, x(j), dec[j], ctx[j], __uint_as_float(bb(j)))) |
-                             (key_of(chain_ieee(k, x(j + 1), dec[j + 1], ctx[j + 1], __uint_as_float(bb(j + 1)))) << 16);
-    }
-    if (partial) {
+        for (int c = 0; c < E / 4; ++c) {
+            if (maybe_exc) ex.m[c0 + c] = 0;
 #pragma unroll
-        for (int j = 0; j < E; j += 2)
-            keys.p[j >> 1] = (ok[j] ? keys.p[j >> 1] & 0xffffu : 0u) | (ok[j + 1] ? keys.p[j >> 1] & 0xffff0000u : 0u);
+            for (int i = 0; i < 4; i += 2) {
+                const int j = 4 * c + i;
+                keys.p[j >> 1] = key_of(chain_ieee(k, x(j), dec[c][i], ctx[c][i], bb(j))) |
+                                 (key_of(chain_ieee(k, x(j + 1), dec[c][i + 1], ctx[c][i + 1], bb(j + 1))) << 16);
+            }
+        }
+    }
+}
+
+// Runs the chain on the listed chunks, one lane each, and hands their keys back to the lanes that
+// hold them.
+template <int E>
+__device__ __forceinline__ void finish_exceptions(const FastChain &f, const ExcList<E> &ex, Keys<E> &keys) {
+    if (!ex.cnt) return;
+#pragma unroll 1
+    for (uint32_t i = (uint32_t)lane_id(); i < ex.cnt; i += 64) {
+        uint32_t *r = ex.mem + i * ExcList<E>::WORDS;
+        const i32x4 w = *(const i32x4 *)r, dec = *(const i32x4 *)(r + 4), ctx = *(const i32x4 *)(r + 8);
+        uint32_t out[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t lw = (uint32_t)w[h], bw = (uint32_t)w[2 + h];
+            const float a = chain_fast(f, __uint_as_float(lw << 16), dec[2 * h], ctx[2 * h], __uint_as_float(bw << 16));
+            const float b = chain_fast(f, __uint_as_float(lw & 0xffff0000u), dec[2 * h + 1], ctx[2 * h + 1],
+                                       __uint_as_float(bw & 0xffff0000u));
+            const f2v v = {a, b};  // both bf16-exact
+            out[h] = packed_keys(__builtin_bit_cast(uint32_t, __builtin_convertvector(v, b2v)));
+        }
+        *(u32x2 *)r = u32x2{out[0], out[1]};
+    }
+    uint32_t base = 0;
+#pragma unroll
+    for (int c = 0; c < E / 4; ++c) {
+        const uint64_t m = ex.m[c];
+        if (!m) continue;
+        if (__builtin_amdgcn_inverse_ballot_w64(m)) {
+            const u32x2 v = *(const u32x2 *)(ex.mem + (base + mbcnt64(m)) * ExcList<E>::WORDS);
+            keys.p[2 * c] = v.x;
+            keys.p[2 * c + 1] = v.y;
+        }
+        base += (uint32_t)__popcll(m);
+    }
+}
+
+// Clears the keys of a tile's columns past the vocabulary, chunk by chunk behind uniform branches:
+// masked in every chunk, the last tiles, which one XCD runs where a row has 8 tiles, set the whole
+// kernel's time (303 verification rows of 128256: 20 -> 21.6 us).
+template <int E>
+__device__ __forceinline__ void mask_absent(int col0, int V, Keys<E> &keys) {
+    if (col0 + SS_BLOCK * E <= V) return;
+#pragma unroll
+    for (int c = 0; c < E / 4; ++c) {
+        const int n = V - (col0 + c * (SS_BLOCK * 4));  // columns from the chunk's first on (uniform)
+        if (n >= SS_BLOCK * 4) continue;
+        if (n <= 0) {
+            keys.p[2 * c] = keys.p[2 * c + 1] = 0;
+            continue;
+        }
+        const int left = n - 4 * (int)threadIdx.x;
+        keys.p[2 * c] &= (left > 0 ? 0xffffu : 0u) | (left > 1 ? 0xffff0000u : 0u);
+        keys.p[2 * c + 1] &= (left > 2 ? 0xffffu : 0u) | (left > 3 ? 0xffff0000u : 0u);
     }
 }
 
@@ -408,8 +490,9 @@ struct HalfRow<false> {
     using Raw = u32x2;
     __amdgpu_buffer_rsrc_t rb;
     __device__ __forceinline__ HalfRow(const uint16_t *row, int n) : rb(row_buffer(row, (int64_t)n * 2)) {}
+    template <int AUX = NT>
     __device__ __forceinline__ Raw load(int voff, int soff) const {
-        return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rb, voff, soff, NT));
+        return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rb, voff, soff, AUX));
     }
     static __device__ __forceinline__ u32x2 words(const Raw &r, const uint16_t *) { return r; }
 };
@@ -423,8 +506,9 @@ struct HalfRow<true> {
     __device__ __forceinline__ HalfRow(const uint16_t *row, int n)
         : rb(row_buffer((const void *)((uintptr_t)row & ~(uintptr_t)3),
                         row ? ((int64_t)n * 2 + (int64_t)((uintptr_t)row & 2) + 3) & ~(int64_t)3 : 0)) {}
+    template <int AUX = NT>
     __device__ __forceinline__ Raw load(int voff, int soff) const {
-        return __builtin_bit_cast(u32x3, __builtin_amdgcn_raw_buffer_load_b96(rb, voff, soff, NT));
+        return __builtin_bit_cast(u32x3, __builtin_amdgcn_raw_buffer_load_b96(rb, voff, soff, AUX));
     }
     static __device__ __forceinline__ u32x2 words(const Raw &r, const uint16_t *row) {
         const uint32_t sh = ((uint32_t)(uintptr_t)row & 2u) << 3;  // 16 for a row at an odd half
@@ -511,7 +595,7 @@ struct Planes {
 
 // Issues every side-plane load of the tile before any loaded word is consumed. A plane that is
 // off reads through an empty buffer, which returns zeros without touching memory.
-template <int E, bool ANY>
+template <int E, bool ANY, int AUX>
 __device__ __forceinline__ void issue_planes(const RowState &rs, const Uses &u, bool on, int col0,
                                              Planes<E, ANY> &pl) {
     const int lane4 = (int)threadIdx.x * 4;
@@ -524,35 +608,45 @@ __device__ __forceinline__ void issue_planes(const RowState &rs, const Uses &u, 
 #pragma unroll
     for (int c = 0; c < E / 4; ++c) {
         const int base = col0 + c * (SS_BLOCK * 4);  // uniform, a multiple of 32
-        pl.dw[c] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(db, lane4 * 4, base * 4, NT));
-        pl.cw[c] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(cb, lane4 * 4, base * 4, NT));
-        pl.bw[c] = bb.load(lane4 * 2, base * 2);
+        pl.dw[c] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(db, lane4 * 4, base * 4, AUX));
+        pl.cw[c] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(cb, lane4 * 4, base * 4, AUX));
+        pl.bw[c] = bb.template load<AUX>(lane4 * 2, base * 2);
         pl.gw[c] = __builtin_amdgcn_raw_buffer_load_b32(gb, (lane4 >> 5) * 4, (base >> 5) * 4, 0);
     }
 }
 
-template <int E, bool ANY>
-__device__ __forceinline__ void direct_keys(const RowState &rs, const Uses &u, int col0, int V,
-                                            const int32_t *hist,
+// Adds the drafted history to the decode counts of a tile's (or pass's) columns. The history never
+// counts token 0: the reference pads the history with 0 and then restores the original count of
+// token 0 (core/naive.py:179-203). Only tokens inside the columns are compared with them.
+template <int E>
+__device__ __forceinline__ void add_history(int hist, int col0, i32x4 (&dec)[E / 4]) {
+    uint64_t m = __ballot(hist != 0 && (uint32_t)(hist - col0) < (uint32_t)(SS_BLOCK * E));
+    while (m) {
+        const int t = __builtin_amdgcn_readlane(hist, __builtin_ctzll(m));
+        m &= m - 1;
+        // offset of the token from the lane's element 0, compared with each element's own
+        const int d = t - col0 - 4 * (int)threadIdx.x;
+#pragma unroll
+        for (int j = 0; j < E; ++j) dec[j >> 2][j & 3] += d == (j >> 2) * (SS_BLOCK * 4) + (j & 3) ? 1 : 0;
+    }
+}
+
+template <int E, bool ANY, int ET>
+__device__ __forceinline__ void direct_keys(const RowState &rs, const Uses &u, int col0,
                                             const typename HalfRow<ANY>::Raw (&lw_in)[E / 4],
-                                            const Planes<E, ANY> &pl, Keys<E> &keys) {
+                                            const Planes<E, ANY> &pl, ExcList<ET> &ex, int c0, Keys<E> &keys) {
     constexpr int NCH = E / 4;
     const int lane4 = (int)threadIdx.x * 4;
     bool all_exc;
     const Chain k = row_chain(rs, u, all_exc);
     // logits and bias stay in their loaded bf16 pairs and are widened where they are used
     u32x2 lw[NCH], bw[NCH];
-    bool ok[E];
-    int32_t dec[E], ctx[E];
+    i32x4 dec[NCH];
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
         lw[c] = HalfRow<ANY>::words(lw_in[c], rs.logits);
         bw[c] = HalfRow<ANY>::words(pl.bw[c], rs.bias);
-        const int col = col0 + c * (SS_BLOCK * 4) + lane4;
-        dec[4 * c + 0] = pl.dw[c].x; dec[4 * c + 1] = pl.dw[c].y; dec[4 * c + 2] = pl.dw[c].z; dec[4 * c + 3] = pl.dw[c].w;
-        ctx[4 * c + 0] = pl.cw[c].x; ctx[4 * c + 1] = pl.cw[c].y; ctx[4 * c + 2] = pl.cw[c].z; ctx[4 * c + 3] = pl.cw[c].w;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ok[4 * c + i] = (ANY ? col + i : col) < V;
+        dec[c] = pl.dw[c];
     }
     if (u.g) {
         // a masked element becomes bf16 -inf (0xff80) in place
@@ -565,60 +659,24 @@ __device__ __forceinline__ void direct_keys(const RowState &rs, const Uses &u, i
             lw[c].y = (g & 8u) ? lw[c].y : ((lw[c].y & 0x0000ffffu) | 0xff800000u);
         }
     }
-    if (u.rep && rs.nhist > 0) {
-        // The history never counts token 0: the reference pads the history with 0 and then
-        // restores the original count of token 0 (core/naive.py:179-203).
-        // Offset of the token from the lane's element 0, compared with each element's constant
-        // offset (j / 4) * 1024 + j % 4, so no per-element column is kept live.
-        const int base = rs.shard + col0 + 4 * (int)threadIdx.x;
-        for (int h = 0; h < rs.nhist; ++h) {
-            const int t = hist[h];
-            if (t == 0) continue;
-            const int d = t - base;
-#pragma unroll
-            for (int j = 0; j < E; ++j) dec[j] += d == (j >> 2) * (SS_BLOCK * 4) + (j & 3) ? 1 : 0;
-        }
-    }
-    auto x = [&](int j) {
-        const uint32_t w = (j & 2) ? lw[j >> 2].y : lw[j >> 2].x;
-        return __uint_as_float((j & 1) ? (w & 0xffff0000u) : (w << 16));
-    };
-    auto bb = [&](int j) {
-        const uint32_t w = (j & 2) ? bw[j >> 2].y : bw[j >> 2].x;
-        return (j & 1) ? (w & 0xffff0000u) : (w << 16);
-    };
-    // the bias word of the element's pair, shifted so that -0 in the high half does not count
-    auto bz = [&](int j) { return ((j & 2) ? bw[j >> 2].y : bw[j >> 2].x) << 1; };
-    auto pair = [&](int j) { return (j & 2) ? lw[j >> 2].y : lw[j >> 2].x; };
-    finish_keys<E>(k, all_exc, col0 + SS_BLOCK * E > V, x, pair, all_exc || u.rep || u.mult || u.bias, ok,
-                   dec, ctx, bb, bz, keys);
+    if (u.rep) add_history<E>(rs.hist, rs.shard + col0, dec);
+    finish_keys<E, ET>(k, all_exc, all_exc || u.rep || u.mult || u.bias, lw, bw, dec, pl.cw, ex, c0, keys);
 }
 
 // Direct layout, row with every side plane off (no grammar, penalty or bias): the keys come from
 // the logits alone and no other plane is read.
 template <int E, bool ANY>
-__device__ __forceinline__ void plain_keys(const RowState &rs, const Uses &u, int col0, int V,
-                                           const typename HalfRow<ANY>::Raw (&lw_in)[E / 4], Keys<E> &keys) {
-    const int lane4 = (int)threadIdx.x * 4;
+__device__ __forceinline__ void plain_keys(const RowState &rs, const Uses &u,
+                                           const typename HalfRow<ANY>::Raw (&lw_in)[E / 4], ExcList<E> &ex,
+                                           Keys<E> &keys) {
     bool all_exc;
     const Chain k = row_chain(rs, u, all_exc);
     u32x2 lw[E / 4];
-    bool ok[E];
+    const u32x2 none[E / 4] = {};
+    const i32x4 zero[E / 4] = {};
 #pragma unroll
-    for (int c = 0; c < E / 4; ++c) {
-        lw[c] = HalfRow<ANY>::words(lw_in[c], rs.logits);
-        const int col = col0 + c * (SS_BLOCK * 4) + lane4;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ok[4 * c + i] = (ANY ? col + i : col) < V;
-    }
-    const int32_t zero[E] = {};
-    auto x = [&](int j) {
-        const uint32_t w = (j & 2) ? lw[j >> 2].y : lw[j >> 2].x;
-        return __uint_as_float((j & 1) ? (w & 0xffff0000u) : (w << 16));
-    };
-    auto none = [](int) { return 0u; };
-    auto pair = [&](int j) { return (j & 2) ? lw[j >> 2].y : lw[j >> 2].x; };
-    finish_keys<E>(k, false, col0 + SS_BLOCK * E > V, x, pair, false, ok, zero, zero, none, none, keys);
+    for (int c = 0; c < E / 4; ++c) lw[c] = HalfRow<ANY>::words(lw_in[c], rs.logits);
+    finish_keys<E, E>(k, false, false, lw, none, zero, zero, ex, 0, keys);
 }
 
 // Gather layout: columns remapped by d2t into the target vocabulary, or a shard that starts inside
@@ -645,37 +703,25 @@ __device__ __forceinline__ void load_d2t(const RowState &rs, int col0, int V, in
 
 // PRE: the d2t targets of the E columns come in `pre` (load_d2t, issued by the caller before the
 // grammar staging's barrier, so that both round trips overlap) instead of being loaded here.
-template <int E, bool ANY, bool PRE = false>
+template <int E, bool ANY, int ET, bool PRE = false>
 __device__ __forceinline__ void gather_keys(const RowState &rs, const Uses &u, int col0, int V,
-                                            const int32_t *hist,
-                                            const typename HalfRow<ANY>::Raw (&lw)[E / 4],
+                                            const typename HalfRow<ANY>::Raw (&lw)[E / 4], ExcList<ET> &ex, int c0,
                                             Keys<E> &keys, const int32_t *pre = nullptr) {
     constexpr int NCH = E / 4;
-    const int lane4 = (int)threadIdx.x * 4;
     bool all_exc;
     const Chain k = row_chain(rs, u, all_exc);
 
     // logits and bias stay in bf16 pairs (element 2i in the low half), as loaded: widened where
     // they are used, they would hold one register per element
-    u32x2 lv[NCH];
-    bool ok[E];
+    u32x2 lv[NCH], bw[NCH];
+    i32x4 dec[NCH], ctx[NCH];
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
         lv[c] = HalfRow<ANY>::words(lw[c], rs.logits);
-        const int col = col0 + c * (SS_BLOCK * 4) + lane4;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ok[4 * c + i] = (ANY ? col + i : col) < V;
+        bw[c] = u32x2{0, 0};
+        dec[c] = i32x4{0, 0, 0, 0};
+        ctx[c] = i32x4{0, 0, 0, 0};
     }
-
-    int32_t dec[E], ctx[E];
-    uint32_t bpk[E / 2];
-#pragma unroll
-    for (int j = 0; j < E; ++j) {
-        dec[j] = 0;
-        ctx[j] = 0;
-    }
-#pragma unroll
-    for (int i = 0; i < E / 2; ++i) bpk[i] = 0;
     if (u.g || u.rep || u.bias) {
         int tcol[E];
 #pragma unroll
@@ -724,38 +770,31 @@ __device__ __forceinline__ void gather_keys(const RowState &rs, const Uses &u, i
         if (u.rep) {
             const __amdgpu_buffer_rsrc_t d = row_buffer(rs.dec, (int64_t)rs.vt * 4);
 #pragma unroll
-            for (int j = 0; j < E; ++j) dec[j] = __builtin_amdgcn_raw_buffer_load_b32(d, tcol[j] * 4, 0, 0);
-            if (rs.nhist > 0) {
-                // The history never counts token 0 (core/naive.py:179-203).
-                for (int h = 0; h < rs.nhist; ++h) {
-                    const int t = hist[h];
-#pragma unroll
-                    for (int j = 0; j < E; ++j) dec[j] += (tcol[j] == t && t != 0) ? 1 : 0;
-                }
-            }
+            for (int j = 0; j < E; ++j) dec[j >> 2][j & 3] = __builtin_amdgcn_raw_buffer_load_b32(d, tcol[j] * 4, 0, 0);
         }
         if (u.mult) {
             const __amdgpu_buffer_rsrc_t q = row_buffer(rs.ctx, (int64_t)rs.vt * 4);
 #pragma unroll
-            for (int j = 0; j < E; ++j) ctx[j] = __builtin_amdgcn_raw_buffer_load_b32(q, tcol[j] * 4, 0, 0);
+            for (int j = 0; j < E; ++j) ctx[j >> 2][j & 3] = __builtin_amdgcn_raw_buffer_load_b32(q, tcol[j] * 4, 0, 0);
         }
         if (u.bias) {
             const __amdgpu_buffer_rsrc_t b = row_buffer(rs.bias, (int64_t)rs.vt * 2);
 #pragma unroll
-            for (int j = 0; j < E; ++j)
-                bpk[j >> 1] |= (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(b, tcol[j] * 2, 0, 0) << (16 * (j & 1));
+            for (int j = 0; j < E; ++j) {
+                const uint32_t h = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(b, tcol[j] * 2, 0, 0) << (16 * (j & 1));
+                if (j & 2) bw[j >> 2].y |= h; else bw[j >> 2].x |= h;
+            }
+        }
+        if (u.rep) {
+            // The history never counts token 0 (core/naive.py:179-203).
+            for (uint64_t m = __ballot(rs.hist != 0); m; m &= m - 1) {
+                const int t = __builtin_amdgcn_readlane(rs.hist, __builtin_ctzll(m));
+#pragma unroll
+                for (int j = 0; j < E; ++j) dec[j >> 2][j & 3] += tcol[j] == t ? 1 : 0;
+            }
         }
     }
-    auto x = [&](int j) {
-        const uint32_t w = (j & 2) ? lv[j >> 2].y : lv[j >> 2].x;
-        return __uint_as_float((j & 1) ? (w & 0xffff0000u) : (w << 16));
-    };
-    auto bb = [&](int j) { return (j & 1) ? (bpk[j >> 1] & 0xffff0000u) : (bpk[j >> 1] << 16); };
-    // the bias word of the element's pair, shifted so that -0 in the high half does not count
-    auto bw = [&](int j) { return bpk[j >> 1] << 1; };
-    auto pair = [&](int j) { return (j & 2) ? lv[j >> 2].y : lv[j >> 2].x; };
-    finish_keys<E>(k, all_exc, col0 + SS_BLOCK * E > V, x, pair, all_exc || u.rep || u.mult || u.bias, ok,
-                   dec, ctx, bb, bw, keys);
+    finish_keys<E, ET>(k, all_exc, all_exc || u.rep || u.mult || u.bias, lv, bw, dec, ctx, ex, c0, keys);
 }
 
 // Quads of workgroup memory a staged grammar row occupies: stage_grammar fills whole blocks of 64
@@ -819,32 +858,43 @@ using LogitChunk = typename HalfRow<(MODE & MODE_ANY) != 0>::Raw;
 // would index the key array at run time and place it in scratch memory.
 template <int E, int MODE, int H>
 __device__ __forceinline__ void gather_pass(const RowState &rs, const Uses &u, int col0, int V,
-                                            const int32_t *hist, Keys<E> &keys) {
+                                            ExcList<E> &ex, Keys<E> &keys) {
     constexpr bool ANY = (MODE & MODE_ANY) != 0;
     if constexpr (H < E / 16) {
         LogitChunk<MODE> lh[4];
         load_logits<16, ANY>(rs.logits, col0 + 4 * 4 * SS_BLOCK * H, V, lh);
         Keys<16> kh;
-        gather_keys<16, ANY>(rs, u, col0 + 4 * 4 * SS_BLOCK * H, V, hist, lh, kh);
+        gather_keys<16, ANY, E>(rs, u, col0 + 4 * 4 * SS_BLOCK * H, V, lh, ex, 4 * H, kh);
 #pragma unroll
         for (int i = 0; i < 8; ++i) keys.p[8 * H + i] = kh.p[i];
-        gather_pass<E, MODE, H + 1>(rs, u, col0, V, hist, keys);
+        gather_pass<E, MODE, H + 1>(rs, u, col0, V, ex, keys);
     }
 }
 
 // Streams one tile of one row through the processor chain and returns the keys (0 = absent).
-// `lw` holds the tile's logits from load_logits.
+// `lw` holds the tile's logits from load_logits, `exc` the memory of the waves' exception lists
+// (SS_WAVES lists of `cap` records).
 // PRE (gather layout, E <= 32): the d2t targets of the tile's columns come in `pre` (load_d2t).
-template <int E, int MODE, bool PRE = false>
-__device__ __forceinline__ void prologue_keys(const RowState &rs, int col0, int V,
-                                              const int32_t *hist, const LogitChunk<MODE> (&lw)[E / 4],
-                                              Keys<E> &keys, const int32_t *pre = nullptr) {
+// AUX: cache policy of the side planes' loads (direct layout).
+template <int E, int MODE, bool PRE = false, int AUX = NT>
+__device__ __forceinline__ void prologue_keys(const RowState &rs, int col0, int V, uint32_t *exc, uint32_t cap,
+                                              const LogitChunk<MODE> (&lw)[E / 4], Keys<E> &keys,
+                                              const int32_t *pre = nullptr) {
     constexpr bool ANY = (MODE & MODE_ANY) != 0;
     static_assert(!PRE || ((MODE & MODE_GATHER) && E <= 32), "pre-loaded d2t targets: gather layout, E <= 32");
     const Uses u = row_uses(rs);
+    const bool planes = u.g || u.rep || u.mult || u.bias;
+    ExcList<E> ex;
+    ex.mem = exc + (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * cap * ExcList<E>::WORDS;
+    ex.cap = cap;
+    ex.cnt = 0;
+    auto finish = [&]() {
+        bool all_exc;
+        finish_exceptions<E>(fast_chain(row_chain(rs, u, all_exc)), ex, keys);
+    };
     if constexpr (!(MODE & MODE_GATHER)) {
-        if (!(u.g || u.rep || u.mult || u.bias)) {
-            plain_keys<E, ANY>(rs, u, col0, V, lw, keys);
+        if (!planes) {
+            plain_keys<E, ANY>(rs, u, lw, ex, keys);
         } else if constexpr (E >= 32) {
             // The processor chain in 4096-column passes: element j of pass h is element j + 16 h
             // of the tile (4 h chunks of 1024 columns further). Its per-element state for all E
@@ -853,31 +903,33 @@ __device__ __forceinline__ void prologue_keys(const RowState &rs, int col0, int 
             // rows alone).
 #pragma unroll
             for (int h = 0; h < E / 16; ++h) {
-                // at E = 64 a pass reloads its logits with its planes (in the same round of loads):
-                // the preloaded ones would stay live through every pass
                 LogitChunk<MODE> lh[4];
-                if constexpr (E >= 64) {
+                if constexpr (E >= 64 && ANY) {
+                    // reloaded with the pass's planes: three dwords a chunk kept live through every
+                    // pass would hold 138 VGPRs (three waves per SIMD)
                     load_logits<16, ANY>(rs.logits, col0 + 4 * 4 * SS_BLOCK * h, V, lh);
                 } else {
 #pragma unroll
                     for (int c = 0; c < 4; ++c) lh[c] = lw[4 * h + c];
                 }
                 Planes<16, ANY> pl;
-                issue_planes<16, ANY>(rs, u, true, rs.shard + col0 + 4 * 4 * SS_BLOCK * h, pl);
+                issue_planes<16, ANY, AUX>(rs, u, true, rs.shard + col0 + 4 * 4 * SS_BLOCK * h, pl);
                 Keys<16> kh;
-                direct_keys<16, ANY>(rs, u, col0 + 4 * 4 * SS_BLOCK * h, V, hist, lh, pl, kh);
+                direct_keys<16, ANY, E>(rs, u, col0 + 4 * 4 * SS_BLOCK * h, lh, pl, ex, 4 * h, kh);
 #pragma unroll
                 for (int i = 0; i < 8; ++i) keys.p[8 * h + i] = kh.p[i];
             }
+            finish();
         } else {
             Planes<E, ANY> pl;
-            issue_planes<E, ANY>(rs, u, true, rs.shard + col0, pl);
-            direct_keys<E, ANY>(rs, u, col0, V, hist, lw, pl, keys);
+            issue_planes<E, ANY, AUX>(rs, u, true, rs.shard + col0, pl);
+            direct_keys<E, ANY, E>(rs, u, col0, lw, pl, ex, 0, keys);
+            finish();
         }
     } else if constexpr (E >= 64) {
         // 4096-column passes, as above: the gathered columns and planes of all elements at once
         // would hold 156 VGPRs at E = 32 (three waves per SIMD).
-        gather_pass<E, MODE, 0>(rs, u, col0, V, hist, keys);
+        gather_pass<E, MODE, 0>(rs, u, col0, V, ex, keys);
     } else if constexpr (E >= 32) {
         // two passes, which the compiler unrolls (and schedules in fewer registers than the
         // recursive form: 96 VGPRs against 102 at E = 32)
@@ -887,13 +939,16 @@ __device__ __forceinline__ void prologue_keys(const RowState &rs, int col0, int 
 #pragma unroll
             for (int c = 0; c < 4; ++c) lh[c] = lw[4 * h + c];
             Keys<16> kh;
-            gather_keys<16, ANY, PRE>(rs, u, col0 + 4 * 4 * SS_BLOCK * h, V, hist, lh, kh, PRE ? pre + 16 * h : nullptr);
+            gather_keys<16, ANY, E, PRE>(rs, u, col0 + 4 * 4 * SS_BLOCK * h, V, lh, ex, 4 * h, kh,
+                                         PRE ? pre + 16 * h : nullptr);
 #pragma unroll
             for (int i = 0; i < 8; ++i) keys.p[8 * h + i] = kh.p[i];
         }
     } else {
-        gather_keys<E, ANY, PRE>(rs, u, col0, V, hist, lw, keys, pre);
+        gather_keys<E, ANY, E, PRE>(rs, u, col0, V, lw, ex, 0, keys, pre);
     }
+    if ((MODE & MODE_GATHER) && planes) finish();
+    mask_absent<E>(col0, V, keys);
 }
 
 // Workgroup-wide sum of one count per thread. All threads call.
@@ -906,10 +961,6 @@ __device__ __forceinline__ uint32_t block_count(uint32_t n, uint32_t *red) {
     for (int w = 0; w < SS_WAVES; ++w) s += red[w];
     __syncthreads();
     return s;
-}
-
-__device__ __forceinline__ uint32_t mbcnt64(uint64_t m) {
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
 // A wave's keys as wave_survivors_masked spilled them to workgroup memory (pair i of lane l at

@@ -308,7 +308,6 @@ __global__ __launch_bounds__(SS_BLOCK) void topk_tiles_kernel(const uint16_t *p_
     const int tile = (int)blockIdx.x - row * tiles;
     const int col0 = tile * p_block_n;
     const uint16_t *lrow = p_logits + (int64_t)row * p_stride;
-    const int lane4 = 4 * (int)threadIdx.x;
     typename HalfRow<ANY>::Raw lw[E / 4];
     load_logits<E, ANY>(lrow, col0, p_vocab, lw);
     Keys<E> keys;
@@ -318,15 +317,7 @@ __global__ __launch_bounds__(SS_BLOCK) void topk_tiles_kernel(const uint16_t *p_
         keys.p[2 * c] = packed_keys(w.x);
         keys.p[2 * c + 1] = packed_keys(w.y);
     }
-    if (col0 + SS_BLOCK * E > p_vocab) {
-        // columns past the vocabulary are absent (key 0)
-#pragma unroll
-        for (int c = 0; c < E / 4; ++c) {
-            const int left = p_vocab - (col0 + c * (SS_BLOCK * 4) + lane4);  // columns of the chunk in it
-            keys.p[2 * c] &= (left > 0 ? 0xffffu : 0u) | (left > 1 ? 0xffff0000u : 0u);
-            keys.p[2 * c + 1] &= (left > 2 ? 0xffffu : 0u) | (left > 3 ? 0xffff0000u : 0u);
-        }
-    }
+    mask_absent<E>(col0, p_vocab, keys);
     tile_stage<E, true>(sm, false, keys, p_scratch + (int64_t)row * p_stride_scratch, tile,
                         min(p_block_n, p_vocab - col0), p_k);
 }
@@ -796,18 +787,20 @@ extern "C" int ss_topk(const ss_topk_args *a) {
     if (a->rows == 0) return SS_OK;
     if (a->strategy < SS_STRATEGY_AUTO || a->strategy > SS_STRATEGY_ROWWISE) return SS_ERR_INVALID_ARGUMENT;
     // One 1024-thread workgroup per row (one launch) serves rows of at most 32768 columns on
-    // request. AUTO takes it where it measured faster than the tile grid: float32, at least 48 rows
-    // of more than 16384 columns and k <= 32 (rows of 32000 columns at k = 32, back to back: 48 rows
-    // 9.3 us against 9.6, 128 rows 9.7 against 11.3, 256 rows 12.1 against 17.0). Fewer rows leave
+    // request. AUTO takes it from 48 rows of more than 16384 columns at k <= 32 on, where it measured
+    // faster than the tile grid. float32 (rows of 32000 columns at k = 32, back to back): 48 rows
+    // 9.3 us against 9.6, 128 rows 9.7 against 11.3, 256 rows 12.1 against 17.0. Fewer rows leave
     // CUs idle while one CU streams each row (32 rows: 9.2 against 8.6 us), narrower rows leave most
     // of a thread's 32 elements empty, and a larger k overflows the survivor list into the exact
-    // selection. bfloat16 rows take the tile grid (20000-32768 columns, k 8 and 32, at the best
-    // width: 48 rows 6.7-7.2 us against 8.4-9.0, 512 rows 11.7-12.9 against 16.6-17.9; only at 256
-    // rows are the two level, 8.9-9.8 against 8.9-9.6).
+    // selection. bfloat16: up to 256 rows, one workgroup a CU, where the GPU's time is near the tile
+    // grid's (128 rows 8.9 us against 8.0, 256 rows 9.1-9.4 against 9.7-9.8) and the launch saved
+    // decides an eager call's (125 rows at k = 8: 13.4 us against 16.0); from there on the tile grid
+    // wins (512 rows 11.7-12.9 us against 16.6-17.9).
     if (a->strategy == SS_STRATEGY_ROWWISE && a->vocab_size > ss::TOPK_WIDE_THREADS * ss::TOPK_WIDE_E) return SS_ERR_UNSUPPORTED;
     const bool wide = a->strategy == SS_STRATEGY_ROWWISE ||
-                      (a->strategy == SS_STRATEGY_AUTO && a->dtype == SS_DTYPE_F32 && a->rows >= 48 && a->k <= 32 &&
-                       a->vocab_size > 16384 && a->vocab_size <= ss::TOPK_WIDE_THREADS * ss::TOPK_WIDE_E);
+                      (a->strategy == SS_STRATEGY_AUTO && a->rows >= 48 &&
+                       (a->dtype == SS_DTYPE_F32 || a->rows <= 256) && a->k <= 32 && a->vocab_size > 16384 &&
+                       a->vocab_size <= ss::TOPK_WIDE_THREADS * ss::TOPK_WIDE_E);
     if (a->dtype == SS_DTYPE_F32)
         return wide ? ss::launch_topk_rows<true, false>(a) : ss::launch_topk<true, false>(a, tiles);
     if (ss::topk_any(a))

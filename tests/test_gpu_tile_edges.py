@@ -125,3 +125,33 @@ def test_rows_at_any_half_word(block, vocab, offset, pad):
                           want, got):
 
         assert torch.equal(a, b), f"{name} differ between aligned rows and rows at offset {offset}, pad {pad}"
+
+
+@pytest.mark.parametrize("density", [0.0005, 0.01, 0.04, 0.1, 0.3])
+@pytest.mark.parametrize("block,vocab", [(1024, 3000), (2048, 8193), (4096, 9000), (8192, 33000), (16384, 40002)])
+def test_count_and_bias_density(block, vocab, density, monkeypatch):
+    """Rows whose counts and biases are nonzero in few columns keep them in the waves' exception
+    lists, in more columns overflow the lists pass by pass: the decode step, the verification (with
+    drafted history) and drafting through d2t against the oracle."""
+
+    import test_gpu_sweep as sweep
+
+    whole = sweep.random_host
+
+    def thinned(slots, timesteps, vocab, seed, indicator=None, **kw):
+
+        host = whole(slots, timesteps, vocab, seed, indicator, **kw)
+        g = torch.Generator().manual_seed(seed)
+
+        for plane in (host.repetition.counts.context, host.repetition.counts.decode, host.bias):
+
+            plane.masked_fill_(torch.rand(plane.shape, generator=g) >= density, 0)
+
+        return host
+
+    monkeypatch.setattr(sweep, "random_host", thinned)
+    seed = 4000 + block + int(1000 * density)
+    sweep.test_sweep_autoregressive(block, vocab, "random", "spiked", seed)
+    sweep.test_sweep_multistep_row_top128(block, vocab, "random", "spiked", seed)
+    sweep.test_sweep_drafting_d2t(block, vocab, "sparse", "spiked", seed)
+    sweep.test_sweep_drafting_d2t(block, vocab, "random", "few", seed + 1)
