@@ -1,4 +1,6 @@
-"""Builds the gfx950 HIP library ``sonic_sampler/_lib/libsonic_sampler.so`` with hipcc.
+"""Builds the gfx950 HIP library ``sonic_sampler/_lib/libsonic_sampler.so`` with hipcc, and the host
+extension ``sonic_sampler/_lib/_sonic_host.so`` (the native part of the eager call path) with g++
+against the running interpreter's torch.
 
 Usage: ``python sonic-sampler_amd/build_native.py`` (also called by ``__graft_entry__.build``).
 The library exports the C-ABI declared in ``include/sonic_sampler.h``. Objects go to ``_build/``
@@ -11,6 +13,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -18,6 +21,8 @@ HERE = Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 BUILD = HERE / "_build"
 OUT = HERE / "sonic_sampler" / "_lib" / "libsonic_sampler.so"
+HOST_SRC = CSRC / "host" / "sonic_host.cpp"
+HOST_OUT = OUT.with_name("_sonic_host.so")
 
 ARCH = os.environ.get("SS_OFFLOAD_ARCH", "gfx950")
 
@@ -57,13 +62,36 @@ def _compile(src: Path) -> Path:
     return obj
 
 
+def _build_host() -> None:
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    cxx = shutil.which(os.environ.get("CXX", "g++"))
+    if not cxx:
+        raise RuntimeError("no C++ compiler found: the host extension of sonic_sampler needs one")
+    tmp = HOST_OUT.with_suffix(".so.tmp")
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-isystem", str(root / "include"), "-isystem", str(root / "include/torch/csrc/api/include"),
+           "-isystem", sysconfig.get_paths()["include"], str(HOST_SRC), "-o", str(tmp),
+           f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"compiling {HOST_SRC.name} failed:\n{proc.stderr}")
+    if proc.stderr.strip():
+        print(proc.stderr, file=sys.stderr)
+    os.replace(tmp, HOST_OUT)
+
+
 def build(verbose: bool = True) -> Path:
     BUILD.mkdir(parents=True, exist_ok=True)
     OUT.parent.mkdir(parents=True, exist_ok=True)
     sources = sorted(CSRC.glob("*.hip")) + sorted(CSRC.glob("*.cpp"))
-    jobs = min(len(sources), max(1, min(8, os.cpu_count() or 1)))
+    jobs = min(len(sources) + 1, max(1, min(8, os.cpu_count() or 1)))
     with ThreadPoolExecutor(max_workers=jobs) as pool:
+        host = pool.submit(_build_host)
         objects = list(pool.map(_compile, sources))
+        host.result()
     tmp = OUT.with_suffix(".so.tmp")
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objects), "-o", str(tmp)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
@@ -71,7 +99,7 @@ def build(verbose: bool = True) -> Path:
         raise RuntimeError(f"linking {OUT.name} failed:\n{proc.stderr}")
     os.replace(tmp, OUT)
     if verbose:
-        print(f"built {OUT.relative_to(HERE.parent)} ({len(sources)} sources, {ARCH})")
+        print(f"built {OUT.relative_to(HERE.parent)} ({len(sources)} sources, {ARCH}) and {HOST_OUT.name}")
     return OUT
 
 

@@ -1,0 +1,238 @@
+// Native part of the eager call path: a Python extension (CPython API and torch's C++ tensors) that
+// turns a call's tensors and scalars into the bytes of its argument struct and allocates its
+// outputs. Both were most of a small call's host time in Python: about 25 attribute and method calls
+// on tensors per argument struct and a keyword-parsed torch.empty per output.
+//
+//   make_layout(size, fields) -> capsule     fields: (code, offset, offset, offset, name) per argument
+//   gather(capsule, *args) -> bytes          the struct, every other byte zero
+//   empty(device, dtype, *sizes) -> Tensor   torch.empty
+//   entry(address) -> callable               the entry point at `address`, taking the struct's bytes
+//
+// Argument codes: a scalar of the field's type ('i', 'I', 'q', 'Q'), or a tensor (None: zeros) whose
+// address goes to the first offset ('T'), with its leading stride ('S'), or its leading and, of a
+// three-dimensional one, its second stride ('U'). Lower case 't', 's', 'u': the tensor must be
+// contiguous along its last dimension (ValueError).
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <torch/csrc/Device.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cstring>
+#include <exception>
+#include <string>
+#include <vector>
+
+namespace {
+
+struct Field {
+    char code;
+    Py_ssize_t at[3];
+    std::string name;
+};
+
+struct Layout {
+    Py_ssize_t size;
+    std::vector<Field> fields;
+};
+
+constexpr const char *CAPSULE = "sonic_sampler.layout";
+
+void destroy(PyObject *capsule) { delete static_cast<Layout *>(PyCapsule_GetPointer(capsule, CAPSULE)); }
+
+int field_bytes(char code) { return code == 'i' || code == 'I' ? 4 : 8; }
+
+PyObject *make_layout(PyObject *, PyObject *args) {
+    Py_ssize_t size = 0;
+    PyObject *list = nullptr;
+    if (!PyArg_ParseTuple(args, "nO!", &size, &PyList_Type, &list)) return nullptr;
+    auto layout = std::make_unique<Layout>();
+    layout->size = size;
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(list); ++i) {
+        int code = 0;
+        const char *name = nullptr;
+        Field f;
+        if (!PyArg_ParseTuple(PyList_GET_ITEM(list, i), "Cnnns", &code, &f.at[0], &f.at[1], &f.at[2], &name)) return nullptr;
+        f.code = (char)code;
+        f.name = name;
+        if (!std::strchr("iIqQTSUtsu", f.code)) {
+            PyErr_Format(PyExc_ValueError, "unknown field code %c", code);
+            return nullptr;
+        }
+        const int used = f.code == 'S' || f.code == 's' ? 2 : f.code == 'U' || f.code == 'u' ? 3 : 1;
+        for (int k = 0; k < used; ++k) {
+            if (f.at[k] < 0 || f.at[k] + field_bytes(f.code) > size) {
+                PyErr_Format(PyExc_ValueError, "field %s outside the struct", name);
+                return nullptr;
+            }
+        }
+        layout->fields.push_back(std::move(f));
+    }
+    return PyCapsule_New(layout.release(), CAPSULE, destroy);
+}
+
+// Writes one argument of the struct; false with a Python error set.
+bool put(const Field &f, PyObject *arg, char *out) {
+    if (f.code == 'q' || f.code == 'i') {
+        const long long v = PyLong_AsLongLong(arg);
+        if (v == -1 && PyErr_Occurred()) return false;
+        if (f.code == 'q') {
+            std::memcpy(out + f.at[0], &v, 8);
+            return true;
+        }
+        const int32_t w = (int32_t)v;
+        if (w != v) {
+            PyErr_Format(PyExc_OverflowError, "%s does not fit 32 bits", f.name.c_str());
+            return false;
+        }
+        std::memcpy(out + f.at[0], &w, 4);
+        return true;
+    }
+    if (f.code == 'Q' || f.code == 'I') {
+        PyObject *index = PyNumber_Index(arg);  // integers of other types (numpy's) too
+        if (!index) return false;
+        const unsigned long long v = PyLong_AsUnsignedLongLong(index);
+        Py_DECREF(index);
+        if (v == (unsigned long long)-1 && PyErr_Occurred()) return false;
+        if (f.code == 'Q') {
+            std::memcpy(out + f.at[0], &v, 8);
+            return true;
+        }
+        const uint32_t w = (uint32_t)v;
+        if (w != v) {
+            PyErr_Format(PyExc_OverflowError, "%s does not fit 32 bits", f.name.c_str());
+            return false;
+        }
+        std::memcpy(out + f.at[0], &w, 4);
+        return true;
+    }
+    if (arg == Py_None) return true;
+    if (!THPVariable_Check(arg)) {
+        PyErr_Format(PyExc_TypeError, "`%s` must be a tensor or None", f.name.c_str());
+        return false;
+    }
+    const at::Tensor &t = THPVariable_Unpack(arg);
+    const bool unit = f.code >= 'a';
+    if (unit && t.dim() > 0 && t.stride(-1) != 1) {
+        PyErr_Format(PyExc_ValueError, "`%s` must be contiguous along its last dimension", f.name.c_str());
+        return false;
+    }
+    const uint64_t p = (uint64_t)(uintptr_t)t.data_ptr();
+    std::memcpy(out + f.at[0], &p, 8);
+    if (f.code != 'T' && f.code != 't') {
+        const int64_t s = t.stride(0);
+        std::memcpy(out + f.at[1], &s, 8);
+        if (f.code == 'U' || f.code == 'u') {
+            const int64_t step = t.dim() >= 3 ? t.stride(1) : 0;
+            std::memcpy(out + f.at[2], &step, 8);
+        }
+    }
+    return true;
+}
+
+// Runs fn, with a C++ exception (torch's among them) as a RuntimeError.
+template <class F>
+PyObject *guarded(F fn) {
+    try {
+        return fn();
+    } catch (const std::exception &e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+    } catch (...) {
+        PyErr_SetString(PyExc_RuntimeError, "unknown C++ exception");
+    }
+    return nullptr;
+}
+
+PyObject *gather(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    if (n < 1) {
+        PyErr_SetString(PyExc_TypeError, "gather(layout, *args)");
+        return nullptr;
+    }
+    const auto *layout = static_cast<Layout *>(PyCapsule_GetPointer(args[0], CAPSULE));
+    if (!layout) return nullptr;
+    if ((size_t)(n - 1) != layout->fields.size()) {
+        PyErr_Format(PyExc_TypeError, "expected %zu arguments, got %zd", layout->fields.size(), n - 1);
+        return nullptr;
+    }
+    PyObject *bytes = PyBytes_FromStringAndSize(nullptr, layout->size);
+    if (!bytes) return nullptr;
+    char *out = PyBytes_AS_STRING(bytes);
+    std::memset(out, 0, (size_t)layout->size);
+    PyObject *done = guarded([&]() -> PyObject * {
+        for (size_t i = 0; i < layout->fields.size(); ++i)
+            if (!put(layout->fields[i], args[i + 1], out)) return nullptr;
+        return bytes;
+    });
+    if (!done) Py_DECREF(bytes);
+    return done;
+}
+
+PyObject *empty(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    if (n < 3 || n > 6 || !THPDevice_Check(args[0]) || !THPDtype_Check(args[1])) {
+        PyErr_SetString(PyExc_TypeError, "empty(device, dtype, *sizes) with 1 to 4 sizes");
+        return nullptr;
+    }
+    int64_t sizes[4];
+    for (Py_ssize_t i = 2; i < n; ++i) {
+        sizes[i - 2] = PyLong_AsLongLong(args[i]);
+        if (sizes[i - 2] == -1 && PyErr_Occurred()) return nullptr;
+    }
+    return guarded([&]() -> PyObject * {
+        const auto options = at::TensorOptions()
+                                 .device(reinterpret_cast<THPDevice *>(args[0])->device)
+                                 .dtype(reinterpret_cast<THPDtype *>(args[1])->scalar_type);
+        return THPVariable_Wrap(at::empty(at::IntArrayRef(sizes, (size_t)(n - 2)), options));
+    });
+}
+
+// An entry point of the library called with the struct's bytes, the GIL released meanwhile.
+PyObject *call_entry(PyObject *self, PyObject *bytes) {
+    using Entry = int (*)(const void *);
+    const auto fn = reinterpret_cast<Entry>(PyLong_AsVoidPtr(self));
+    if (!fn) {
+        if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "no entry point");
+        return nullptr;
+    }
+    if (!PyBytes_Check(bytes)) {
+        PyErr_SetString(PyExc_TypeError, "the argument struct's bytes are expected");
+        return nullptr;
+    }
+    // the argument structs hold 8-byte fields: a payload off an 8-byte boundary is copied
+    const char *p = PyBytes_AS_STRING(bytes);
+    std::vector<uint64_t> aligned;
+    if ((uintptr_t)p % 8 != 0) {
+        aligned.resize(((size_t)PyBytes_GET_SIZE(bytes) + 7) / 8);
+        std::memcpy(aligned.data(), p, (size_t)PyBytes_GET_SIZE(bytes));
+        p = reinterpret_cast<const char *>(aligned.data());
+    }
+    int status = 0;
+    Py_BEGIN_ALLOW_THREADS
+    status = fn(p);
+    Py_END_ALLOW_THREADS
+    return PyLong_FromLong(status);
+}
+
+PyMethodDef call_entry_def = {"call", (PyCFunction)call_entry, METH_O, nullptr};
+
+PyObject *entry(PyObject *, PyObject *address) {
+    if (!PyLong_Check(address)) {
+        PyErr_SetString(PyExc_TypeError, "entry(address)");
+        return nullptr;
+    }
+    return PyCFunction_New(&call_entry_def, address);
+}
+
+PyMethodDef methods[] = {
+    {"make_layout", (PyCFunction)make_layout, METH_VARARGS, nullptr},
+    {"gather", (PyCFunction)(void (*)(void))gather, METH_FASTCALL, nullptr},
+    {"empty", (PyCFunction)(void (*)(void))empty, METH_FASTCALL, nullptr},
+    {"entry", (PyCFunction)entry, METH_O, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_sonic_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__sonic_host() { return PyModule_Create(&module); }

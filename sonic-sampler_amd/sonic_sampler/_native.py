@@ -1,4 +1,5 @@
-"""ctypes binding of the gfx950 HIP library (C-ABI declared in ``include/sonic_sampler.h``).
+"""ctypes binding of the gfx950 HIP library (C-ABI declared in ``include/sonic_sampler.h``), and the
+host extension that packs the eager calls' argument structs and allocates their outputs.
 
 The library is loaded after ``torch`` so that it binds to the HIP runtime torch already mapped
 (both carry the soname ``libamdhip64.so.7``), which makes torch's stream handles valid inside it.
@@ -8,6 +9,9 @@ There is deliberately no CPU fallback: if the library is missing every entry poi
 from __future__ import annotations
 
 import ctypes
+import functools
+import importlib.machinery
+import importlib.util
 import os
 import struct
 from pathlib import Path
@@ -15,6 +19,7 @@ from pathlib import Path
 import torch  # noqa: F401  (must be imported before the HIP library is loaded)
 
 _LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libsonic_sampler.so"
+_HOST_PATH = _LIB_PATH.with_name("_sonic_host.so")
 
 c_p = ctypes.c_void_p
 c_i32 = ctypes.c_int32
@@ -161,6 +166,42 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+@functools.lru_cache(maxsize=None)
+def host():
+    """The host extension (``csrc/host/sonic_host.cpp``); raises if it is absent."""
+
+    if not _HOST_PATH.is_file():
+        raise RuntimeError(
+            f"sonic_sampler host extension not found at {_HOST_PATH}; build it with "
+            "`python sonic-sampler_amd/build_native.py`"
+        )
+
+    loader = importlib.machinery.ExtensionFileLoader("_sonic_host", str(_HOST_PATH))
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_sonic_host", loader))
+    loader.exec_module(module)
+
+    return module
+
+
+_empty = None
+
+
+def empty(device: torch.device | None, dtype: torch.dtype, *sizes: int) -> torch.Tensor:
+    """``torch.empty(sizes, dtype=dtype, device=device)``; natively where the device is known."""
+
+    global _empty
+
+    if device is None:
+
+        return torch.empty(sizes, dtype=dtype)
+
+    if _empty is None:
+
+        _empty = host().empty
+
+    return _empty(device, dtype, *sizes)
+
+
 def check(status: int, what: str) -> None:
 
     if status != SS_OK:
@@ -252,21 +293,56 @@ class Packer:
                                f"the struct {ctypes.sizeof(cls)}")
 
 
+class Gatherer:
+    """The bytes of a ctypes argument struct from a call's tensors and scalars, given positionally in
+    declaration order, packed by the host extension. ``tensors`` names the pointer fields that come
+    as tensors (or None, for zeros) and what is taken of each: "T" its address; "S" also its leading
+    stride, into the field behind (which then is no argument of its own); "U" also the second
+    stride of a three-dimensional one, into the field behind that. In lower case the tensor must be
+    contiguous along its last dimension (ValueError). ``labels`` renames fields in error messages.
+    ``fields`` lists the positions' names."""
+
+    def __init__(self, cls, tensors: dict, labels: dict | None = None):
+
+        layout = _flat_layout(cls)
+        labels = labels or {}
+        rows, i = [], 0
+
+        while i < len(layout):
+
+            name, offset, _, code = layout[i]
+            code = tensors.get(name, code)
+            used = {"S": 2, "U": 3}.get(code.upper(), 1)
+            at = [layout[i + k][1] if k < used else 0 for k in range(3)]
+            rows.append((code, *at, name))
+            i += used
+
+        if unknown := set(tensors) - {name for *_, name in rows}:
+
+            raise ValueError(f"{cls.__name__} has no fields {sorted(unknown)}")
+
+        self.fields = tuple(name for *_, name in rows)
+        self._layout = (ctypes.sizeof(cls), [(*row, labels.get(name, name)) for *row, name in rows])
+
+    @functools.cached_property
+    def gather(self):
+        """gather(*args) -> bytes (built on first use, when the extension is loaded)."""
+
+        return functools.partial(host().gather, host().make_layout(*self._layout))
+
+
 _packed_entries: dict = {}
 
 
 def packed_entry(name: str):
-    """Entry point `name` taking its argument struct as packed bytes (``Packer.pack``) instead of
-    a ctypes struct: a function pointer of its own, apart from ``load().<name>``."""
+    """Entry point `name` taking its argument struct as packed bytes (``Packer.pack``,
+    ``Gatherer.gather``), called natively."""
 
     fn = _packed_entries.get(name)
 
     if fn is None:
 
-        fn = load()[name]
-        fn.restype = c_i32
-        fn.argtypes = [ctypes.c_char_p]
-        _packed_entries[name] = fn
+        fn = _packed_entries[name] = host().entry(ctypes.cast(load()[name], c_p).value)
 
     return fn
 
@@ -301,7 +377,7 @@ def require_device(*tensors: torch.Tensor | None) -> None:
 
     for tensor in tensors:
 
-        if tensor is not None and tensor.device.type != "cuda":
+        if tensor is not None and not tensor.is_cuda:
 
             raise ValueError(
                 f"sonic_sampler kernels run on the GPU only; got a tensor on {tensor.device}"

@@ -14,6 +14,8 @@ import torch
 
 from torch import Tensor
 
+from sonic_sampler import _native
+
 
 DEFAULT_TOP_LOGPROBS: Final[int] = 5
 
@@ -38,8 +40,7 @@ class TopTargets:
 
             shape = (batch_size, timesteps, targets) if timesteps > 1 else (batch_size, targets)
 
-            return cls(tokens=torch.empty(shape, dtype=I32, device=device),
-                       logprobs=torch.empty(shape, dtype=BF16, device=device))
+            return cls(tokens=_native.empty(device, I32, *shape), logprobs=_native.empty(device, BF16, *shape))
 
         return None
 
@@ -48,10 +49,8 @@ class TopTargets:
 
         if targets > 0:
 
-            return cls(
-                tokens=torch.empty(num_tokens, targets, dtype=I32, device=device),
-                logprobs=torch.empty(num_tokens, targets, dtype=BF16, device=device),
-            )
+            return cls(tokens=_native.empty(device, I32, num_tokens, targets),
+                       logprobs=_native.empty(device, BF16, num_tokens, targets))
 
         return None
 
@@ -71,14 +70,14 @@ class LogProbabilities:
         """`device` None: the current default device (the reference allocates under a device
         context; an explicit device avoids entering one on every call)."""
 
-        selected = torch.empty(batch_size, timesteps, dtype=BF16, device=device)
+        selected = _native.empty(device, BF16, batch_size, timesteps)
 
         return cls(selected=selected, top_k=TopTargets.empty_blocked(batch_size, top_k, timesteps, device=device))
 
     @classmethod
     def empty_varlen(cls, num_tokens: int, top_k: int = 0, device=None) -> "LogProbabilities":
 
-        selected = torch.empty(num_tokens, dtype=BF16, device=device)
+        selected = _native.empty(device, BF16, num_tokens)
 
         return cls(selected=selected, top_k=TopTargets.empty_varlen(num_tokens, top_k, device=device))
 
@@ -158,7 +157,7 @@ class Verification:
 
         buffer = None
         device = tokens.device
-        offsets = tokens.new_empty(batch_size, 1, dtype=I32)
+        offsets = _native.empty(device, I32, batch_size, 1)
 
         if logprobs:
 

@@ -62,7 +62,7 @@ def resolve_scratchpad(logits: Tensor, block_n: int, buffer: Optional[Tensor] = 
 
 def collapse_2d(value: Tensor) -> Tensor:
 
-    return value.flatten(0, -2)
+    return value if value.dim() == 2 else value.flatten(0, -2)
 
 
 def unit_stride(name: str, tensor: Optional[Tensor]) -> None:

@@ -46,6 +46,17 @@ TINY: float = torch.finfo(BF16).tiny
 
 MULTISTEP_ARGS = _native.Packer(_native.MultistepArgs)
 
+# the same struct from the call's tensors; their addresses and strides are taken natively
+MULTISTEP_CALL = _native.Gatherer(
+    _native.MultistepArgs,
+    dict(logits="s", cu_seqlens="T", indicators="t", slot_mapping="T", drafted_tokens="T", grammar="u",
+         context_counts="s", decode_counts="s", repetition="T", frequency="T", presence="T", logit_bias="s",
+         temperature="T", top_k="T", top_p="T", min_p="T", top_logprobs="T", draft_probabilities="u", uniform="S",
+         gumbel="u", out_tokens="T", offsets="T", logprobs="T", top_values="T", top_tokens="S", values="T",
+         indices="T", scratch="S"),
+    labels=dict(gumbel="gumbel_noise"),
+)
+
 
 def resolve_batch_vocab(logits: Tensor, cu_seqlens: Optional[Tensor], lookahead: Optional[int]):
     """(varlen, batch, gamma, vocab) from the logits layout (reference ``:50-106``)."""
@@ -122,7 +133,7 @@ def resolve_tokens(drafted: Tensor, output: Optional[Tensor]) -> Tensor:
     token at its offset), so a new buffer holds the same tokens without a copy launch ahead of the
     tile stage."""
 
-    return output if output is not None else torch.empty_like(drafted, memory_format=torch.contiguous_format)
+    return output if output is not None else _native.empty(drafted.device, drafted.dtype, *drafted.shape)
 
 
 def fused_multistep(
@@ -205,13 +216,6 @@ def fused_multistep(
 
     flat_logits = collapse_2d(logits)
 
-    for name, t in (("logits", flat_logits), ("grammar", grammar), ("context_counts", context_counts),
-                    ("decode_counts", decode_counts), ("logit_bias", logit_bias),
-                    ("gumbel_noise", gumbel_noise), ("draft_probabilities", draft_probabilities),
-                    ("indicators", indicators)):
-
-        unit_stride(name, t)
-
     if not drafted_tokens.is_contiguous():
 
         raise ValueError("drafted_tokens must be contiguous")
@@ -259,37 +263,30 @@ def fused_multistep(
             top_values = collapse_2d(verification.logprobs.top_k.logprobs)
             top_tokens = collapse_2d(verification.logprobs.top_k.tokens)
 
-    a = _native.addr
-    s = _native.stride0
-
-    def step_stride(t: Optional[Tensor]) -> int:
-
-        return 0 if t is None else (t.stride(1) if t.dim() >= 3 else 0)
-
     philox_on = philox_seed is not None
     tile_start, tile_end = _native.event_pair(tile_events)
 
-    # ss_multistep_args, field by field in declaration order (MULTISTEP_ARGS.fields names them).
+    if philox_on:
+
+        # not read, but held to the same layout
+        unit_stride("gumbel_noise", gumbel_noise)
+        gumbel_noise = None
+
+    # ss_multistep_args in declaration order (MULTISTEP_CALL.fields names the positions).
     # all_greedy: the caller vouches that every row is greedy, so each request's argmax is taken in
     # the request stage and the row launch is skipped. A hint, never inferred here: a captured graph
     # replays whatever was decided at capture while the indicators may change in place between
     # replays.
-    packed = MULTISTEP_ARGS.pack(
-        a(flat_logits), flat_logits.stride(0), rows, batch_size, vocab_size, block_n, gamma,
+    packed = MULTISTEP_CALL.gather(
+        flat_logits, rows, batch_size, vocab_size, block_n, gamma,
         max_top_logprobs if top_values is not None else 0, int(update_counts), int(token_logprobs is not None),
-        a(cu_seqlens), a(indicators), a(slot_mapping), a(drafted_tokens),
-        a(grammar), s(grammar), step_stride(grammar),
-        a(context_counts), s(context_counts), a(decode_counts), s(decode_counts),
-        a(repetition_penalties), a(frequency_penalties), a(presence_penalties), a(logit_bias), s(logit_bias),
-        a(temperature), a(top_k), a(top_p), a(min_p), a(top_k_logprobs),
-        a(draft_probabilities), s(draft_probabilities), step_stride(draft_probabilities),
-        a(uniform_weights), s(uniform_weights),
-        0 if philox_on else a(gumbel_noise), 0 if philox_on else s(gumbel_noise),
-        0 if philox_on else step_stride(gumbel_noise),
+        cu_seqlens, indicators, slot_mapping, drafted_tokens, grammar, context_counts, decode_counts,
+        repetition_penalties, frequency_penalties, presence_penalties, logit_bias,
+        temperature, top_k, top_p, min_p, top_k_logprobs, draft_probabilities, uniform_weights, gumbel_noise,
         philox_seed & 0xFFFFFFFFFFFFFFFF if philox_on else 0, philox_offset & 0xFFFFFFFF if philox_on else 0,
         int(philox_on),
-        a(tokens), a(verification.offsets), a(token_logprobs), a(top_values), a(top_tokens), s(top_values),
-        a(values_buffer), a(indices_buffer), a(bitpacked), bitpacked.stride(0), _native.stream_of(logits),
+        tokens, verification.offsets, token_logprobs, top_values, top_tokens,
+        values_buffer, indices_buffer, bitpacked, _native.stream_of(logits),
         tile_start or 0, tile_end or 0, int(bool(all_greedy)),
     )
 

@@ -60,10 +60,20 @@ STAGES = {None: 0, "tiles": _native.STAGE_TILES, "rows": _native.STAGE_ROWS}
 
 SINGULAR_ARGS = _native.Packer(_native.SingularArgs)
 
+# the same struct from the call's tensors; their addresses and strides are taken natively
+SINGULAR_CALL = _native.Gatherer(
+    _native.SingularArgs,
+    dict(logits="s", indicators="t", slot_mapping="T", d2t="T", grammar="s", context_counts="s", decode_counts="s",
+         drafted_tokens="s", repetition="T", frequency="T", presence="T", logit_bias="s", temperature="T", top_k="T",
+         top_p="T", min_p="T", top_logprobs="T", gumbel="s", tokens="S", logprobs="S", top_values="T", top_tokens="S",
+         probabilities="s", scratch="S"),
+    labels=dict(gumbel="gumbel_noise", probabilities="draft_probabilities"),
+)
+
 
 def resolve_tokens(buffer: Optional[Tensor], batch_size: int, source: Tensor) -> Tensor:
 
-    return buffer if buffer is not None else source.new_empty(batch_size, 1, dtype=I32)
+    return buffer if buffer is not None else _native.empty(source.device, I32, batch_size, 1)
 
 
 def resolve_probabilities(precondition: bool, source: Tensor, batch_size: int,
@@ -160,13 +170,6 @@ def fused_singular(
 
         raise ValueError(f"top logprobs must be within the interval [0, {MAX_K}]")
 
-    for name, t in (("logits", logits), ("grammar", grammar), ("context_counts", context_counts),
-                    ("decode_counts", decode_counts), ("logit_bias", logit_bias),
-                    ("gumbel_noise", gumbel_noise), ("draft_probabilities", draft_probabilities),
-                    ("indicators", indicators), ("drafted_tokens", drafted_tokens)):
-
-        unit_stride(name, t)
-
     _native.require_device(logits, indicators)
 
     batch_size, vocab_size = logits.shape
@@ -243,29 +246,27 @@ def fused_singular(
         history = timestep if timestep is not None else min(lookahead, drafted_tokens.size(1))
         history = max(0, min(history, drafted_tokens.size(1)))
 
-    a = _native.addr
-    s = _native.stride0
     philox_on = philox_seed is not None
     tile_start, tile_end = _native.event_pair(tile_events)
 
-    # ss_singular_args, field by field in declaration order (SINGULAR_ARGS.fields names them)
-    packed = SINGULAR_ARGS.pack(
-        a(logits), logits.stride(0), batch_size, vocab_size,
+    if philox_on:
+
+        # not read, but held to the same layout
+        unit_stride("gumbel_noise", gumbel_noise)
+        gumbel_noise = None
+
+    # ss_singular_args in declaration order (SINGULAR_CALL.fields names the positions)
+    packed = SINGULAR_CALL.gather(
+        logits, batch_size, vocab_size,
         target_width, block_n, lookahead, history, max_top_logprobs if top_values is not None else 0,
         int(is_prefill), int(update_counts), int(token_logprobs is not None), int(probabilities is not None),
         KERNEL_LAYOUTS[kernel_layout],
-        a(indicators), a(slot_mapping), a(d2t_mapping),
-        a(grammar), s(grammar), a(context_counts), s(context_counts), a(decode_counts), s(decode_counts),
-        a(drafted_tokens) if history else 0, s(drafted_tokens),
-        a(repetition_penalties), a(frequency_penalties), a(presence_penalties),
-        a(logit_bias), s(logit_bias),
-        a(temperature), a(top_k), a(top_p), a(min_p), a(top_k_logprobs),
-        0 if philox_on else a(gumbel_noise), 0 if philox_on else s(gumbel_noise),
+        indicators, slot_mapping, d2t_mapping, grammar, context_counts, decode_counts, drafted_tokens,
+        repetition_penalties, frequency_penalties, presence_penalties, logit_bias,
+        temperature, top_k, top_p, min_p, top_k_logprobs, gumbel_noise,
         philox_seed & 0xFFFFFFFFFFFFFFFF if philox_on else 0, philox_offset & 0xFFFFFFFF if philox_on else 0,
         int(philox_on), philox_step, STAGES[stage],
-        a(final_tokens), final_tokens.stride(0), a(token_logprobs), s(token_logprobs),
-        a(top_values), a(top_tokens), s(top_values), a(probabilities), s(probabilities),
-        a(bitpacked), s(bitpacked), _native.stream_of(logits),
+        final_tokens, token_logprobs, top_values, top_tokens, probabilities, bitpacked, _native.stream_of(logits),
         tile_start or 0, tile_end or 0, world_size, local_rank, shard_size, 0,
     )
 

@@ -31,7 +31,7 @@ BF16 = torch.bfloat16
 FP32 = torch.float32
 I32 = torch.int32
 
-TOPK_ARGS = _native.Packer(_native.TopKArgs)
+TOPK_CALL = _native.Gatherer(_native.TopKArgs, dict(logits="s", scratch="S", values="T", indices="T"))
 
 
 @dataclass(eq=False, kw_only=True)
@@ -162,17 +162,18 @@ class UnshardedBoundedTopK(TwoStageTiling):
             scratch, values = self.scratchpad, self.values
             dtype = _native.SS_DTYPE_BF16
 
-        # ss_topk_args, field by field in declaration order (TOPK_ARGS.fields names them)
-        packed = TOPK_ARGS.pack(
-            flat.data_ptr(), flat.stride(0), dtype, n_rows, flat.size(-1), self.k, block_n, 0,
-            scratch.data_ptr(), scratch.stride(0), values.data_ptr(), self.indices.data_ptr(),
-            _native.stream_of(flat),
-        )
+        # ss_topk_args in declaration order (TOPK_CALL.fields names the positions)
+        packed = TOPK_CALL.gather(flat, dtype, n_rows, self.vocabulary.size, self.k, block_n, 0, scratch, values,
+                                  self.indices, _native.stream_of(flat))
 
         _native.check(_native.packed_entry("ss_topk")(packed), "ss_topk")
 
-        k = self.k
-        dense_values = values.view(-1)[: n_rows * k].view(n_rows, k)
-        dense_indices = self.indices.view(-1)[: n_rows * k].view(n_rows, k)
+        # the first rows * k entries of the buffers, dense in the logits' leading shape
+        shape, strides, step = [*batch_step, self.k], [1], self.k
 
-        return dense_values.unflatten(0, batch_step), dense_indices.unflatten(0, batch_step)
+        for size in reversed(batch_step):
+
+            strides.insert(0, step)
+            step *= size
+
+        return values.as_strided(shape, strides), self.indices.as_strided(shape, strides)

@@ -1,0 +1,75 @@
+"""The host extension's packing, allocation and entry calls (CPU): each refuses what does not fit."""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from sonic_sampler import _native
+
+
+class Example(ctypes.Structure):
+    _fields_ = [("count", ctypes.c_int32), ("mask", ctypes.c_uint32), ("plane", ctypes.c_void_p),
+                ("stride_plane", ctypes.c_int64), ("stride_step", ctypes.c_int64), ("seed", ctypes.c_uint64),
+                ("row", ctypes.c_void_p), ("stride_row", ctypes.c_int64), ("one", ctypes.c_void_p)]
+
+
+def gatherer():
+
+    return _native.Gatherer(Example, dict(plane="u", row="S", one="t"), labels=dict(plane="the plane"))
+
+
+@pytest.mark.parametrize("plane", [torch.zeros(3, 4, 5), torch.zeros(3, 5), torch.zeros(6, 4, 5)[::2, 1:], None])
+def test_gathers_addresses_strides_and_scalars(plane):
+
+    row = torch.zeros(7, 9).T
+    g = gatherer()
+    assert g.fields == ("count", "mask", "plane", "seed", "row", "one")
+    got = Example.from_buffer_copy(g.gather(np.int64(-5), np.uint32(2 ** 32 - 1), plane, 2 ** 64 - 1, row, None))
+    assert (got.count, got.mask, got.seed, got.one) == (-5, 2 ** 32 - 1, 2 ** 64 - 1, None)
+    assert (got.row, got.stride_row) == (row.data_ptr(), 1)
+    want = (None, 0, 0) if plane is None else (plane.data_ptr(), plane.stride(0), plane.stride(1) if plane.dim() == 3 else 0)
+    assert (got.plane, got.stride_plane, got.stride_step) == want
+
+
+@pytest.mark.parametrize("args,error,text", [
+    ((2 ** 31, 0, None, 0, None, None), OverflowError, "count"),
+    ((0, 2 ** 32, None, 0, None, None), OverflowError, "mask"),
+    ((0, -1, None, 0, None, None), OverflowError, "negative"),
+    ((0, 0, None, 0.5, None, None), TypeError, "integer"),
+    ((0, 0, torch.zeros(4, 4).T, 0, None, None), ValueError, "`the plane` must be contiguous"),
+    ((0, 0, None, 0, None, torch.zeros(8)[::2]), ValueError, "`one` must be contiguous"),
+    ((0, 0, 7, 0, None, None), TypeError, "plane"),
+    ((0, 0, None, 0, None), TypeError, "arguments"),
+])
+def test_refuses_what_does_not_fit(args, error, text):
+
+    with pytest.raises(error, match=text):
+
+        gatherer().gather(*args)
+
+
+def test_empty_is_torch_empty():
+
+    t = _native.empty(torch.device("cpu"), torch.bfloat16, 3, 0, 2)
+    assert t.shape == (3, 0, 2) and t.dtype == torch.bfloat16 and t.device.type == "cpu" and not t.requires_grad
+
+    with pytest.raises(RuntimeError):
+
+        _native.empty(torch.device("cpu"), torch.int32, -3)
+
+    with pytest.raises(TypeError):
+
+        _native.host().empty("cpu", torch.int32, 3)
+
+
+def test_entries_take_bytes_only():
+
+    call = _native.packed_entry("ss_topk")
+
+    with pytest.raises(TypeError):
+
+        call(None)
+
+    assert call(bytes(ctypes.sizeof(_native.TopKArgs))) == 1  # no logits
