@@ -76,7 +76,13 @@ __global__ __launch_bounds__(SS_BLOCK) void singular_tiles_kernel(const uint16_t
     const int slot = p_slots ? uniform_i32(p_slots, row) : row;
     const uint32_t ind = uniform_u16(p_ind, slot);
     RowState rs = singular_row_state(a, row, slot, ind);
-    const Uses u = row_uses(rs);
+    const Uses whole = row_uses(rs);
+    // below 2048 columns the survivors' count lines are as many as the columns'
+    constexpr bool DEFER = (MODE & MODE_GATHER) && E >= 8;
+    const int valid = min(a.block_n, a.vocab_size - tile * a.block_n);
+    const bool defer = DEFER && valid >= SS_K && counts_can_wait(rs, whole);
+    Uses u = whole;
+    if (defer) u.remap = rs.d2t != nullptr && u.bias;
     if ((MODE & MODE_GATHER) && stage_words > 0 && u.g && u.remap) {
         stage_grammar(rs.grammar, rs.vt, grammar_words);
         rs.glds = grammar_words;
@@ -105,9 +111,22 @@ __global__ __launch_bounds__(SS_BLOCK) void singular_tiles_kernel(const uint16_t
     // this shard's slice of the row's [world_size, tiles, 128] lists
     uint32_t *scr = computed_here(a.scratch + (int64_t)row * a.stride_scratch +
                                   (a.world_size > 1 ? a.local_rank * tiles * SS_K : 0));
+    const int col0 = tile * a.block_n;
+    const bool greedy = (ind & IND_GREEDY) != 0;
     Keys<E> keys;
-    prologue_keys<E, MODE, PRE>(rs, tile * a.block_n, a.vocab_size, exc, cap, lw, keys, pre);
-    tile_stage<E>(sm, (ind & IND_GREEDY) != 0, keys, scr, tile, min(a.block_n, a.vocab_size - tile * a.block_n));
+    if constexpr (DEFER) {
+        if (defer && threadIdx.x == 0)
+            sm.defer = DeferState{(uint64_t)(uintptr_t)rs.logits, (uint64_t)(uintptr_t)rs.d2t, (uint64_t)(uintptr_t)rs.dec,
+                                  (uint64_t)(uintptr_t)rs.ctx, (uint64_t)(uintptr_t)rs.bias, rs.rep, rs.freq, rs.pres,
+                                  rs.temp, rs.ind, rs.vt, rs.shard, col0, a.vocab_size, 0};
+        const DeferredCounts counts{defer, &sm.defer, rs.hist};
+        if (defer) rs.ind &= ~(IND_MULT | IND_FREQ | IND_PRES);
+        prologue_keys<E, MODE, PRE>(rs, col0, a.vocab_size, exc, cap, lw, keys, pre);
+        tile_stage<E, false>(sm, greedy, keys, scr, tile, valid, SS_K, counts);
+    } else {
+        prologue_keys<E, MODE, PRE>(rs, col0, a.vocab_size, exc, cap, lw, keys, pre);
+        tile_stage<E>(sm, greedy, keys, scr, tile, valid);
+    }
 }
 
 // Greedy row (wave 0): the argmax over the tiles' maxima, d2t remap, count update, outputs.

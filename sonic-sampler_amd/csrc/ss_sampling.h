@@ -8,6 +8,8 @@
 //   * top-k / top-p / min-p truncation in the reference's order (core/naive.py:270-328).
 #pragma once
 
+#include <type_traits>
+
 #include "ss_philox.h"
 #include "ss_select.h"
 
@@ -36,6 +38,16 @@ struct SampleSmem {
     float qcand[SS_K];         // verification: their draft probabilities
 };
 
+// Request state of a row whose penalties wait for the selection (DeferredCounts), kept in workgroup
+// memory: in scalar registers across the whole selection it spilled them for every row.
+struct DeferState {
+    uint64_t logits, d2t, dec, ctx, bias;
+    float rep, freq, pres, temp;
+    uint32_t ind;
+    int32_t vt, shard, col0, V, pad;
+};
+static_assert(sizeof(DeferState) == 80, "whole 16-byte blocks");
+
 // Workgroup memory of the tile kernels (E keys per thread). The members from `run` on are written
 // only after the tile stage's first barrier, when every wave has finished its prologue, so a
 // grammar row staged for the prologue (stage_grammar) may overlay them (TILE_OVERLAY).
@@ -44,6 +56,8 @@ struct TileSmem {
     uint32_t scan[SS_WAVES * 16];  // workgroup scans of up to 16 values per thread
     uint32_t red[SS_WAVES];
     uint32_t cnt[SS_WAVES];       // survivors of each wave
+    uint32_t kept[SS_WAVES];      // of them, those still at the bound after deferred counts
+    DeferState defer;
     uint32_t run[SS_WAVES][SS_K + 64];  // each wave's survivors, then its sorted run
     uint32_t run2[2][SS_K];       // merge tree: the top-128 of runs (0, 1) and (2, 3)
     // each wave's packed keys, pair i of lane l at [i * 64 + l], read back by the survivors of
@@ -52,7 +66,7 @@ struct TileSmem {
 };
 
 // Byte offset in TileSmem where a staged grammar row may begin.
-constexpr int TILE_OVERLAY = (SS_WAVES * 16 + 2 * SS_WAVES) * 4;
+constexpr int TILE_OVERLAY = (SS_WAVES * 16 + 3 * SS_WAVES) * 4 + (int)sizeof(DeferState);
 static_assert(TILE_OVERLAY % 16 == 0, "16-byte grammar stores");
 static_assert(TILE_OVERLAY == __builtin_offsetof(TileSmem<16>, run), "overlay starts at the runs");
 
@@ -306,7 +320,7 @@ struct ExcList {
 };
 
 // Records of the list in the gather layout with a staged grammar row, which lies behind the row:
-// 40368 bytes of workgroup memory in all at 8192 grammar words, four workgroups a CU.
+// 40464 bytes of workgroup memory in all at 8192 grammar words, four workgroups a CU.
 constexpr uint32_t EXC_STAGED_CAP = 38;
 
 // Keys of the E / 4 chunks of one pass from their (grammar-masked) logits, decode counts, context
@@ -1089,6 +1103,119 @@ __device__ __forceinline__ uint32_t wave_survivors_masked(TileSmem<E> &sm, const
     return total;
 }
 
+// Penalties that only lower logits (a repetition penalty of at least 1, frequency and presence
+// penalties of at least 0, on counts that are histograms) can wait for the selection: with r the
+// element's value without them and p with them, p <= r (every processor and every rounding is
+// monotone), so of the elements with r >= lo, of which at least 128 keep p >= lo, the top 128 by p
+// are the tile's. Through d2t, where a count costs a cache line a column and plane (a heavy tile is
+// bound by what its CU takes from L2), the count planes are then read at the survivors
+// only: drafting for mixed requests, 32000 -> 128256 ids, 64 rows 31.6 -> 19.1 us, 256 rows
+// 124 -> 36.5. With counts on a third of all ids most tiles start again (64 rows 33.7 us against
+// 31.1); on 5% none do (16.7 against 31.2). In the direct layout, whose counts come in whole
+// lines, the deferral measured 168 -> 145 us at 1280 penalized verification rows, but its code cost
+// rows without penalties 3-5% (303 rows 28.8 -> 30.1) and dense counts 30%: not taken there.
+constexpr int DEFER_WANT = 160;  // candidates asked of the bound: at least 32 may fall below it
+
+struct NoCounts {
+    static constexpr bool on = false;
+};
+
+struct DeferredCounts {
+    bool on;
+    const DeferState *state;  // valid after the selection's first barrier
+    int hist;                 // RowState::hist
+
+    // `state` in scalar registers.
+    __device__ __forceinline__ RowState row(int &col0, int &V) const {
+        auto word = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
+        auto pointer = [&](uint64_t v) { return ((uint64_t)word((uint32_t)(v >> 32)) << 32) | word((uint32_t)v); };
+        auto real = [&](float v) { return __uint_as_float(word(__float_as_uint(v))); };
+        const DeferState s = *state;
+        RowState rs;
+        rs.ind = word(s.ind);
+        rs.logits = (const uint16_t *)pointer(s.logits);
+        rs.d2t = (const int32_t *)pointer(s.d2t);
+        rs.dec = (const int32_t *)pointer(s.dec);
+        rs.ctx = (const int32_t *)pointer(s.ctx);
+        rs.bias = (const uint16_t *)pointer(s.bias);
+        rs.grammar = nullptr;
+        rs.glds = nullptr;
+        rs.rep = real(s.rep);
+        rs.freq = real(s.freq);
+        rs.pres = real(s.pres);
+        rs.temp = real(s.temp);
+        rs.vt = (int)word((uint32_t)s.vt);
+        rs.shard = (int)word((uint32_t)s.shard);
+        rs.hist = hist;
+        col0 = (int)word((uint32_t)s.col0);
+        V = (int)word((uint32_t)s.V);
+        return rs;
+    }
+
+    // keys of the N (1 or 4) consecutive columns from `col` on, in place; `in` false: none of them
+    template <int N>
+    __device__ __forceinline__ void lower(bool in, int col, uint32_t (&key)[N]) const {
+        int col0, V;
+        const RowState rs = row(col0, V);
+        const Uses u = row_uses(rs);
+        const __amdgpu_buffer_rsrc_t db = row_buffer(rs.dec, (int64_t)rs.vt * 4);
+        const __amdgpu_buffer_rsrc_t cb = row_buffer(u.mult ? rs.ctx : nullptr, u.mult ? (int64_t)rs.vt * 4 : 0);
+        int t[N], dec[N], ctx[N], any = 0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            t[i] = rs.shard + col0 + col + i;
+            if (rs.d2t)
+                t[i] = __builtin_amdgcn_raw_buffer_load_b32(row_buffer(rs.d2t, (int64_t)(rs.shard + V) * 4), t[i] * 4, 0, 0);
+        }
+        const __amdgpu_buffer_rsrc_t lg = row_buffer(rs.logits, (int64_t)V * 2);
+        const __amdgpu_buffer_rsrc_t bb = row_buffer(u.bias ? rs.bias : nullptr, u.bias ? (int64_t)rs.vt * 2 : 0);
+        uint32_t x[N], b[N];
+        auto load_values = [&]() {
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                x[i] = __builtin_amdgcn_raw_buffer_load_b16(lg, (col0 + col + i) * 2, 0, 0);
+                b[i] = __builtin_amdgcn_raw_buffer_load_b16(bb, t[i] * 2, 0, 0);
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            dec[i] = __builtin_amdgcn_raw_buffer_load_b32(db, t[i] * 4, 0, 0);
+            ctx[i] = __builtin_amdgcn_raw_buffer_load_b32(cb, t[i] * 4, 0, 0);
+        }
+        // whole chunks: the logits and biases in the same round of loads; single survivors, of
+        // which few have a count: only where one has
+        if constexpr (N == 4) load_values();
+        // the history never counts token 0 (core/naive.py:179-203)
+        for (uint64_t m = __ballot(rs.hist != 0); m; m &= m - 1) {
+            const int token = __builtin_amdgcn_readlane(rs.hist, __builtin_ctzll(m));
+#pragma unroll
+            for (int i = 0; i < N; ++i) dec[i] += t[i] == token ? 1 : 0;
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) any |= dec[i] | ctx[i];
+        if (in && any != 0) {
+            if constexpr (N != 4) load_values();
+            bool all_exc;
+            const FastChain f = fast_chain(row_chain(rs, u, all_exc));
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const uint32_t low = key_of(chain_fast(f, bf2f(x[i]), dec[i], ctx[i], bf2f(b[i])));
+                if ((dec[i] | ctx[i]) != 0 && key[i] != 0) key[i] = low;  // key 0: past the vocabulary
+            }
+        }
+    }
+};
+
+// Whether the penalties of a row can wait (DeferredCounts). A row under a grammar keeps the whole
+// chain: a tile that admits fewer than 128 tokens has no bound to hold them to.
+__device__ __forceinline__ bool counts_can_wait(const RowState &rs, const Uses &u) {
+    if (!u.rep || u.g || (rs.ind & IND_GREEDY)) return false;
+    bool all_exc;
+    const Chain k = row_chain(rs, u, all_exc);
+    return (!k.mult || (k.rdiv.fast && k.rep >= 1.0f)) && (!k.freq || (k.fr >= 0.0f && !all_exc)) &&
+           (!k.pres || k.pr >= 0.0f) && (!k.temp || (k.tdiv.fast && k.tdiv.d > 0.0f));
+}
+
 // The wave's share of a tile's `want` candidates, in proportion to the columns it holds of the
 // tile's `valid` (rounded up, so the shares add up to at least `want`): want / 4 in a full tile.
 // A row's partial last tile fills its first waves first; with the full tile's share a wave of few
@@ -1101,6 +1228,16 @@ __device__ __forceinline__ int wave_share(int want, int valid, int wave) {
     const int rest = valid & (SS_BLOCK * 4 - 1);
     const int n = (valid >> 10) * 256 + min(max(rest - 256 * wave, 0), 256);
     return (want * n + valid - 1) / valid;
+}
+
+// The lane's keys from its spill. By recursion: as a loop in the retry's cycle the compiler left it
+// rolled, with the key registers indexed at run time.
+template <int E, int I = 0>
+__device__ __forceinline__ void reload_keys(const uint32_t *spill, Keys<E> &keys) {
+    if constexpr (I < E / 2) {
+        keys.p[I] = spill[I * 64];
+        reload_keys<E, I + 1>(spill, keys);
+    }
 }
 
 // Tile stage. Greedy rows store one u32 per tile: (key << 16) | (0xffff - column offset), whose
@@ -1124,9 +1261,17 @@ __device__ __forceinline__ int wave_share(int want, int valid, int wave) {
 //
 // TOPK (the bounded top-k): only the first k <= 128 of the tile's list are stored, at
 // scratch[tile * k ...].
-template <int E, bool TOPK = false>
-__device__ __forceinline__ void tile_stage(TileSmem<E> &sm, bool greedy, const Keys<E> &keys,
-                                           uint32_t *scr, int tile, int valid, int k = SS_K) {
+//
+// With deferred counts (`counts`, on a tile of at least 128 valid columns) every wave lowers its
+// survivors' keys before it sorts them. When fewer than 128 of the tile's stay at the bound, or the
+// survivors do not fit, the waves lower all of their spilled keys, chunk by chunk, and the
+// selection starts again from those.
+template <int E, bool TOPK = false, class Counts = NoCounts>
+__device__ __forceinline__ void tile_stage(TileSmem<E> &sm, bool greedy, Keys<E> &keys,
+                                           uint32_t *scr, int tile, int valid, int k = SS_K,
+                                           const Counts &counts = Counts{}) {
+    constexpr bool DEFER = !std::is_same_v<Counts, NoCounts>;
+    bool deferred = counts.on;
     const int lane = lane_id();
     const int wave = (int)threadIdx.x >> 6;
     if (greedy) {
@@ -1147,8 +1292,9 @@ __device__ __forceinline__ void tile_stage(TileSmem<E> &sm, bool greedy, const K
         return;
     }
     typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+select:
     // keys the wave's bound must leave: its share of the list's length by its valid columns
-    const int want = TOPK ? k : SS_K;
+    const int want = TOPK ? k : deferred ? DEFER_WANT : SS_K;
     const int need = wave_share<E>(want, valid, __builtin_amdgcn_readfirstlane(wave));
     uint32_t bound = 0;
     if (valid <= SS_BLOCK * 4 && valid < SS_BLOCK * E) {
@@ -1212,6 +1358,23 @@ __device__ __forceinline__ void tile_stage(TileSmem<E> &sm, bool greedy, const K
     const bool floored = lo == KEY_NEG_INF + 1;
     uint32_t T = lo ? lo - 1 : 0u;  // key 0 (absent) never survives
     const uint32_t cnt = wave_survivors_masked<E>(sm, keys, T);
+    if constexpr (DEFER) {
+        if (deferred && cnt <= (uint32_t)SS_K) {
+            uint32_t *run = sm.run[wave];
+            uint32_t kept = 0;
+#pragma unroll 1
+            for (uint32_t i0 = 0; i0 < cnt; i0 += 64) {
+                const uint32_t i = i0 + (uint32_t)lane;
+                const bool mine = i < cnt;
+                const uint32_t c = mine ? run[i] : 0xffffu;
+                uint32_t key[1] = {c >> 16};
+                counts.template lower<1>(mine, (int)(0xffffu - (c & 0xffffu)), key);
+                kept += (uint32_t)__popcll(__ballot(mine && key[0] > T));
+                if (mine) run[i] = (key[0] << 16) | (c & 0xffffu);
+            }
+            if (lane == 0) sm.kept[wave] = kept;
+        }
+    }
     if (cnt <= 64) {
         uint32_t *run = sm.run[wave];
         uint32_t v = lane < (int)cnt ? run[lane] : 0u;
@@ -1230,6 +1393,27 @@ __device__ __forceinline__ void tile_stage(TileSmem<E> &sm, bool greedy, const K
     __syncthreads();
     const uint32_t n0 = sm.cnt[0], n1 = sm.cnt[1], n2 = sm.cnt[2], n3 = sm.cnt[3];
     bool exact = max(max(n0, n1), max(n2, n3)) > (uint32_t)SS_K;
+    if constexpr (DEFER) {
+        const uint32_t kept = sm.kept[0] + sm.kept[1] + sm.kept[2] + sm.kept[3];
+        // the answer in a scalar register, so that the retry is a uniform branch: as a divergent one
+        // it made every step of the selection's first round a masked one (404 scalar instructions a
+        // wave -> 529 at 16384 columns)
+        if (__builtin_amdgcn_readfirstlane(deferred && (exact || floored || kept < (uint32_t)SS_K))) {
+            __syncthreads();  // every wave has read the counts
+            uint32_t *spill = sm.keys[wave] + lane;
+#pragma unroll 1
+            for (int c = 0; c < E / 4; ++c) {
+                const uint32_t w0 = spill[2 * c * 64], w1 = spill[(2 * c + 1) * 64];
+                uint32_t key[4] = {w0 & 0xffffu, w0 >> 16, w1 & 0xffffu, w1 >> 16};
+                counts.template lower<4>(true, c * (SS_BLOCK * 4) + 4 * (int)threadIdx.x, key);
+                spill[2 * c * 64] = key[0] | (key[1] << 16);
+                spill[(2 * c + 1) * 64] = key[2] | (key[3] << 16);
+            }
+            reload_keys<E>(spill, keys);
+            deferred = false;
+            goto select;
+        }
+    }
     // Fewer than 128 survivors, all of the keys above -inf: the tile's first 128 are those and
     // then its first 128 - survivors -inf keys in column order. When the tile's first 256 columns
     // (wave 0's elements 0-3, whose keys the survivor pass spilled) hold that many, wave 0 appends

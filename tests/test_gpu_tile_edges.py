@@ -155,3 +155,38 @@ def test_count_and_bias_density(block, vocab, density, monkeypatch):
     sweep.test_sweep_multistep_row_top128(block, vocab, "random", "spiked", seed)
     sweep.test_sweep_drafting_d2t(block, vocab, "sparse", "spiked", seed)
     sweep.test_sweep_drafting_d2t(block, vocab, "random", "few", seed + 1)
+
+
+@pytest.mark.parametrize("density", [0.002, 0.05, 0.3, 1.0])
+@pytest.mark.parametrize("block,vocab", [(2048, 8193), (4096, 9000), (8192, 33000), (16384, 40002)])
+def test_drafting_with_penalties_that_only_lower(block, vocab, density, monkeypatch):
+    """Drafting rows whose penalties only lower logits read their counts at the selection's survivors,
+    and start the selection again where too many of those fall below its bound (dense counts, tied
+    values): against the oracle, with rows at the neutral ends of the ranges and drafted history."""
+
+    import test_gpu_sweep as sweep
+
+    whole = sweep.random_host
+
+    def lowering(slots, timesteps, vocab, seed, indicator=None, **kw):
+
+        host = whole(slots, timesteps, vocab, seed, indicator & ~0x1, **kw)  # no grammar
+        g = torch.Generator().manual_seed(seed)
+        rep = host.repetition
+
+        for plane in (rep.counts.context, rep.counts.decode):
+
+            plane.masked_fill_(torch.rand(plane.shape, generator=g) >= density, 0)
+
+        rep.multiplicative.copy_(1 + (rep.multiplicative - 1).abs())
+        rep.frequency.abs_()
+        rep.presence.abs_()
+        rep.multiplicative[0], rep.frequency[1], rep.presence[2] = 1.0, 0.0, 0.0
+        rep.multiplicative[3], rep.frequency[4] = 0.9, -0.5  # these rows cannot wait
+
+        return host
+
+    monkeypatch.setattr(sweep, "random_host", lowering)
+    seed = 6000 + block + int(1000 * density)
+    sweep.test_sweep_drafting_d2t(block, vocab, "random", "spiked", seed)
+    sweep.test_sweep_drafting_d2t(block, vocab, "random", "few", seed + 1)
