@@ -197,7 +197,7 @@ __device__ __forceinline__ float div_bf16(float x, const Divisor &v) {
 // Order-preserving 16-bit key (key16) of a bf16-exact float: 0x8000 plus the signed magnitude
 // of its top 16 bits (negation by xor with the sign mask and subtraction of it).
 // Key of bf16 -inf (key_of and packed_keys): every finite or +inf value has a larger one.
-constexpr uint32_t KEY_NEG_INF = 0x0080;
+constexpr uint32_t KEY_NEG_INF = 0x0080, KEY_POS_INF = 0xff80;
 
 __device__ __forceinline__ uint32_t key_of(float x) {
     const uint32_t u = __float_as_uint(x);
@@ -1240,6 +1240,40 @@ __device__ __forceinline__ void reload_keys(const uint32_t *spill, Keys<E> &keys
     }
 }
 
+// The lane's largest key.
+template <int E>
+__device__ __forceinline__ uint32_t lane_maximum(const Keys<E> &keys) {
+    u2v a1 = {0, 0};
+#pragma unroll
+    for (int i = 0; i < E / 2; ++i) a1 = __builtin_elementwise_max(a1, __builtin_bit_cast(u2v, keys.p[i]));
+    return max((uint32_t)a1.x, (uint32_t)a1.y);
+}
+
+// The lane's largest and second-largest key: the two largest of its even and of its odd elements
+// with packed 16-bit max / min, then the two largest of those four.
+template <int E>
+__device__ __forceinline__ void lane_maxima(const Keys<E> &keys, uint32_t &m1, uint32_t &m2) {
+    u2v a1 = {0, 0}, a2 = {0, 0};
+#pragma unroll
+    for (int i = 0; i < E / 2; ++i) {
+        const u2v v = __builtin_bit_cast(u2v, keys.p[i]);
+        a2 = __builtin_elementwise_max(a2, __builtin_elementwise_min(a1, v));
+        a1 = __builtin_elementwise_max(a1, v);
+    }
+    m1 = max((uint32_t)a1.x, (uint32_t)a1.y);
+    m2 = max(min((uint32_t)a1.x, (uint32_t)a1.y), max((uint32_t)a2.x, (uint32_t)a2.y));
+}
+
+// Puts NaN behind -inf (the key of a negative NaN), where the bounded top-k has it.
+template <int E>
+__device__ __forceinline__ void nan_last(Keys<E> &keys) {
+#pragma unroll
+    for (int i = 0; i < E / 2; ++i) {
+        const uint32_t w = keys.p[i], a = w & 0xffffu, b = w >> 16;
+        keys.p[i] = (a > KEY_POS_INF ? 0x40u : a) | ((b > KEY_POS_INF ? 0x40u : b) << 16);
+    }
+}
+
 // Tile stage. Greedy rows store one u32 per tile: (key << 16) | (0xffff - column offset), whose
 // maximum picks the lowest column among equal maxima. Other rows store their exact top-128 as the
 // same composites, sorted in descending order (0 for absent entries), at scratch[tile * 128 ...].
@@ -1260,7 +1294,8 @@ __device__ __forceinline__ void reload_keys(const uint32_t *spill, Keys<E> &keys
 // can exceed 128.
 //
 // TOPK (the bounded top-k): only the first k <= 128 of the tile's list are stored, at
-// scratch[tile * k ...].
+// scratch[tile * k ...], and NaN stands behind -inf (a wave whose largest key is one reorders its
+// keys first); the fused kernels' rows keep the keys' order, NaN by its sign.
 //
 // With deferred counts (`counts`, on a tile of at least 128 valid columns) every wave lowers its
 // survivors' keys before it sorts them. When fewer than 128 of the tile's stay at the bound, or the
@@ -1291,13 +1326,14 @@ __device__ __forceinline__ void tile_stage(TileSmem<E> &sm, bool greedy, Keys<E>
         }
         return;
     }
-    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 select:
     // keys the wave's bound must leave: its share of the list's length by its valid columns
     const int want = TOPK ? k : deferred ? DEFER_WANT : SS_K;
     const int need = wave_share<E>(want, valid, __builtin_amdgcn_readfirstlane(wave));
     uint32_t bound = 0;
+    auto above_inf = [&](uint32_t key) { return TOPK && __builtin_expect(__ballot(key > KEY_POS_INF) != 0ull, 0); };
     if (valid <= SS_BLOCK * 4 && valid < SS_BLOCK * E) {
+        if (above_inf(max(max(keys.p[0] & 0xffffu, keys.p[0] >> 16), max(keys.p[1] & 0xffffu, keys.p[1] >> 16)))) nan_last<E>(keys);
         // One partly filled chunk: the lane's four keys are all it holds, and a wave may hold most
         // of the tile's columns, so that its share exceeds what its lanes' largest keys can bound
         // (and all 16 key bits count: a share near 128 leaves a run of 128 no slack).
@@ -1312,29 +1348,26 @@ select:
         // At 64 elements a lane its largest key alone bounds well: the bound is the largest t (to
         // 14 of the 16 key bits) that at least `need` lane maxima reach, so the wave holds at least
         // `need` keys >= t. One packed max a pair, one ballot a bisection step.
-        u16x2 a1 = {0, 0};
-#pragma unroll
-        for (int i = 0; i < E / 2; ++i) a1 = __builtin_elementwise_max(a1, __builtin_bit_cast(u16x2, keys.p[i]));
-        const uint32_t m1 = max((uint32_t)a1.x, (uint32_t)a1.y);
+        uint32_t m1 = lane_maximum<E>(keys);
+        if (above_inf(m1)) {
+            nan_last<E>(keys);
+            m1 = lane_maximum<E>(keys);
+        }
 #pragma unroll
         for (int b = 15; b >= 2; --b) {
             const uint32_t c = bound | (1u << b);
             if ((int)__popcll(__ballot(m1 >= c)) >= need) bound = c;
         }
     } else {
-        // The lane's largest and second-largest key: the two largest of its even and of its odd
-        // elements with packed 16-bit max / min, then the two largest of those four. With few
-        // elements a lane (and on the partial last tile of a row) the second-largest keeps the
-        // bound tight enough that the survivors fit a wave's run.
-        u16x2 a1 = {0, 0}, a2 = {0, 0};
-#pragma unroll
-        for (int i = 0; i < E / 2; ++i) {
-            const u16x2 v = __builtin_bit_cast(u16x2, keys.p[i]);
-            a2 = __builtin_elementwise_max(a2, __builtin_elementwise_min(a1, v));
-            a1 = __builtin_elementwise_max(a1, v);
+        // The lane's largest and second-largest key. With few elements a lane (and on the partial
+        // last tile of a row) the second-largest keeps the bound tight enough that the survivors
+        // fit a wave's run.
+        uint32_t m1, m2;
+        lane_maxima<E>(keys, m1, m2);
+        if (above_inf(m1)) {
+            nan_last<E>(keys);
+            lane_maxima<E>(keys, m1, m2);
         }
-        const uint32_t m1 = max((uint32_t)a1.x, (uint32_t)a1.y);
-        const uint32_t m2 = max(min((uint32_t)a1.x, (uint32_t)a1.y), max((uint32_t)a2.x, (uint32_t)a2.y));
         // 14 of the 16 key bits: the bound may sit up to 3 keys low, which only adds a few survivors
 #pragma unroll
         for (int b = 15; b >= 2; --b) {

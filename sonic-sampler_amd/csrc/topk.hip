@@ -351,6 +351,12 @@ __device__ __forceinline__ uint32_t float_key(float v) {
     return u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
 }
 
+constexpr uint32_t KEY32_NEG_INF = 0x007fffffu;
+
+// NaN of either sign as the negative one, whose key stands behind -inf (as in the bfloat16 tile
+// stage, nan_last) and above the key 0 of absent elements.
+__device__ __forceinline__ float negative_nan(float v) { return v != v ? __uint_as_float(0xffc00000u) : v; }
+
 template <int E>
 __global__ __launch_bounds__(SS_BLOCK) void topk_block_kernel(const void *p_logits, int64_t p_stride,
                                                               int p_block_n, int p_vocab, int p_k, int tiles,
@@ -390,7 +396,7 @@ __global__ __launch_bounds__(SS_BLOCK) void topk_block_kernel(const void *p_logi
     float m = v[0];
 #pragma unroll
     for (int j = 1; j < E; ++j) m = fmaxf(m, v[j]);
-    uint32_t mk = float_key(m);
+    uint32_t mk = float_key(negative_nan(m));  // NaN where the lane holds nothing else
     wave_sort64_desc(mk);
     // The wave's share of k is proportional to the valid columns it holds (chunk c gives it
     // columns c * 1024 + 256 * wave .. + 255), so a partial last tile, whose columns sit in its
@@ -405,7 +411,7 @@ __global__ __launch_bounds__(SS_BLOCK) void topk_block_kernel(const void *p_logi
     if (need > 0 && need <= 64 && lane == need - 1) sm.red[wave] = mk;
     __syncthreads();
     const uint32_t lo = min(min(sm.red[0], sm.red[1]), min(sm.red[2], sm.red[3]));
-    const bool no_bound = lo == 0u;
+    const bool no_bound = lo < KEY32_NEG_INF;  // no share, or a lane of NaN alone among it
     // the float whose key is lo (lo is the key of a lane maximum, so it is a value of the row)
     const float lo_f = __uint_as_float((lo & 0x80000000u) ? (lo & 0x7fffffffu) : ~lo);
     __syncthreads();
@@ -478,6 +484,8 @@ __global__ __launch_bounds__(SS_BLOCK) void topk_block_kernel(const void *p_logi
     }
 
     // ---- exact selection over the whole block (ties at the k-th value kept in column order) -------
+#pragma unroll
+    for (int j = 0; j < E; ++j) v[j] = negative_nan(v[j]);
     auto keys_of = [&](int, uint32_t(&out)[E]) {
 #pragma unroll
         for (int j = 0; j < E; ++j) out[j] = col_of(j) < V ? float_key(v[j]) : 0u;
@@ -601,7 +609,7 @@ __global__ __launch_bounds__(TOPK_WIDE_THREADS) void topk_wide_kernel(const void
     float m = v[0];
 #pragma unroll
     for (int j = 1; j < E; ++j) m = fmaxf(m, v[j]);
-    uint32_t mk = float_key(m);
+    uint32_t mk = float_key(negative_nan(m));  // NaN where the lane holds nothing else
     wave_sort64_desc(mk);
     int nw = 0;  // columns of the row this wave holds (256 of every chunk)
 #pragma unroll
@@ -614,7 +622,7 @@ __global__ __launch_bounds__(TOPK_WIDE_THREADS) void topk_wide_kernel(const void
     uint32_t lo = 0xffffffffu;
 #pragma unroll
     for (int w = 0; w < TOPK_WIDE_WAVES; ++w) lo = min(lo, sm.red[w]);
-    const bool no_bound = lo == 0u;
+    const bool no_bound = lo < KEY32_NEG_INF;  // no share, or a lane of NaN alone among it
     const float lo_f = __uint_as_float((lo & 0x80000000u) ? (lo & 0x7fffffffu) : ~lo);
     __syncthreads();
 
@@ -680,7 +688,10 @@ __global__ __launch_bounds__(TOPK_WIDE_THREADS) void topk_wide_kernel(const void
     __syncthreads();
     uint32_t key[E];
 #pragma unroll
-    for (int j = 0; j < E; ++j) key[j] = col_of(j) < V ? float_key(v[j]) : 0u;
+    for (int j = 0; j < E; ++j) {
+        v[j] = negative_nan(v[j]);
+        key[j] = col_of(j) < V ? float_key(v[j]) : 0u;
+    }
     uint32_t T = 0;  // the largest t with at least k keys >= t
 #pragma unroll 1
     for (int b = 31; b >= 0; --b) {

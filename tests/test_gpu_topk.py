@@ -263,3 +263,44 @@ def test_more_than_512_tiles(k):
     logits = spiked_logits(3, 600_000, seed=600 + k)
     print(f"top-k over 586 tiles, k={k}", flush=True)
     check(logits, k, block_size=1024)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("values", ["spread", "tied"])
+@pytest.mark.parametrize("rows", [5, 47, 48, 260])
+def test_nan_stands_behind_every_number(rows, values, dtype):
+    """NaN of either sign is no candidate of a row with k numbers, whichever launch form the row
+    count selects and whether the survivors fit their lists or an exact cut runs (ties)."""
+
+    from sonic_sampler.interface import UnshardedBoundedTopK
+
+    vocab = 20001
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, vocab, generator=g) * 3
+
+    if values == "tied":
+
+        x = torch.randint(-2, 3, (rows, vocab), generator=g).float()
+
+    x = x.to(dtype)
+    nan = torch.rand(rows, vocab, generator=g) < torch.tensor([0.001, 0.05, 0.5])[torch.arange(rows) % 3, None]
+    # whole lanes, wherever a block of columns starts: four columns of every chunk; and the last columns
+    nan[1::2] |= torch.arange(vocab) % 1024 < 16
+    nan[:, -3:] = True
+    want = {k: oracle_topk(x.masked_fill(nan, -float("inf")), k) for k in (1, 32, 128)}
+    # by their bits (a conversion from float32 makes them all one): both signs, any payload
+    bits = torch.randint(1, 0x80, (rows, vocab), generator=g) | 0x7f80 | torch.randint(0, 2, (rows, vocab), generator=g) << 15
+    bits = (bits - (bits >= 0x8000) * 0x10000).to(torch.int16)
+    bits = bits if dtype == torch.bfloat16 else bits.to(torch.int32) << 16
+    x = torch.where(nan, bits, x.view(bits.dtype)).view(dtype)
+    assert torch.equal(x.isnan(), nan)
+
+    for k in (1, 32, 128):
+
+        for block in (1024, 4096, 16384):
+
+            print(f"rows {rows} {values} {dtype} k {k} block {block}", flush=True)
+            topk = UnshardedBoundedTopK.initialize(vocab_size=vocab, batch_size=rows, k=k, block_size=block, device=DEV)
+            got_values, got = topk(x.to(DEV))
+            assert torch.equal(got.cpu(), want[k][1])
+            assert torch.equal(got_values.cpu(), want[k][0])
