@@ -76,13 +76,11 @@ __global__ __launch_bounds__(SS_BLOCK) void singular_tiles_kernel(const uint16_t
     const int slot = p_slots ? uniform_i32(p_slots, row) : row;
     const uint32_t ind = uniform_u16(p_ind, slot);
     RowState rs = singular_row_state(a, row, slot, ind);
-    const Uses whole = row_uses(rs);
+    const Uses u = row_uses(rs);
     // below 2048 columns the survivors' count lines are as many as the columns'
     constexpr bool DEFER = (MODE & MODE_GATHER) && E >= 8;
     const int valid = min(a.block_n, a.vocab_size - tile * a.block_n);
-    const bool defer = DEFER && valid >= SS_K && counts_can_wait(rs, whole);
-    Uses u = whole;
-    if (defer) u.remap = rs.d2t != nullptr && u.bias;
+    const bool may_defer = DEFER && valid >= SS_K && counts_may_wait(rs, u);
     if ((MODE & MODE_GATHER) && stage_words > 0 && u.g && u.remap) {
         stage_grammar(rs.grammar, rs.vt, grammar_words);
         rs.glds = grammar_words;
@@ -92,13 +90,23 @@ __global__ __launch_bounds__(SS_BLOCK) void singular_tiles_kernel(const uint16_t
     constexpr bool PRE = (MODE & MODE_GATHER) && E <= 32;
     int32_t pre[PRE ? E : 1];
     if constexpr (PRE) {
-        if (u.remap) load_d2t<E>(rs, tile * a.block_n, a.vocab_size, pre);
+        if (u.remap && !may_defer) load_d2t<E>(rs, tile * a.block_n, a.vocab_size, pre);
     }
     if (a.drafted_tokens && (ind & (IND_MULT | IND_FREQ | IND_PRES)) && lane_id() < a.timestep)
         rs.hist = a.drafted_tokens[(int64_t)row * a.stride_drafted + lane_id()];
     if (rs.glds) {
         stage_grammar_finish(rs.vt, grammar_words);
         __syncthreads();
+    }
+    // The row's parameters decide whether its penalties wait. Asked for ahead of the d2t targets, they
+    // held those back by a round trip on every row, and one tile selection for both kinds of rows cost
+    // those that never wait its retry: grammar rows 256 of 32000 -> 262144 ids 18.7 -> 19.4 us a call.
+    bool defer = false;
+    if (__builtin_expect(may_defer, 0)) {
+        defer = counts_can_wait(rs, u);
+        if constexpr (PRE) {
+            if (defer ? rs.d2t && u.bias : u.remap) load_d2t<E>(rs, tile * a.block_n, a.vocab_size, pre);
+        }
     }
     // the waves' exception lists: in the memory of their spilled keys, or behind a staged grammar
     // row, which overlays it
@@ -119,14 +127,16 @@ __global__ __launch_bounds__(SS_BLOCK) void singular_tiles_kernel(const uint16_t
             sm.defer = DeferState{(uint64_t)(uintptr_t)rs.logits, (uint64_t)(uintptr_t)rs.d2t, (uint64_t)(uintptr_t)rs.dec,
                                   (uint64_t)(uintptr_t)rs.ctx, (uint64_t)(uintptr_t)rs.bias, rs.rep, rs.freq, rs.pres,
                                   rs.temp, rs.ind, rs.vt, rs.shard, col0, a.vocab_size, 0};
-        const DeferredCounts counts{defer, &sm.defer, rs.hist};
         if (defer) rs.ind &= ~(IND_MULT | IND_FREQ | IND_PRES);
-        prologue_keys<E, MODE, PRE>(rs, col0, a.vocab_size, exc, cap, lw, keys, pre);
-        tile_stage<E, false>(sm, greedy, keys, scr, tile, valid, SS_K, counts);
-    } else {
-        prologue_keys<E, MODE, PRE>(rs, col0, a.vocab_size, exc, cap, lw, keys, pre);
-        tile_stage<E>(sm, greedy, keys, scr, tile, valid);
     }
+    prologue_keys<E, MODE, PRE>(rs, col0, a.vocab_size, exc, cap, lw, keys, pre);
+    if constexpr (DEFER) {
+        if (__builtin_expect(defer, 0)) {
+            tile_stage<E, false>(sm, false, keys, scr, tile, valid, SS_K, DeferredCounts{&sm.defer, rs.hist});
+            return;
+        }
+    }
+    tile_stage<E>(sm, greedy, keys, scr, tile, valid);
 }
 
 // Greedy row (wave 0): the argmax over the tiles' maxima, d2t remap, count update, outputs.

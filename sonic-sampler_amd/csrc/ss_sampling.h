@@ -1121,7 +1121,7 @@ struct NoCounts {
 };
 
 struct DeferredCounts {
-    bool on;
+    static constexpr bool on = true;
     const DeferState *state;  // valid after the selection's first barrier
     int hist;                 // RowState::hist
 
@@ -1206,10 +1206,14 @@ struct DeferredCounts {
     }
 };
 
-// Whether the penalties of a row can wait (DeferredCounts). A row under a grammar keeps the whole
-// chain: a tile that admits fewer than 128 tokens has no bound to hold them to.
+// Whether the penalties of a row may wait (DeferredCounts), by its indicator. A row under a grammar
+// keeps the whole chain: a tile that admits fewer than 128 tokens has no bound to hold them to.
+__device__ __forceinline__ bool counts_may_wait(const RowState &rs, const Uses &u) {
+    return u.rep && !u.g && !(rs.ind & IND_GREEDY);
+}
+
+// Whether they can: by its parameters.
 __device__ __forceinline__ bool counts_can_wait(const RowState &rs, const Uses &u) {
-    if (!u.rep || u.g || (rs.ind & IND_GREEDY)) return false;
     bool all_exc;
     const Chain k = row_chain(rs, u, all_exc);
     return (!k.mult || (k.rdiv.fast && k.rep >= 1.0f)) && (!k.freq || (k.fr >= 0.0f && !all_exc)) &&
