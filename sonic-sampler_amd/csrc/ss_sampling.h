@@ -940,6 +940,12 @@ __device__ __forceinline__ void prologue_keys(const RowState &rs, int col0, int 
             direct_keys<E, ANY, E>(rs, u, col0, lw, pl, ex, 0, keys);
             finish();
         }
+    } else if (E < 64 && __builtin_expect(!planes, 0)) {
+        // Rows of the logits alone, as in the direct layout: through the passes below 256 drafting rows
+        // of 32000 columns took 15.4 us a call instead of 14.7, and the kernel of 8192 columns kept its
+        // gathers in an order that cost rows with counts under a grammar 2%. At 64 elements a lane
+        // the logits kept for it spill.
+        plain_keys<E, ANY>(rs, u, lw, ex, keys);
     } else if constexpr (E >= 64) {
         // 4096-column passes, as above: the gathered columns and planes of all elements at once
         // would hold 156 VGPRs at E = 32 (three waves per SIMD).
