@@ -785,6 +785,15 @@ __device__ __forceinline__ void gather_keys(const RowState &rs, const Uses &u, i
             const __amdgpu_buffer_rsrc_t d = row_buffer(rs.dec, (int64_t)rs.vt * 4);
 #pragma unroll
             for (int j = 0; j < E; ++j) dec[j >> 2][j & 3] = __builtin_amdgcn_raw_buffer_load_b32(d, tcol[j] * 4, 0, 0);
+            // The history never counts token 0 (core/naive.py:179-203). It waits for the decode counts here,
+            // ahead of the other planes' gathers: the count planes of the rows an XCD works on exceed
+            // its L2 together, one after the other they fit it better (256 rows under a grammar with
+            // penalties, 32000 -> 128256 ids: 149 us with every gather in flight, 144.5 so).
+            for (uint64_t m = __ballot(rs.hist != 0); m; m &= m - 1) {
+                const int t = __builtin_amdgcn_readlane(rs.hist, __builtin_ctzll(m));
+#pragma unroll
+                for (int j = 0; j < E; ++j) dec[j >> 2][j & 3] += tcol[j] == t ? 1 : 0;
+            }
         }
         if (u.mult) {
             const __amdgpu_buffer_rsrc_t q = row_buffer(rs.ctx, (int64_t)rs.vt * 4);
@@ -797,14 +806,6 @@ __device__ __forceinline__ void gather_keys(const RowState &rs, const Uses &u, i
             for (int j = 0; j < E; ++j) {
                 const uint32_t h = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(b, tcol[j] * 2, 0, 0) << (16 * (j & 1));
                 if (j & 2) bw[j >> 2].y |= h; else bw[j >> 2].x |= h;
-            }
-        }
-        if (u.rep) {
-            // The history never counts token 0 (core/naive.py:179-203).
-            for (uint64_t m = __ballot(rs.hist != 0); m; m &= m - 1) {
-                const int t = __builtin_amdgcn_readlane(rs.hist, __builtin_ctzll(m));
-#pragma unroll
-                for (int j = 0; j < E; ++j) dec[j >> 2][j & 3] += tcol[j] == t ? 1 : 0;
             }
         }
     }
