@@ -1238,7 +1238,13 @@ __device__ __forceinline__ int wave_share(int want, int valid, int wave) {
     // whole 1024-column chunks give every wave 256 columns; the last chunk fills the waves in turn
     const int rest = valid & (SS_BLOCK * 4 - 1);
     const int n = (valid >> 10) * 256 + min(max(rest - 256 * wave, 0), 256);
-    return (want * n + valid - 1) / valid;
+    // ceil(want * n / valid), with the reciprocal's rounding put right by one comparison: as an integer
+    // division its dependent instructions held a partial tile up by 0.1 us, and with it a kernel of
+    // one generation of tiles (16 drafting rows under a grammar 10.75 -> 10.65 us a call; 160 plain
+    // verification rows in 4096-column tiles 28.7 -> 28.2)
+    const int p = want * n;
+    const int q = (int)((float)p * __builtin_amdgcn_rcpf((float)valid));
+    return __builtin_amdgcn_readfirstlane(q + (q * valid < p ? 1 : 0));
 }
 
 // The lane's keys from its spill. By recursion: as a loop in the retry's cycle the compiler left it

@@ -616,6 +616,55 @@ def test_direct_grammar_staging_stays_in_its_region_and_reproduces_the_row(vt):
 KEY_NEG_INF = 0x0080   # key of bf16 -inf; -NaN keys lie below it, absent elements are 0
 
 
+def wave_share(want, valid, wave, block):
+    """Keys that a wave's bound must leave: its share of `want` by its columns of the `valid` ones."""
+
+    if valid == block:
+
+        return -(-want // 4)
+
+    n = (valid >> 10) * 256 + min(max((valid & 1023) - 256 * wave, 0), 256)
+
+    return -(-want * n // valid)
+
+
+@pytest.mark.parametrize("block", [1024, 2048, 4096, 8192, 16384])
+def test_wave_share_by_a_reciprocal(block):
+    """The kernel's quotient, a float product with a reciprocal within 1 ulp and one comparison, is the
+    exact ceiling wherever that reciprocal lies; the waves' shares add up to the list's length."""
+
+    valid = np.arange(1, block, dtype=np.int64)
+    exact = np.float32(1) / valid.astype(np.float32)
+
+    for want in (1, 2, 4, 8, 16, 32, 64, 128, 160):
+
+        total = np.zeros_like(valid)
+
+        for wave in range(4):
+
+            n = (valid >> 10) * 256 + np.clip((valid & 1023) - 256 * wave, 0, 256)
+            p = want * n
+
+            for rcp in (exact, np.nextafter(exact, np.float32(0)), np.nextafter(exact, np.float32(2))):
+
+                q = (p.astype(np.float32) * rcp).astype(np.int64)
+                assert np.array_equal(q + (q * valid < p), -(-p // valid))
+
+            total += -(-p // valid)
+
+        assert (total >= want).all()
+
+    for v in (1, 255, 1023, 1025, block - 1):
+
+        assert [wave_share(128, min(v, block - 1), w, block) for w in range(4)] == \
+            [-(-128 * c // min(v, block - 1)) for c in wave_columns(min(v, block - 1))]
+
+
+def wave_columns(valid):
+
+    return [sum(1 for c in range(valid) if (c % 1024) // 256 == w) for w in range(4)]
+
+
 def tile_stage_emulation(keys, E, valid):
     """The tile's candidate list as tile_stage builds it, restated step by step: `keys` is the
     tile's 256 * E keys by column (0 past `valid`). Returns the list's (key, column) entries in
@@ -632,18 +681,26 @@ def tile_stage_emulation(keys, E, valid):
         m1 = [max(v) for v in lanes]
         m2 = [sorted(v)[-2] for v in lanes]
         bound = 0
+        need = wave_share(SS_K, valid, w, block)
 
-        for b in range(15, 1, -1):
+        if valid <= 1024 and valid < block:   # one partly filled chunk: the lanes' elements 0-3, all key bits
+
+            first, low = [k for v in lanes for k in v[:4]], 0
+
+        else:
+
+            first, low = (m1 if E >= 64 else m1 + m2), 2
+
+        for b in range(15, low - 1, -1):
 
             c = bound | (1 << b)
-            n = sum(x >= c for x in m1) + (0 if E >= 64 else sum(x >= c for x in m2))
-            bound = c if n >= 32 else bound
+            bound = c if sum(x >= c for x in first) >= need else bound
 
         if bound <= KEY_NEG_INF and valid >= SS_K:
 
             bound = KEY_NEG_INF + 1
 
-        bounds.append(bound)
+        bounds.append(bound if need else 0xfffc)   # no columns: no part in the tile's bound
 
     lo = min(bounds)
     t0 = lo - 1 if lo else 0
