@@ -186,14 +186,15 @@ def host():
 _empty = None
 
 
-def empty(device: torch.device | None, dtype: torch.dtype, *sizes: int) -> torch.Tensor:
-    """``torch.empty(sizes, dtype=dtype, device=device)``; natively where the device is known."""
+def empty(device, dtype: torch.dtype, *sizes: int) -> torch.Tensor:
+    """``torch.empty(sizes, dtype=dtype, device=device)``; natively on a GPU's ``torch.device``, through
+    torch for any other form of a device (None, a string, an index) and for other devices."""
 
     global _empty
 
-    if device is None:
+    if type(device) is not torch.device or device.type != "cuda":
 
-        return torch.empty(sizes, dtype=dtype)
+        return torch.empty(sizes, dtype=dtype, device=device)
 
     if _empty is None:
 

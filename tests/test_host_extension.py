@@ -64,6 +64,36 @@ def test_empty_is_torch_empty():
         _native.host().empty("cpu", torch.int32, 3)
 
 
+@pytest.mark.parametrize("device", ["cpu", torch.device("cpu"), None])
+def test_output_containers_take_any_form_of_a_device(device, monkeypatch):
+    """As torch.empty does; on the CPU without the host extension."""
+
+    from sonic_sampler.base.sampler import LogProbabilities, TopTargets
+
+    monkeypatch.setattr(_native, "host", lambda: pytest.fail("the host extension was asked for"))
+    monkeypatch.setattr(_native, "_empty", None)
+
+    for t in (LogProbabilities.empty_blocked(2, 3, 4, device=device), LogProbabilities.empty_varlen(6, 4, device=device)):
+
+        assert t.selected.device.type == "cpu" and t.selected.dtype == torch.bfloat16
+        assert t.top_k.tokens.dtype == torch.int32 and t.top_k.logprobs.numel() == 24
+
+    assert TopTargets.empty_blocked(2, 4, device=device).tokens.shape == (2, 4)
+    assert TopTargets.empty_varlen(6, 4, device=device).logprobs.shape == (6, 4)
+
+
+@pytest.mark.parametrize("device", ["cuda", "cuda:0", 0])
+def test_output_containers_name_a_gpu_as_torch_does(device, monkeypatch):
+    """A GPU's name or index goes to torch.empty as it is."""
+
+    from sonic_sampler.base.sampler import LogProbabilities
+
+    seen = []
+    monkeypatch.setattr(torch, "empty", lambda *a, **kw: seen.append(kw["device"]))
+    LogProbabilities.empty_varlen(6, device=device)
+    assert seen == [device]
+
+
 def test_entries_take_bytes_only():
 
     call = _native.packed_entry("ss_topk")
