@@ -203,6 +203,16 @@ def empty(device, dtype: torch.dtype, *sizes: int) -> torch.Tensor:
     return _empty(device, dtype, *sizes)
 
 
+def new_empty(source: torch.Tensor, dtype: torch.dtype, *sizes: int) -> torch.Tensor:
+    """``source.new_empty(sizes, dtype=dtype)``: on the source's device, of its tensor class."""
+
+    if type(source) is not torch.Tensor:
+
+        return source.new_empty(sizes, dtype=dtype)
+
+    return empty(source.device, dtype, *sizes)
+
+
 def check(status: int, what: str) -> None:
 
     if status != SS_OK:

@@ -157,7 +157,7 @@ class Verification:
 
         buffer = None
         device = tokens.device
-        offsets = _native.empty(device, I32, batch_size, 1)
+        offsets = _native.new_empty(tokens, I32, batch_size, 1)
 
         if logprobs:
 

@@ -133,7 +133,7 @@ def resolve_tokens(drafted: Tensor, output: Optional[Tensor]) -> Tensor:
     token at its offset), so a new buffer holds the same tokens without a copy launch ahead of the
     tile stage."""
 
-    return output if output is not None else _native.empty(drafted.device, drafted.dtype, *drafted.shape)
+    return output if output is not None else _native.new_empty(drafted, drafted.dtype, *drafted.shape)
 
 
 def fused_multistep(

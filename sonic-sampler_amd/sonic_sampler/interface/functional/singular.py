@@ -73,7 +73,7 @@ SINGULAR_CALL = _native.Gatherer(
 
 def resolve_tokens(buffer: Optional[Tensor], batch_size: int, source: Tensor) -> Tensor:
 
-    return buffer if buffer is not None else _native.empty(source.device, I32, batch_size, 1)
+    return buffer if buffer is not None else _native.new_empty(source, I32, batch_size, 1)
 
 
 def resolve_probabilities(precondition: bool, source: Tensor, batch_size: int,

@@ -94,6 +94,23 @@ def test_output_containers_name_a_gpu_as_torch_does(device, monkeypatch):
     assert seen == [device]
 
 
+def test_outputs_are_of_their_source_class():
+    """Token and offset buffers made for a tensor subclass are of that class, as new_empty and
+    empty_like make them: the buffers' prefix-contiguous slices index differently."""
+
+    from sonic_sampler.base.sampler import Verification
+    from sonic_sampler.base.tensor import PrefixContiguousTensor, prefix_contiguous
+    from sonic_sampler.interface.functional import multistep, singular
+
+    drafted = prefix_contiguous(torch.zeros(4, 3, dtype=torch.int32))
+    tokens = multistep.resolve_tokens(drafted, None)
+    assert type(tokens) is PrefixContiguousTensor and tokens.shape == (4, 3) and tokens.dtype == torch.int32
+    assert type(Verification.from_tokens(tokens, 4, 3).offsets) is PrefixContiguousTensor
+    logits = prefix_contiguous(torch.zeros(4, 8, dtype=torch.bfloat16))
+    assert type(singular.resolve_tokens(None, 4, logits)) is PrefixContiguousTensor
+    assert type(multistep.resolve_tokens(drafted.as_subclass(torch.Tensor), None)) is torch.Tensor
+
+
 def test_entries_take_bytes_only():
 
     call = _native.packed_entry("ss_topk")
