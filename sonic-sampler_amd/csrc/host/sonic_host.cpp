@@ -17,10 +17,11 @@
 #include <ATen/ATen.h>
 #include <torch/csrc/Device.h>
 #include <torch/csrc/Dtype.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstring>
-#include <exception>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -131,17 +132,13 @@ bool put(const Field &f, PyObject *arg, char *out) {
     return true;
 }
 
-// Runs fn, with a C++ exception (torch's among them) as a RuntimeError.
+// Runs fn, with a C++ exception as the Python one that torch's own bindings raise for it
+// (torch.OutOfMemoryError, IndexError, NotImplementedError, ...).
 template <class F>
 PyObject *guarded(F fn) {
-    try {
-        return fn();
-    } catch (const std::exception &e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
-    } catch (...) {
-        PyErr_SetString(PyExc_RuntimeError, "unknown C++ exception");
-    }
-    return nullptr;
+    HANDLE_TH_ERRORS
+    return fn();
+    END_HANDLE_TH_ERRORS
 }
 
 PyObject *gather(PyObject *, PyObject *const *args, Py_ssize_t n) {

@@ -111,6 +111,46 @@ def test_outputs_are_of_their_source_class():
     assert type(multistep.resolve_tokens(drafted.as_subclass(torch.Tensor), None)) is torch.Tensor
 
 
+def test_errors_are_those_of_torch():
+    """A failed allocation and a stride that a tensor does not have raise what torch's own calls do."""
+
+    call = _native.host().empty
+    backend = torch.device("xla")
+
+    with pytest.raises(Exception) as want:
+
+        torch.empty(3, device=backend)
+
+    with pytest.raises(type(want.value)) as got:
+
+        call(backend, torch.float32, 3)
+
+    assert type(want.value) is not RuntimeError and type(got.value) is type(want.value)
+
+    with pytest.raises(IndexError):
+
+        gatherer().gather(0, 0, None, 0, torch.tensor(1.0), None)
+
+
+@pytest.mark.gpu
+def test_out_of_memory_is_torchs():
+    """With the process held to a small share of the card, which the allocator checks itself."""
+
+    device = torch.device("cuda:0")
+    total = torch.cuda.get_device_properties(device).total_memory
+    torch.cuda.set_per_process_memory_fraction(0.05, device)
+
+    try:
+
+        with pytest.raises(torch.OutOfMemoryError):
+
+            _native.empty(device, torch.uint8, total // 10)
+
+    finally:
+
+        torch.cuda.set_per_process_memory_fraction(1.0, device)
+
+
 def test_entries_take_bytes_only():
 
     call = _native.packed_entry("ss_topk")
