@@ -19,10 +19,12 @@
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/device_lazy_init.h>
 
 #include <cstring>
 #include <memory>
 #include <string>
+#include <utility>
 #include <vector>
 
 namespace {
@@ -141,6 +143,13 @@ PyObject *guarded(F fn) {
     END_HANDLE_TH_ERRORS
 }
 
+// The GIL given up for a scope, as torch's own factories do: an allocation that misses the cache
+// waits for the device, and other threads (a host callback that the wait depends on, too) go on.
+struct ReleasedGil {
+    PyThreadState *state = PyEval_SaveThread();
+    ~ReleasedGil() { PyEval_RestoreThread(state); }
+};
+
 PyObject *gather(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (n < 1) {
         PyErr_SetString(PyExc_TypeError, "gather(layout, *args)");
@@ -166,11 +175,12 @@ PyObject *gather(PyObject *, PyObject *const *args, Py_ssize_t n) {
 }
 
 PyObject *empty(PyObject *, PyObject *const *args, Py_ssize_t n) {
-    if (n < 3 || n > 6 || !THPDevice_Check(args[0]) || !THPDtype_Check(args[1])) {
-        PyErr_SetString(PyExc_TypeError, "empty(device, dtype, *sizes) with 1 to 4 sizes");
+    constexpr Py_ssize_t MAX_DIMS = 8;
+    if (n < 2 || n > 2 + MAX_DIMS || !THPDevice_Check(args[0]) || !THPDtype_Check(args[1])) {
+        PyErr_SetString(PyExc_TypeError, "empty(device, dtype, *sizes) with at most 8 sizes");
         return nullptr;
     }
-    int64_t sizes[4];
+    int64_t sizes[MAX_DIMS];
     for (Py_ssize_t i = 2; i < n; ++i) {
         sizes[i - 2] = PyLong_AsLongLong(args[i]);
         if (sizes[i - 2] == -1 && PyErr_Occurred()) return nullptr;
@@ -179,7 +189,13 @@ PyObject *empty(PyObject *, PyObject *const *args, Py_ssize_t n) {
         const auto options = at::TensorOptions()
                                  .device(reinterpret_cast<THPDevice *>(args[0])->device)
                                  .dtype(reinterpret_cast<THPDtype *>(args[1])->scalar_type);
-        return THPVariable_Wrap(at::empty(at::IntArrayRef(sizes, (size_t)(n - 2)), options));
+        torch::utils::maybe_initialize_device(options);
+        at::Tensor t;
+        {
+            const ReleasedGil released;
+            t = at::empty(at::IntArrayRef(sizes, (size_t)(n - 2)), options);
+        }
+        return THPVariable_Wrap(std::move(t));
     });
 }
 

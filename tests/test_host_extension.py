@@ -1,6 +1,8 @@
 """The host extension's packing, allocation and entry calls (CPU): each refuses what does not fit."""
 
 import ctypes
+import threading
+import time
 
 import numpy as np
 import pytest
@@ -130,6 +132,40 @@ def test_errors_are_those_of_torch():
     with pytest.raises(IndexError):
 
         gatherer().gather(0, 0, None, 0, torch.tensor(1.0), None)
+
+
+def test_allocation_lets_other_threads_run():
+    """A second thread goes on while an allocation takes its time (here: the fill of deterministic
+    mode), as it does beside torch.empty."""
+
+    call, stamps, stop = _native.host().empty, [], threading.Event()
+
+    def tick():
+
+        while not stop.is_set():
+
+            stamps.append(time.perf_counter())
+            time.sleep(0.001)
+
+    thread = threading.Thread(target=tick)
+    torch.use_deterministic_algorithms(True)
+
+    try:
+
+        thread.start()
+        start = time.perf_counter()
+        kept = call(torch.device("cpu"), torch.float32, 2 ** 28)
+        end = time.perf_counter()
+
+    finally:
+
+        stop.set()
+        thread.join()
+        torch.use_deterministic_algorithms(False)
+
+    assert kept[0].isnan() and end - start > 0.02, "the fill was too short to tell"
+    inside = [s for s in stamps if start + 0.2 * (end - start) < s < end - 0.2 * (end - start)]
+    assert inside, "no other thread ran during the allocation"
 
 
 @pytest.mark.gpu
