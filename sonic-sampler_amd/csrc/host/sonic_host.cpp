@@ -6,7 +6,7 @@
 //   make_layout(size, fields) -> capsule     fields: (code, offset, offset, offset, name) per argument
 //   gather(capsule, *args) -> bytes          the struct, every other byte zero
 //   empty(device, dtype, *sizes) -> Tensor   torch.empty
-//   entry(address) -> callable               the entry point at `address`, taking the struct's bytes
+//   entry(address, size) -> callable         the entry point at `address`, taking its struct's `size` bytes
 //
 // Argument codes: a scalar of the field's type ('i', 'I', 'q', 'Q'), or a tensor (None: zeros) whose
 // address goes to the first offset ('T'), with its leading stride ('S'), or its leading and, of a
@@ -199,48 +199,57 @@ PyObject *empty(PyObject *, PyObject *const *args, Py_ssize_t n) {
     });
 }
 
-// An entry point of the library called with the struct's bytes, the GIL released meanwhile.
+// An entry point of the library called with the struct's bytes, the GIL released meanwhile. `self`
+// is its (address, size of the struct): bytes of any other length are refused, the entry point would
+// read past them.
 PyObject *call_entry(PyObject *self, PyObject *bytes) {
     using Entry = int (*)(const void *);
-    const auto fn = reinterpret_cast<Entry>(PyLong_AsVoidPtr(self));
-    if (!fn) {
-        if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "no entry point");
-        return nullptr;
-    }
+    const auto fn = reinterpret_cast<Entry>(PyLong_AsVoidPtr(PyTuple_GET_ITEM(self, 0)));
+    const Py_ssize_t size = PyLong_AsSsize_t(PyTuple_GET_ITEM(self, 1));
+    if (PyErr_Occurred()) return nullptr;
     if (!PyBytes_Check(bytes)) {
         PyErr_SetString(PyExc_TypeError, "the argument struct's bytes are expected");
         return nullptr;
     }
-    // the argument structs hold 8-byte fields: a payload off an 8-byte boundary is copied
-    const char *p = PyBytes_AS_STRING(bytes);
-    std::vector<uint64_t> aligned;
-    if ((uintptr_t)p % 8 != 0) {
-        aligned.resize(((size_t)PyBytes_GET_SIZE(bytes) + 7) / 8);
-        std::memcpy(aligned.data(), p, (size_t)PyBytes_GET_SIZE(bytes));
-        p = reinterpret_cast<const char *>(aligned.data());
+    if (PyBytes_GET_SIZE(bytes) != size) {
+        PyErr_Format(PyExc_ValueError, "an argument struct of %zd bytes is expected, got %zd", size, PyBytes_GET_SIZE(bytes));
+        return nullptr;
     }
-    int status = 0;
-    Py_BEGIN_ALLOW_THREADS
-    status = fn(p);
-    Py_END_ALLOW_THREADS
-    return PyLong_FromLong(status);
+    return guarded([&]() -> PyObject * {
+        // the argument structs hold 8-byte fields: a payload off an 8-byte boundary is copied
+        const char *p = PyBytes_AS_STRING(bytes);
+        std::vector<uint64_t> aligned;
+        if ((uintptr_t)p % 8 != 0) {
+            aligned.resize(((size_t)size + 7) / 8);
+            std::memcpy(aligned.data(), p, (size_t)size);
+            p = reinterpret_cast<const char *>(aligned.data());
+        }
+        int status = 0;
+        {
+            const ReleasedGil released;
+            status = fn(p);
+        }
+        return PyLong_FromLong(status);
+    });
 }
 
 PyMethodDef call_entry_def = {"call", (PyCFunction)call_entry, METH_O, nullptr};
 
-PyObject *entry(PyObject *, PyObject *address) {
-    if (!PyLong_Check(address)) {
-        PyErr_SetString(PyExc_TypeError, "entry(address)");
+PyObject *entry(PyObject *, PyObject *args) {
+    PyObject *address = nullptr, *size = nullptr;
+    if (!PyArg_ParseTuple(args, "O!O!", &PyLong_Type, &address, &PyLong_Type, &size)) return nullptr;
+    if (!PyLong_AsVoidPtr(address)) {
+        if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "no entry point");
         return nullptr;
     }
-    return PyCFunction_New(&call_entry_def, address);
+    return PyCFunction_New(&call_entry_def, args);
 }
 
 PyMethodDef methods[] = {
     {"make_layout", (PyCFunction)make_layout, METH_VARARGS, nullptr},
     {"gather", (PyCFunction)(void (*)(void))gather, METH_FASTCALL, nullptr},
     {"empty", (PyCFunction)(void (*)(void))empty, METH_FASTCALL, nullptr},
-    {"entry", (PyCFunction)entry, METH_O, nullptr},
+    {"entry", (PyCFunction)entry, METH_VARARGS, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
 

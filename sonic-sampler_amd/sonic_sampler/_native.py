@@ -116,6 +116,11 @@ def library_path() -> Path:
     return Path(os.environ.get("SONIC_SAMPLER_LIB", _LIB_PATH))
 
 
+# the entry points that take one argument struct
+_ENTRIES = {"ss_topk": TopKArgs, "ss_fused_singular": SingularArgs, "ss_fused_singular_noalloc": SingularArgs,
+            "ss_fused_multistep": MultistepArgs, "ss_indexed_copy": IndexedCopyArgs}
+
+
 def load() -> ctypes.CDLL:
     """Loads (once) and returns the HIP library; raises if it is absent or mismatched."""
 
@@ -140,9 +145,7 @@ def load() -> ctypes.CDLL:
     lib.ss_args_size.restype = c_i64
     lib.ss_args_size.argtypes = [c_i32]
 
-    for name, struct in (("ss_topk", TopKArgs), ("ss_fused_singular", SingularArgs),
-                         ("ss_fused_singular_noalloc", SingularArgs),
-                         ("ss_fused_multistep", MultistepArgs), ("ss_indexed_copy", IndexedCopyArgs)):
+    for name, struct in _ENTRIES.items():
         fn = getattr(lib, name)
         fn.restype = c_i32
         fn.argtypes = [ctypes.POINTER(struct)]
@@ -353,7 +356,8 @@ def packed_entry(name: str):
 
     if fn is None:
 
-        fn = _packed_entries[name] = host().entry(ctypes.cast(load()[name], c_p).value)
+        fn = _packed_entries[name] = host().entry(ctypes.cast(load()[name], c_p).value,
+                                                  ctypes.sizeof(_ENTRIES[name]))
 
     return fn
 

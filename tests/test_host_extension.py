@@ -195,4 +195,15 @@ def test_entries_take_bytes_only():
 
         call(None)
 
+    # a struct that ends early would be read past its end
+    for size in (0, ctypes.sizeof(_native.TopKArgs) - 1, ctypes.sizeof(_native.TopKArgs) + 8):
+
+        with pytest.raises(ValueError, match="bytes"):
+
+            call(bytes(size))
+
+    with pytest.raises(ValueError):
+
+        _native.host().entry(0, 8)
+
     assert call(bytes(ctypes.sizeof(_native.TopKArgs))) == 1  # no logits
