@@ -46,35 +46,6 @@ void destroy(PyObject *capsule) { delete static_cast<Layout *>(PyCapsule_GetPoin
 
 int field_bytes(char code) { return code == 'i' || code == 'I' ? 4 : 8; }
 
-PyObject *make_layout(PyObject *, PyObject *args) {
-    Py_ssize_t size = 0;
-    PyObject *list = nullptr;
-    if (!PyArg_ParseTuple(args, "nO!", &size, &PyList_Type, &list)) return nullptr;
-    auto layout = std::make_unique<Layout>();
-    layout->size = size;
-    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(list); ++i) {
-        int code = 0;
-        const char *name = nullptr;
-        Field f;
-        if (!PyArg_ParseTuple(PyList_GET_ITEM(list, i), "Cnnns", &code, &f.at[0], &f.at[1], &f.at[2], &name)) return nullptr;
-        f.code = (char)code;
-        f.name = name;
-        if (!std::strchr("iIqQTSUtsu", f.code)) {
-            PyErr_Format(PyExc_ValueError, "unknown field code %c", code);
-            return nullptr;
-        }
-        const int used = f.code == 'S' || f.code == 's' ? 2 : f.code == 'U' || f.code == 'u' ? 3 : 1;
-        for (int k = 0; k < used; ++k) {
-            if (f.at[k] < 0 || f.at[k] + field_bytes(f.code) > size) {
-                PyErr_Format(PyExc_ValueError, "field %s outside the struct", name);
-                return nullptr;
-            }
-        }
-        layout->fields.push_back(std::move(f));
-    }
-    return PyCapsule_New(layout.release(), CAPSULE, destroy);
-}
-
 // Writes one argument of the struct; false with a Python error set.
 bool put(const Field &f, PyObject *arg, char *out) {
     if (f.code == 'q' || f.code == 'i') {
@@ -141,6 +112,39 @@ PyObject *guarded(F fn) {
     HANDLE_TH_ERRORS
     return fn();
     END_HANDLE_TH_ERRORS
+}
+
+PyObject *make_layout(PyObject *, PyObject *args) {
+    Py_ssize_t size = 0;
+    PyObject *list = nullptr;
+    if (!PyArg_ParseTuple(args, "nO!", &size, &PyList_Type, &list)) return nullptr;
+    return guarded([&]() -> PyObject * {
+        auto layout = std::make_unique<Layout>();
+        layout->size = size;
+        for (Py_ssize_t i = 0; i < PyList_GET_SIZE(list); ++i) {
+            int code = 0;
+            const char *name = nullptr;
+            Field f;
+            if (!PyArg_ParseTuple(PyList_GET_ITEM(list, i), "Cnnns", &code, &f.at[0], &f.at[1], &f.at[2], &name)) return nullptr;
+            if (code <= 0 || code > 127 || !std::strchr("iIqQTSUtsu", code)) {
+                PyErr_Format(PyExc_ValueError, "unknown field code %d", code);
+                return nullptr;
+            }
+            f.code = (char)code;
+            f.name = name;
+            const int used = f.code == 'S' || f.code == 's' ? 2 : f.code == 'U' || f.code == 'u' ? 3 : 1;
+            for (int k = 0; k < used; ++k) {
+                if (f.at[k] < 0 || f.at[k] > size - field_bytes(f.code)) {
+                    PyErr_Format(PyExc_ValueError, "field %s outside the struct", name);
+                    return nullptr;
+                }
+            }
+            layout->fields.push_back(std::move(f));
+        }
+        PyObject *capsule = PyCapsule_New(layout.get(), CAPSULE, destroy);
+        if (capsule) layout.release();
+        return capsule;
+    });
 }
 
 // The GIL given up for a scope, as torch's own factories do: an allocation that misses the cache

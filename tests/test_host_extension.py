@@ -52,6 +52,18 @@ def test_refuses_what_does_not_fit(args, error, text):
         gatherer().gather(*args)
 
 
+@pytest.mark.parametrize("size,field,error", [
+    (16, ("\0", 0, 0, 0, "x"), ValueError), (16, ("x", 0, 0, 0, "x"), ValueError), (16, ("\u0169", 0, 0, 0, "x"), ValueError),
+    (16, ("q", 9, 0, 0, "x"), ValueError), (16, ("q", 2 ** 63 - 1, 0, 0, "x"), ValueError), (4, ("q", 0, 0, 0, "x"), ValueError),
+    (16, ("S", 0, 16, 0, "x"), ValueError), (16, ("i", -1, 0, 0, "x"), ValueError), (16, ("i", 0), TypeError),
+])
+def test_layouts_refuse_fields_outside_the_struct(size, field, error):
+
+    with pytest.raises(error):
+
+        _native.host().make_layout(size, [field])
+
+
 def test_empty_is_torch_empty():
 
     t = _native.empty(torch.device("cpu"), torch.bfloat16, 3, 0, 2)
