@@ -5,13 +5,14 @@
 //
 //   make_layout(size, fields) -> capsule     fields: (code, offset, offset, offset, name) per argument
 //   gather(capsule, *args) -> bytes          the struct, every other byte zero
+//   unit_strides(names, *tensors)            ValueError naming the first tensor (None: skipped) that is not
+//                                            contiguous along its last dimension
 //   empty(device, dtype, *sizes) -> Tensor   torch.empty
 //   entry(address, size) -> callable         the entry point at `address`, taking its struct's `size` bytes
 //
 // Argument codes: a scalar of the field's type ('i', 'I', 'q', 'Q'), or a tensor (None: zeros) whose
 // address goes to the first offset ('T'), with its leading stride ('S'), or its leading and, of a
-// three-dimensional one, its second stride ('U'). Lower case 't', 's', 'u': the tensor must be
-// contiguous along its last dimension (ValueError).
+// three-dimensional one, its second stride ('U').
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -87,17 +88,12 @@ bool put(const Field &f, PyObject *arg, char *out) {
         return false;
     }
     const at::Tensor &t = THPVariable_Unpack(arg);
-    const bool unit = f.code >= 'a';
-    if (unit && t.dim() > 0 && t.stride(-1) != 1) {
-        PyErr_Format(PyExc_ValueError, "`%s` must be contiguous along its last dimension", f.name.c_str());
-        return false;
-    }
     const uint64_t p = (uint64_t)(uintptr_t)t.data_ptr();
     std::memcpy(out + f.at[0], &p, 8);
-    if (f.code != 'T' && f.code != 't') {
+    if (f.code != 'T') {
         const int64_t s = t.stride(0);
         std::memcpy(out + f.at[1], &s, 8);
-        if (f.code == 'U' || f.code == 'u') {
+        if (f.code == 'U') {
             const int64_t step = t.dim() >= 3 ? t.stride(1) : 0;
             std::memcpy(out + f.at[2], &step, 8);
         }
@@ -126,13 +122,13 @@ PyObject *make_layout(PyObject *, PyObject *args) {
             const char *name = nullptr;
             Field f;
             if (!PyArg_ParseTuple(PyList_GET_ITEM(list, i), "Cnnns", &code, &f.at[0], &f.at[1], &f.at[2], &name)) return nullptr;
-            if (code <= 0 || code > 127 || !std::strchr("iIqQTSUtsu", code)) {
+            if (code <= 0 || code > 127 || !std::strchr("iIqQTSU", code)) {
                 PyErr_Format(PyExc_ValueError, "unknown field code %d", code);
                 return nullptr;
             }
             f.code = (char)code;
             f.name = name;
-            const int used = f.code == 'S' || f.code == 's' ? 2 : f.code == 'U' || f.code == 'u' ? 3 : 1;
+            const int used = f.code == 'S' ? 2 : f.code == 'U' ? 3 : 1;
             for (int k = 0; k < used; ++k) {
                 if (f.at[k] < 0 || f.at[k] > size - field_bytes(f.code)) {
                     PyErr_Format(PyExc_ValueError, "field %s outside the struct", name);
@@ -176,6 +172,29 @@ PyObject *gather(PyObject *, PyObject *const *args, Py_ssize_t n) {
     });
     if (!done) Py_DECREF(bytes);
     return done;
+}
+
+PyObject *unit_strides(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    if (n < 1 || !PyTuple_Check(args[0]) || PyTuple_GET_SIZE(args[0]) != n - 1) {
+        PyErr_SetString(PyExc_TypeError, "unit_strides(names, *tensors) with a tuple of a name for each tensor");
+        return nullptr;
+    }
+    return guarded([&]() -> PyObject * {
+        for (Py_ssize_t i = 1; i < n; ++i) {
+            if (args[i] == Py_None) continue;
+            PyObject *name = PyTuple_GET_ITEM(args[0], i - 1);
+            if (!THPVariable_Check(args[i])) {
+                PyErr_Format(PyExc_TypeError, "`%S` must be a tensor or None", name);
+                return nullptr;
+            }
+            const at::Tensor &t = THPVariable_Unpack(args[i]);
+            if (t.dim() > 0 && t.stride(-1) != 1) {
+                PyErr_Format(PyExc_ValueError, "`%S` must be contiguous along its last dimension", name);
+                return nullptr;
+            }
+        }
+        Py_RETURN_NONE;
+    });
 }
 
 PyObject *empty(PyObject *, PyObject *const *args, Py_ssize_t n) {
@@ -252,6 +271,7 @@ PyObject *entry(PyObject *, PyObject *args) {
 PyMethodDef methods[] = {
     {"make_layout", (PyCFunction)make_layout, METH_VARARGS, nullptr},
     {"gather", (PyCFunction)(void (*)(void))gather, METH_FASTCALL, nullptr},
+    {"unit_strides", (PyCFunction)(void (*)(void))unit_strides, METH_FASTCALL, nullptr},
     {"empty", (PyCFunction)(void (*)(void))empty, METH_FASTCALL, nullptr},
     {"entry", (PyCFunction)entry, METH_VARARGS, nullptr},
     {nullptr, nullptr, 0, nullptr},

@@ -206,6 +206,12 @@ def empty(device, dtype: torch.dtype, *sizes: int) -> torch.Tensor:
     return _empty(device, dtype, *sizes)
 
 
+def unit_strides(names: tuple, *tensors: torch.Tensor | None) -> None:
+    """ValueError naming the first of the tensors that is not contiguous along its last dimension."""
+
+    host().unit_strides(names, *tensors)
+
+
 def new_empty(source: torch.Tensor, dtype: torch.dtype, *sizes: int) -> torch.Tensor:
     """``source.new_empty(sizes, dtype=dtype)``: on the source's device, of its tensor class."""
 
@@ -312,9 +318,8 @@ class Gatherer:
     declaration order, packed by the host extension. ``tensors`` names the pointer fields that come
     as tensors (or None, for zeros) and what is taken of each: "T" its address; "S" also its leading
     stride, into the field behind (which then is no argument of its own); "U" also the second
-    stride of a three-dimensional one, into the field behind that. In lower case the tensor must be
-    contiguous along its last dimension (ValueError). ``labels`` renames fields in error messages.
-    ``fields`` lists the positions' names."""
+    stride of a three-dimensional one, into the field behind that. ``labels`` renames fields in error
+    messages. ``fields`` lists the positions' names."""
 
     def __init__(self, cls, tensors: dict, labels: dict | None = None):
 
@@ -326,7 +331,7 @@ class Gatherer:
 
             name, offset, _, code = layout[i]
             code = tensors.get(name, code)
-            used = {"S": 2, "U": 3}.get(code.upper(), 1)
+            used = {"S": 2, "U": 3}.get(code, 1)
             at = [layout[i + k][1] if k < used else 0 for k in range(3)]
             rows.append((code, *at, name))
             i += used

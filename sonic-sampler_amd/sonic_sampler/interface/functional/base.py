@@ -65,13 +65,6 @@ def collapse_2d(value: Tensor) -> Tensor:
     return value if value.dim() == 2 else value.flatten(0, -2)
 
 
-def unit_stride(name: str, tensor: Optional[Tensor]) -> None:
-
-    if tensor is not None and tensor.dim() > 0 and tensor.stride(-1) != 1:
-
-        raise ValueError(f"`{name}` must be contiguous along its last dimension")
-
-
 def require_cover(name: str, tensor: Optional[Tensor], rows: int, cols: int, steps: int = 1) -> None:
     """A buffer the kernels address by slot: rows [0, rows), columns [0, cols) and, for a
     [slots, steps, cols] buffer, steps [0, steps). Its storage must hold the last such element: a

@@ -34,7 +34,6 @@ from sonic_sampler.interface.functional.base import (
     fresh_seed,
     require_cover,
     resolve_scratchpad,
-    unit_stride,
     validate_block,
     validate_count_update,
 )
@@ -49,13 +48,16 @@ MULTISTEP_ARGS = _native.Packer(_native.MultistepArgs)
 # the same struct from the call's tensors; their addresses and strides are taken natively
 MULTISTEP_CALL = _native.Gatherer(
     _native.MultistepArgs,
-    dict(logits="s", cu_seqlens="T", indicators="t", slot_mapping="T", drafted_tokens="T", grammar="u",
-         context_counts="s", decode_counts="s", repetition="T", frequency="T", presence="T", logit_bias="s",
-         temperature="T", top_k="T", top_p="T", min_p="T", top_logprobs="T", draft_probabilities="u", uniform="S",
-         gumbel="u", out_tokens="T", offsets="T", logprobs="T", top_values="T", top_tokens="S", values="T",
+    dict(logits="S", cu_seqlens="T", indicators="T", slot_mapping="T", drafted_tokens="T", grammar="U",
+         context_counts="S", decode_counts="S", repetition="T", frequency="T", presence="T", logit_bias="S",
+         temperature="T", top_k="T", top_p="T", min_p="T", top_logprobs="T", draft_probabilities="U", uniform="S",
+         gumbel="U", out_tokens="T", offsets="T", logprobs="T", top_values="T", top_tokens="S", values="T",
          indices="T", scratch="S"),
     labels=dict(gumbel="gumbel_noise"),
 )
+
+ROW_PLANES = ("logits", "grammar", "context_counts", "decode_counts", "logit_bias", "gumbel_noise",
+              "draft_probabilities", "indicators")
 
 
 def resolve_batch_vocab(logits: Tensor, cu_seqlens: Optional[Tensor], lookahead: Optional[int]):
@@ -216,6 +218,10 @@ def fused_multistep(
 
     flat_logits = collapse_2d(logits)
 
+    # ahead of everything that a refused call must not have done: outputs, seeds, events
+    _native.unit_strides(ROW_PLANES, flat_logits, grammar, context_counts, decode_counts, logit_bias, gumbel_noise,
+                         draft_probabilities, indicators)
+
     if not drafted_tokens.is_contiguous():
 
         raise ValueError("drafted_tokens must be contiguous")
@@ -268,8 +274,6 @@ def fused_multistep(
 
     if philox_on:
 
-        # not read, but held to the same layout
-        unit_stride("gumbel_noise", gumbel_noise)
         gumbel_noise = None
 
     # ss_multistep_args in declaration order (MULTISTEP_CALL.fields names the positions).

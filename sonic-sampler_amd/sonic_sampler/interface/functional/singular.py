@@ -46,7 +46,6 @@ from sonic_sampler.interface.functional.base import (
     I32,
     fresh_seed,
     require_cover,
-    unit_stride,
     validate_block,
     validate_count_update,
 )
@@ -63,12 +62,15 @@ SINGULAR_ARGS = _native.Packer(_native.SingularArgs)
 # the same struct from the call's tensors; their addresses and strides are taken natively
 SINGULAR_CALL = _native.Gatherer(
     _native.SingularArgs,
-    dict(logits="s", indicators="t", slot_mapping="T", d2t="T", grammar="s", context_counts="s", decode_counts="s",
-         drafted_tokens="s", repetition="T", frequency="T", presence="T", logit_bias="s", temperature="T", top_k="T",
-         top_p="T", min_p="T", top_logprobs="T", gumbel="s", tokens="S", logprobs="S", top_values="T", top_tokens="S",
-         probabilities="s", scratch="S"),
+    dict(logits="S", indicators="T", slot_mapping="T", d2t="T", grammar="S", context_counts="S", decode_counts="S",
+         drafted_tokens="S", repetition="T", frequency="T", presence="T", logit_bias="S", temperature="T", top_k="T",
+         top_p="T", min_p="T", top_logprobs="T", gumbel="S", tokens="S", logprobs="S", top_values="T", top_tokens="S",
+         probabilities="S", scratch="S"),
     labels=dict(gumbel="gumbel_noise", probabilities="draft_probabilities"),
 )
+
+ROW_PLANES = ("logits", "grammar", "context_counts", "decode_counts", "logit_bias", "gumbel_noise",
+              "draft_probabilities", "indicators", "drafted_tokens")
 
 
 def resolve_tokens(buffer: Optional[Tensor], batch_size: int, source: Tensor) -> Tensor:
@@ -170,6 +172,9 @@ def fused_singular(
 
         raise ValueError(f"top logprobs must be within the interval [0, {MAX_K}]")
 
+    # ahead of everything that a refused call must not have done: outputs, seeds, events
+    _native.unit_strides(ROW_PLANES, logits, grammar, context_counts, decode_counts, logit_bias, gumbel_noise,
+                         draft_probabilities, indicators, drafted_tokens)
     _native.require_device(logits, indicators)
 
     batch_size, vocab_size = logits.shape
@@ -251,8 +256,6 @@ def fused_singular(
 
     if philox_on:
 
-        # not read, but held to the same layout
-        unit_stride("gumbel_noise", gumbel_noise)
         gumbel_noise = None
 
     # ss_singular_args in declaration order (SINGULAR_CALL.fields names the positions)

@@ -31,7 +31,7 @@ BF16 = torch.bfloat16
 FP32 = torch.float32
 I32 = torch.int32
 
-TOPK_CALL = _native.Gatherer(_native.TopKArgs, dict(logits="s", scratch="S", values="T", indices="T"))
+TOPK_CALL = _native.Gatherer(_native.TopKArgs, dict(logits="S", scratch="S", values="T", indices="T"))
 
 
 @dataclass(eq=False, kw_only=True)

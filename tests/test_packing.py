@@ -406,3 +406,49 @@ def test_undersized_probability_buffers_are_rejected(captured):
 
     fm.fused_multistep(**base, draft_probabilities=torch.zeros(5, gamma, vocab, dtype=torch.bfloat16))
     assert len(captured.calls) == 2
+
+
+ROW_PLANES = ["logits", "indicators", "grammar", "context_counts", "decode_counts", "logit_bias", "gumbel_noise",
+              "draft_probabilities", "drafted_tokens"]
+
+
+@pytest.mark.parametrize("plane", ROW_PLANES)
+@pytest.mark.parametrize("driver", ["singular", "multistep"])
+def test_a_refused_layout_leaves_nothing_behind(driver, plane, captured, monkeypatch):
+    """A plane that is not contiguous along its last dimension is refused before outputs are allocated,
+    a seed or uniforms are drawn from the default generator, or events are touched."""
+
+    from sonic_sampler.interface.functional import multistep as fm
+
+    slots, vocab = 6, 9000
+    t = tensors(rows=6, vocab=vocab, slots=slots, target=vocab)
+    t["draft_probabilities"] = torch.zeros(slots, 1, vocab, dtype=torch.bfloat16)
+    call = fm.fused_multistep
+
+    if driver == "singular":
+
+        t["draft_probabilities"] = t["draft_probabilities"][:, 0]
+        t["drafted_tokens"] = torch.zeros(6, 2, dtype=torch.int32)
+        call = fs.fused_singular
+
+    else:
+
+        t["drafted_tokens"] = torch.zeros(6, dtype=torch.int32)
+        t["lookahead"] = 1
+        t["grammar"] = t["grammar"][:, None].expand(slots, 2, -1)
+
+    if plane == "gumbel_noise":
+
+        t["gumbel_noise"] = torch.zeros(slots, 2 if driver == "multistep" else 1, vocab)[:, 0 if driver == "singular" else slice(None)]
+
+    good = t[plane]
+    t[plane] = torch.zeros(*good.shape, 2, dtype=good.dtype)[..., 0]
+    state = torch.random.get_rng_state()
+    monkeypatch.setattr(_native, "event_pair", lambda e: pytest.fail("events were touched"))
+    monkeypatch.setattr(_native, "empty", lambda *a: pytest.fail("an output was allocated"))
+
+    with pytest.raises(ValueError, match=f"`?{plane}`? must be contiguous"):
+
+        call(**t)
+
+    assert torch.equal(torch.random.get_rng_state(), state) and not captured.calls
