@@ -13,7 +13,6 @@ import functools
 import importlib.machinery
 import importlib.util
 import os
-import struct
 from pathlib import Path
 
 import torch  # noqa: F401  (must be imported before the HIP library is loaded)
@@ -236,17 +235,6 @@ def ptr(tensor: torch.Tensor | None) -> int | None:
     return None if tensor is None else tensor.data_ptr()
 
 
-def addr(tensor: torch.Tensor | None) -> int:
-    """A tensor's device address, 0 for an absent one (a field of a packed argument struct)."""
-
-    return 0 if tensor is None else tensor.data_ptr()
-
-
-def stride0(tensor: torch.Tensor | None) -> int:
-
-    return 0 if tensor is None else tensor.stride(0)
-
-
 # torch's current stream of a device index as the raw hipStream_t, without building a Stream
 # object (about a fifteenth of the cost of torch.cuda.current_stream(device).cuda_stream)
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
@@ -287,39 +275,13 @@ def _flat_layout(cls, base: int = 0, prefix: str = "") -> list:
     return layout
 
 
-class Packer:
-    """The bytes of a ctypes argument struct from its field values given positionally, in
-    declaration order (a nested struct's members in its place, pointers as integers, 0 for NULL):
-    one ``struct.Struct.pack`` instead of the keyword constructor, about a sixth of its cost on a
-    call's host path. ``fields`` lists the positions' names."""
-
-    def __init__(self, cls):
-
-        fmt, end = "<", 0
-
-        for _, offset, size, code in _flat_layout(cls):
-
-            fmt += f"{offset - end}x{code}" if offset > end else code
-            end = offset + size
-
-        fmt += f"{ctypes.sizeof(cls) - end}x" if ctypes.sizeof(cls) > end else ""
-        self.fields = tuple(name for name, *_ in _flat_layout(cls))
-        self.struct = struct.Struct(fmt)
-        self.pack = self.struct.pack
-
-        if self.struct.size != ctypes.sizeof(cls):
-
-            raise RuntimeError(f"packed layout of {cls.__name__} is {self.struct.size} bytes, "
-                               f"the struct {ctypes.sizeof(cls)}")
-
-
 class Gatherer:
     """The bytes of a ctypes argument struct from a call's tensors and scalars, given positionally in
     declaration order, packed by the host extension. ``tensors`` names the pointer fields that come
     as tensors (or None, for zeros) and what is taken of each: "T" its address; "S" also its leading
     stride, into the field behind (which then is no argument of its own); "U" also the second
     stride of a three-dimensional one, into the field behind that. ``labels`` renames fields in error
-    messages. ``fields`` lists the positions' names."""
+    messages. ``fields`` lists the positions' names, ``codes`` what each takes."""
 
     def __init__(self, cls, tensors: dict, labels: dict | None = None):
 
@@ -341,6 +303,7 @@ class Gatherer:
             raise ValueError(f"{cls.__name__} has no fields {sorted(unknown)}")
 
         self.fields = tuple(name for *_, name in rows)
+        self.codes = tuple(code for code, *_ in rows)
         self._layout = (ctypes.sizeof(cls), [(*row, labels.get(name, name)) for *row, name in rows])
 
     @functools.cached_property
@@ -354,8 +317,8 @@ _packed_entries: dict = {}
 
 
 def packed_entry(name: str):
-    """Entry point `name` taking its argument struct as packed bytes (``Packer.pack``,
-    ``Gatherer.gather``), called natively."""
+    """Entry point `name` taking its argument struct as packed bytes (``Gatherer.gather``),
+    called natively."""
 
     fn = _packed_entries.get(name)
 

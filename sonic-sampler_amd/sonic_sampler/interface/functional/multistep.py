@@ -43,9 +43,7 @@ from sonic_sampler.ops.base import MAX_K
 FP32 = torch.float32
 TINY: float = torch.finfo(BF16).tiny
 
-MULTISTEP_ARGS = _native.Packer(_native.MultistepArgs)
-
-# the same struct from the call's tensors; their addresses and strides are taken natively
+# ss_multistep_args from the call's tensors; their addresses and strides are taken natively
 MULTISTEP_CALL = _native.Gatherer(
     _native.MultistepArgs,
     dict(logits="S", cu_seqlens="T", indicators="T", slot_mapping="T", drafted_tokens="T", grammar="U",

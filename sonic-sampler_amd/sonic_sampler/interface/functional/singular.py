@@ -57,9 +57,7 @@ KERNEL_LAYOUTS = {None: _native.STRATEGY_AUTO, "tiles": _native.STRATEGY_TILES,
 
 STAGES = {None: 0, "tiles": _native.STAGE_TILES, "rows": _native.STAGE_ROWS}
 
-SINGULAR_ARGS = _native.Packer(_native.SingularArgs)
-
-# the same struct from the call's tensors; their addresses and strides are taken natively
+# ss_singular_args from the call's tensors; their addresses and strides are taken natively
 SINGULAR_CALL = _native.Gatherer(
     _native.SingularArgs,
     dict(logits="S", indicators="T", slot_mapping="T", d2t="T", grammar="S", context_counts="S", decode_counts="S",

@@ -1,9 +1,9 @@
 """The packed argument structs of the eager call path (CPU).
 
 ``fused_singular``, ``fused_multistep`` and ``UnshardedBoundedTopK`` hand the library their
-argument structs as bytes packed positionally (``_native.Packer``) instead of ctypes structs built
+argument structs as bytes gathered positionally (``_native.Gatherer``) instead of ctypes structs built
 by keyword. These tests
-pin that path two ways: the packer's layout against ctypes' own for every argument struct, and the
+pin that path two ways: the gatherer's layout against ctypes' own for every argument struct, and the
 bytes each driver packs against a struct built field by field by name from the same tensors, for
 calls that set every field a caller can reach. The packed entry point is also called into the
 library's argument validation, which must answer as it does for the ctypes struct.
@@ -47,21 +47,21 @@ def named_struct(cls, fields, values):
 
 
 @pytest.mark.parametrize("cls", STRUCTS, ids=lambda c: c.__name__)
-def test_packer_layout_is_the_ctypes_layout(cls):
+def test_gatherer_layout_is_the_ctypes_layout(cls):
 
-    packer = _native.Packer(cls)
-    g = torch.Generator().manual_seed(len(packer.fields))
-    values = [int(v) for v in torch.randint(1, 2 ** 31 - 1, (len(packer.fields),), generator=g)]
+    gatherer = _native.Gatherer(cls, {})
+    g = torch.Generator().manual_seed(len(gatherer.fields))
+    values = [int(v) for v in torch.randint(1, 2 ** 31 - 1, (len(gatherer.fields),), generator=g)]
 
-    assert len(set(packer.fields)) == len(packer.fields)
-    assert packer.pack(*values) == bytes(named_struct(cls, packer.fields, values))
+    assert len(set(gatherer.fields)) == len(gatherer.fields)
+    assert gatherer.gather(*values) == bytes(named_struct(cls, gatherer.fields, values))
 
 
 @pytest.mark.parametrize("cls", STRUCTS, ids=lambda c: c.__name__)
-def test_packer_takes_every_field_type_to_its_limits(cls):
+def test_gatherer_takes_every_field_type_to_its_limits(cls):
     """Each field at its type's extremes (and -1 for the signed ones) packs to the ctypes bytes."""
 
-    packer = _native.Packer(cls)
+    gatherer = _native.Gatherer(cls, {})
     codes = [code for *_, code in _native._flat_layout(cls)]
     limits = {"i": (-2 ** 31, 2 ** 31 - 1, -1), "q": (-2 ** 63, 2 ** 63 - 1, -1),
               "I": (0, 2 ** 32 - 1, 1), "Q": (0, 2 ** 64 - 1, 1)}
@@ -70,7 +70,7 @@ def test_packer_takes_every_field_type_to_its_limits(cls):
 
         values = [limits[c][(pick + j) % 3] for j, c in enumerate(codes)]
 
-        assert packer.pack(*values) == bytes(named_struct(cls, packer.fields, values)), pick
+        assert gatherer.gather(*values) == bytes(named_struct(cls, gatherer.fields, values)), pick
 
 
 class Captured:
@@ -219,22 +219,38 @@ def test_static_scratch_takes_the_no_allocation_entry(captured):
 
 def test_packed_entry_reads_the_bytes_as_the_struct():
     """Into the library's own argument checks (which return before any launch): the packed entry
-    point answers every case as the ctypes entry point does."""
+    point answers the bytes that calls gather as the ctypes entry point does the same struct."""
 
     lib = _native.load()
-    packer = fs.SINGULAR_ARGS
-    base = dict(logits=0x1000, stride_logits=8192, rows=4, vocab_size=8192, target_vocab=8192,
-                block_n=1024, indicators=0x1000, tokens=0x1000, stride_tokens=1, scratch=0x10000,
-                stride_scratch=8 * 128, philox_seed=1, philox_offset=0, philox_enabled=1)
+    plane, tokens = torch.zeros(4, 8192, dtype=torch.bfloat16), torch.zeros(4, 1, dtype=torch.int32)
+    base = dict(logits=plane, rows=4, vocab_size=8192, target_vocab=8192, block_n=1024, indicators=tokens,
+                tokens=tokens, scratch=torch.zeros(4, 8 * 128, dtype=torch.int32), philox_seed=1, philox_enabled=1)
+    answers = set()
 
-    for change in (dict(block_n=512), dict(vocab_size=1024), dict(stride_scratch=100), dict(timestep=65),
-                   dict(max_top_logprobs=129), dict(philox_enabled=0), dict(rows=0)):
+    for change in (dict(block_n=512), dict(vocab_size=1024), dict(scratch=torch.zeros(4, 100, dtype=torch.int32)),
+                   dict(timestep=65), dict(max_top_logprobs=129), dict(philox_enabled=0), dict(rows=0)):
 
-        values = [dict(base, **change).get(f, 0) for f in packer.fields]
-        args = named_struct(_native.SingularArgs, packer.fields, values)
+        fields = [n for n, *_ in _native._flat_layout(_native.SingularArgs)]
+        call = {f: None if code in "TSU" else 0 for f, code in zip(fs.SINGULAR_CALL.fields, fs.SINGULAR_CALL.codes)}
+        call.update(base, **change)
+        named = dict.fromkeys(fields, 0)
 
-        assert _native.packed_entry("ss_fused_singular")(packer.pack(*values)) == \
-            lib.ss_fused_singular(ctypes.byref(args)), change
+        for f, v in call.items():
+
+            named[f] = v.data_ptr() if isinstance(v, torch.Tensor) else v or 0
+
+            # the leading stride stands behind its address
+            if isinstance(v, torch.Tensor) and f in ("logits", "tokens", "scratch"):
+
+                named[fields[fields.index(f) + 1]] = v.stride(0)
+
+        args = named_struct(_native.SingularArgs, fields, [named[f] for f in fields])
+        packed = fs.SINGULAR_CALL.gather(*(call[f] for f in fs.SINGULAR_CALL.fields))
+        assert packed == bytes(args)
+        answers.add(status := _native.packed_entry("ss_fused_singular")(packed))
+        assert status == lib.ss_fused_singular(ctypes.byref(args)), change
+
+    assert len(answers) > 1  # the checks were reached one by one
 
 
 def multistep_expected(call, ver, t, flat, scratch, values, indices, uniform, stream=0x5EA3):
