@@ -121,7 +121,10 @@ int ss_topk(const ss_topk_args *args);
  * Caller contract, not checked on the device (as in the reference): slot_mapping values lie in
  * [0, slots) of every slot-indexed buffer, d2t values in [0, target_vocab), and `probabilities`
  * has a row for every slot a row may map to (the Python driver checks the last against the
- * buffer's storage before the call).
+ * buffer's storage before the call). context_counts and decode_counts are histograms: no count is
+ * negative. Through d2t a row whose penalties can then only lower a logit reads the counts of its
+ * candidates alone, so that a frequency penalty on a negative count would not lift a token that is
+ * no candidate without it.
  * ------------------------------------------------------------------------------------------- */
 typedef struct ss_singular_args {
     /* logits [rows, vocab] bf16 */

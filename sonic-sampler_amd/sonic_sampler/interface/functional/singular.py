@@ -4,6 +4,10 @@
 ``ss_fused_singular``, which launches the tile stage (prologue + tile top-128 per (row, tile)
 workgroup) and the row stage (merge + selection per row) back to back.
 
+``context_counts`` and ``decode_counts`` are histograms, never negative: through ``d2t_mapping`` a row
+whose penalties can then only lower a logit (repetition >= 1, frequency and presence >= 0, no grammar)
+reads the counts of its candidates alone.
+
 Additions to the reference's keywords (all optional):
 
 * ``timestep`` -- number of leading ``drafted_tokens`` columns that count as decode history. The
