@@ -70,9 +70,12 @@ def shifted(plane, offset, pad):
 @pytest.mark.parametrize("offset,pad", [(1, 0), (0, 1), (3, 3), (2, 0), (0, 2)])
 @pytest.mark.parametrize("block,vocab", [(1024, 2052), (2048, 9000), (4096, 8196), (8192, 33000), (16384, 50280)])
 def test_rows_at_any_half_word(block, vocab, offset, pad):
-    """Logit and bias rows at every 2-byte address and stride take the three-dword loads; the same
-    values in aligned rows take the aligned ones. Every output of the decode step, of drafting
-    through d2t, of the verification and of the top-k is the same bits."""
+    """Logit and bias rows at an odd half-word or with an odd stride take the three-dword loads; at an
+    offset or pad of 2 every row still starts on a dword and takes the two-dword loads at addresses that
+    8 does not divide. The same values in contiguous rows take the two-dword loads, but for drafting
+    over vocab - 1 columns, whose ragged width takes the three-dword loads wherever its rows start.
+    Every output of the decode step, of drafting through d2t, of the verification and of the top-k is
+    the same bits."""
 
     from sonic_sampler.core.buffer import SamplingBuffers
     from sonic_sampler.core.flags import Flags, Indicator
@@ -88,7 +91,7 @@ def test_rows_at_any_half_word(block, vocab, offset, pad):
     kinds = [0x7BF, 0x400, 0x40E, 0x410, 0x05E, 0x4B1]
     buffers.flags = Flags.from_values(rows, 1, [Indicator(k) for k in kinds], device=torch.device(DEV))
     rep = buffers.repetition
-    d2t = torch.randperm(vocab, generator=g)[: vocab - 1].to(torch.int32).to(DEV)
+    d2t = torch.randperm(vocab, generator=g).to(torch.int32).to(DEV)
     common = dict(
         indicators=buffers.flags.target, block_n=block, context_counts=rep.counts.context,
         repetition_penalties=rep.multiplicative, frequency_penalties=rep.frequency,
@@ -100,10 +103,16 @@ def test_rows_at_any_half_word(block, vocab, offset, pad):
         print(f"block {block} vocab {vocab} offset {offset} pad {pad}", flush=True)
         grammar = buffers.grammar[:, 0].as_subclass(torch.Tensor)
         one = fused_singular(x, logit_bias=bias, grammar=grammar, decode_counts=rep.counts.decode, **common)
-        probabilities = torch.zeros(rows, vocab, dtype=torch.bfloat16, device=DEV)
-        draft = fused_singular(x[:, : vocab - 1], logit_bias=bias, grammar=grammar, decode_counts=rep.counts.decode,
-                               d2t_mapping=d2t, target_vocab=vocab, return_probabilities=True,
-                               draft_probabilities=probabilities, **common)
+        drafts = []
+
+        for width in (vocab - 4, vocab - 1):
+
+            probabilities = torch.zeros(rows, vocab, dtype=torch.bfloat16, device=DEV)
+            draft = fused_singular(x[:, :width], logit_bias=bias, grammar=grammar, decode_counts=rep.counts.decode,
+                                   d2t_mapping=d2t[:width], target_vocab=vocab, return_probabilities=True,
+                                   draft_probabilities=probabilities, **common)
+            drafts += [draft.tokens, probabilities]
+
         values = torch.zeros(rows, 128, device=DEV)
         indices = torch.zeros(rows, 128, dtype=torch.int32, device=DEV)
         drafted = x.float().argmax(-1).to(torch.int32)
@@ -115,13 +124,13 @@ def test_rows_at_any_half_word(block, vocab, offset, pad):
         topk = UnshardedBoundedTopK.initialize(vocab_size=vocab, batch_size=rows, k=128, block_size=block, device=DEV)
         best, columns = topk(x)
 
-        return [t.clone() for t in (one.tokens, draft.tokens, probabilities, check.tokens, check.offsets, indices, values,
-                                    best, columns)]
+        return [t.clone() for t in (one.tokens, *drafts, check.tokens, check.offsets, indices, values, best,
+                                    columns)]
 
     want = outputs(logits, buffers.bias)
     got = outputs(shifted(logits, offset, pad), shifted(buffers.bias, offset, pad))
 
-    for name, a, b in zip(("decode", "drafts", "probabilities", "tokens", "offsets", "indices", "values", "top-k", "columns"),
+    for name, a, b in zip(("decode", "drafts", "probabilities", "ragged drafts", "their probabilities", "tokens", "offsets", "indices", "values", "top-k", "columns"),
                           want, got):
 
         assert torch.equal(a, b), f"{name} differ between aligned rows and rows at offset {offset}, pad {pad}"
