@@ -317,7 +317,7 @@ __global__ __launch_bounds__(SS_BLOCK) void topk_tiles_kernel(const uint16_t *p_
         keys.p[2 * c] = packed_keys(w.x);
         keys.p[2 * c + 1] = packed_keys(w.y);
     }
-    mask_absent<E>(col0, p_vocab, keys);
+    mask_absent<E, ANY>(col0, p_vocab, keys);
     tile_stage<E, true>(sm, false, keys, p_scratch + (int64_t)row * p_stride_scratch, tile,
                         min(p_block_n, p_vocab - col0), p_k);
 }
