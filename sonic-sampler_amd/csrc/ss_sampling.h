@@ -309,8 +309,12 @@ __device__ __forceinline__ float chain_ieee(const Chain &k, float x, int32_t dec
 // and every lane fetches its own chunks' keys back. 1280 verification rows of 128256 columns with such
 // requests: 2180 vector instructions a wave -> 1213, the tile kernel 240 -> 153 us (with the planes
 // cached between a request's rows and the logits no longer loaded twice: 0.58 GB fetched, not 1.25).
+// Tiles of at most 2048 columns, which a few rows take, keep no list: their 8 elements a lane are soon
+// done in place, and the list's round trip through workgroup memory was 0.35 us of a call of one row
+// with penalties (10.2 us; in place 9.9).
 template <int E>
 struct ExcList {
+    static constexpr bool ON = E > 8;
     static constexpr uint32_t CAP = E / 2 * 64 * 4 / 48;  // records that fit TileSmem::keys
     static constexpr int WORDS = 12;                      // of a record
     uint32_t *mem;       // the wave's records
@@ -326,8 +330,8 @@ constexpr uint32_t EXC_STAGED_CAP = 38;
 // Keys of the E / 4 chunks of one pass from their (grammar-masked) logits, decode counts, context
 // counts and bias bits. The temperature division, the chain's whole effect on an element with zero
 // counts and bias, runs for all elements with one multiply each; the chunks with a nonzero count or
-// bias go to `ex` (chunk c of the pass as chunk c0 + c of the tile), or, where the list has no room
-// for the pass's (or a non-finite frequency penalty turns 0 * f into NaN), the chain runs on every
+// bias go to `ex` (chunk c of the pass as chunk c0 + c of the tile), or, where the tile keeps no list or
+// it has no room for the pass's (or a non-finite frequency penalty turns 0 * f into NaN), the chain runs on every
 // element. Rows whose divisors have no exact reciprocal take the IEEE chain on every element.
 // lw / bw: the (grammar-masked) logits and the biases as loaded pairs. maybe_exc is false when no
 // element can have a nonzero count or bias (no penalty or bias plane is read) and the chain is not
@@ -365,7 +369,7 @@ __device__ __forceinline__ void finish_keys(const Chain &k, bool all_exc, bool m
             ex.m[c0 + c] = __ballot(((uint32_t)(n.x | n.y | n.z | n.w) | bw[c].x | bw[c].y) != 0u);
             total += (uint32_t)__popcll(ex.m[c0 + c]);
         }
-        if (all_exc || ex.cnt + total > ex.cap) {
+        if (all_exc || (ExcList<ET>::ON ? ex.cnt + total > ex.cap : total != 0)) {
 #pragma unroll
             for (int c = 0; c < E / 4; ++c) {
                 ex.m[c0 + c] = 0;
@@ -376,7 +380,7 @@ __device__ __forceinline__ void finish_keys(const Chain &k, bool all_exc, bool m
                                      (key_of(chain_fast(f, x(j + 1), dec[c][i + 1], ctx[c][i + 1], bb(j + 1))) << 16);
                 }
             }
-        } else if (total) {
+        } else if (ExcList<ET>::ON && total) {
 #pragma unroll
             for (int c = 0; c < E / 4; ++c) {
                 const uint64_t m = ex.m[c0 + c];
@@ -408,7 +412,7 @@ __device__ __forceinline__ void finish_keys(const Chain &k, bool all_exc, bool m
 // hold them.
 template <int E>
 __device__ __forceinline__ void finish_exceptions(const FastChain &f, const ExcList<E> &ex, Keys<E> &keys) {
-    if (!ex.cnt) return;
+    if (!ExcList<E>::ON || !ex.cnt) return;
 #pragma unroll 1
     for (uint32_t i = (uint32_t)lane_id(); i < ex.cnt; i += 64) {
         uint32_t *r = ex.mem + i * ExcList<E>::WORDS;
