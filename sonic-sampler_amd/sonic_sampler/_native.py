@@ -17,6 +17,8 @@ from pathlib import Path
 
 import torch  # noqa: F401  (must be imported before the HIP library is loaded)
 
+_Device, _Tensor = torch.device, torch.Tensor
+
 _LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libsonic_sampler.so"
 _HOST_PATH = _LIB_PATH.with_name("_sonic_host.so")
 
@@ -189,16 +191,22 @@ _empty = None
 
 
 def empty(device, dtype: torch.dtype, *sizes: int) -> torch.Tensor:
-    """``torch.empty(sizes, dtype=dtype, device=device)``; natively on a GPU's ``torch.device``, through
-    torch for any other form of a device (None, a string, an index) and for other devices."""
+    """``torch.empty(sizes, dtype=dtype, device=device)``; natively on a ``torch.device`` once a GPU's has
+    loaded the host extension, through torch for any other form of a device (None, a string, an index)
+    and where no GPU is in use. (The device's type is read only until then: on each call it cost
+    0.2 us an output.)"""
 
     global _empty
 
-    if type(device) is not torch.device or device.type != "cuda":
+    if type(device) is not _Device:
 
         return torch.empty(sizes, dtype=dtype, device=device)
 
     if _empty is None:
+
+        if device.type != "cuda":
+
+            return torch.empty(sizes, dtype=dtype, device=device)
 
         _empty = host().empty
 
@@ -206,15 +214,19 @@ def empty(device, dtype: torch.dtype, *sizes: int) -> torch.Tensor:
 
 
 def unit_strides(names: tuple, *tensors: torch.Tensor | None) -> None:
-    """ValueError naming the first of the tensors that is not contiguous along its last dimension."""
+    """ValueError naming the first of the tensors that is not contiguous along its last dimension. The
+    first call puts the host extension's function in this one's place."""
 
-    host().unit_strides(names, *tensors)
+    global unit_strides
+
+    unit_strides = host().unit_strides
+    unit_strides(names, *tensors)
 
 
 def new_empty(source: torch.Tensor, dtype: torch.dtype, *sizes: int) -> torch.Tensor:
     """``source.new_empty(sizes, dtype=dtype)``: on the source's device, of its tensor class."""
 
-    if type(source) is not torch.Tensor:
+    if type(source) is not _Tensor:
 
         return source.new_empty(sizes, dtype=dtype)
 
