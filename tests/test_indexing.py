@@ -683,7 +683,8 @@ def tile_stage_emulation(keys, E, valid):
         bound = 0
         need = wave_share(SS_K, valid, w, block)
 
-        if valid <= 1024 and valid < block:   # one partly filled chunk: the lanes' elements 0-3, all key bits
+        # few columns: the lanes' elements 0-3, all key bits
+        if valid < block and (valid <= 1024 if E >= 64 else valid < 512):
 
             first, low = [k for v in lanes for k in v[:4]], 0
 
@@ -741,7 +742,7 @@ def tile_cases():
 
         block = 256 * E
 
-        for valid in (block, block - 1, 1280 if E == 16 else block // 3, 200, 127, 100, 1):
+        for valid in (block, block - 1, 1280 if E == 16 else block // 3, 1000, 513, 512, 511, 200, 127, 100, 1):
 
             for admitted in (None, 3, 60, 127, 128, 200, 700):
 
