@@ -307,8 +307,8 @@ __device__ __forceinline__ float chain_ieee(const Chain &k, float x, int32_t dec
 // three for one lane's sake. Instead the 4-column chunks that hold one go to a list in workgroup
 // memory (logits, bias, decode and context counts: 48 bytes), one lane then takes one chunk of it,
 // and every lane fetches its own chunks' keys back. 1280 verification rows of 128256 columns with such
-// requests: 2180 vector instructions a wave -> 1213, the tile kernel 240 -> 153 us (with the planes
-// cached between a request's rows and the logits no longer loaded twice: 0.58 GB fetched, not 1.25).
+// requests: 2180 vector instructions a wave -> 1193, the tile kernel 240 -> 145 us (with the planes
+// cached between a request's rows and the logits no longer loaded twice: 0.59 GB fetched, not 1.25).
 // Tiles of at most 2048 columns, which a few rows take, keep no list: their 8 elements a lane are soon
 // done in place, and the list's round trip through workgroup memory was 0.35 us of a call of one row
 // with penalties (10.2 us; in place 9.9).

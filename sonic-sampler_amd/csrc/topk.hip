@@ -295,8 +295,8 @@ __global__ __launch_bounds__(SS_BLOCK) void topk_merge_kernel(void *p_scratch, i
 // bfloat16 tile stage: tile blockIdx.x % tiles of row blockIdx.x / tiles, its exact top-k by the
 // fused kernels' tile selection (tile_stage) on 16-bit keys held two per register and 32-bit
 // composites. Selected as the float32 logits below (values widened to a register each, 64-bit
-// composites) a wave of a 16384-column tile took 1770 vector instructions; it takes 566, and the
-// kernel 17.2 us instead of 45.5 at 256 rows of 128256 (3.8 TB/s; bound by its instructions and the
+// composites) a wave of a 16384-column tile took 1770 vector instructions; it takes 581, and the
+// kernel 15.2 us instead of 45.5 at 256 rows of 128256 (4.3 TB/s; bound by its instructions and the
 // four workgroups a CU that the spilled keys leave).
 // ---------------------------------------------------------------------------------------------
 template <bool ANY, int E>
